@@ -123,6 +123,15 @@ __device__ __forceinline__ T* sgpr_ptr(T* p) {
     return (T*)g;
 }
 
+// A load through a pointer whose address space the compiler has lost (one
+// picked per lane among kernel arguments): as a global instruction. A flat one
+// counts as an LDS access too, so every wait for it drains all loads in flight.
+template <typename T>
+__device__ __forceinline__ T ld_global(const void* p) {
+    using G = const __attribute__((address_space(1))) T;
+    return *reinterpret_cast<G*>(reinterpret_cast<uint64_t>(p));
+}
+
 // A wave-uniform int32 read with a scalar load (through the constant address
 // space): its wait counts scalar loads only, so vector loads issued before it
 // stay in flight while it is waited for. The value must not change while the

@@ -191,6 +191,13 @@ struct qora_hip_ctx {
     std::vector<DevWeight> weights;
     long long* ws_acc = nullptr;         // kernel-level fixed-point accumulator
     uint64_t ws_acc_n = 0;
+    // one-launch GEMV entries: the K slices' terms, and the column tiles'
+    // arrival counters (0 between calls; only calls on the context's own
+    // stream outside a capture use them, one behind the other)
+    long long* ws_part = nullptr;
+    uint64_t ws_part_n = 0;
+    uint32_t* ws_count = nullptr;
+    uint64_t ws_count_n = 0;
     // on-device sampling scratch (grown to the largest vocab seen)
     float* smp_work = nullptr;
     unsigned long long* smp_cand = nullptr;
@@ -266,6 +273,41 @@ int ensure_acc_ws(qora_hip_ctx* c, uint64_t n) {
     if (int rc = dalloc(c, nn * sizeof(long long), &p)) return rc;
     c->ws_acc = (long long*)p;
     c->ws_acc_n = nn;
+    return QORA_HIP_OK;
+}
+
+// Terms and counters of a one-launch GEMV of `terms` int64 words and `tiles`
+// column tiles. qora_hip_create asks for kGemvWsTerms and kGemvWsTiles once
+// (the largest GEMV of SmolLM3-3B takes 352256 terms), so that a first call
+// allocates nothing here.
+constexpr uint64_t kGemvWsTerms = 1u << 19, kGemvWsTiles = 256;
+
+int ensure_gemv_ws(qora_hip_ctx* c, uint64_t terms, uint64_t tiles) {
+    const uint64_t words = tiles * kGemvCountStride;
+    if (terms <= c->ws_part_n && words <= c->ws_count_n) return QORA_HIP_OK;
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    void* p;
+    if (terms > c->ws_part_n) {
+        if (c->ws_part) (void)hipFree(c->ws_part);
+        c->ws_part = nullptr;
+        c->ws_part_n = 0;
+        if (int rc = dalloc(c, terms * sizeof(long long), &p)) return rc;
+        c->ws_part = (long long*)p;
+        c->ws_part_n = terms;
+    }
+    if (words > c->ws_count_n) {
+        if (c->ws_count) (void)hipFree(c->ws_count);
+        c->ws_count = nullptr;
+        c->ws_count_n = 0;
+        if (int rc = dalloc(c, words * sizeof(uint32_t), &p)) return rc;
+        const hipError_t e = hipMemsetAsync(p, 0, words * sizeof(uint32_t), c->stream);
+        if (e != hipSuccess) {
+            (void)hipFree(p);
+            return fail(c, QORA_HIP_E_DEVICE, std::string("GEMV counters: ") + hipGetErrorString(e));
+        }
+        c->ws_count = (uint32_t*)p;
+        c->ws_count_n = words;
+    }
     return QORA_HIP_OK;
 }
 
@@ -522,6 +564,8 @@ extern "C" int qora_hip_create(int device, qora_hip_ctx** out) {
     } else {
         c->h_tok = nullptr;
     }
+    // (without room for it here the first GEMV call asks again and reports it)
+    (void)ensure_gemv_ws(c, kGemvWsTerms, kGemvWsTiles);
     *out = c;
     return QORA_HIP_OK;
 }
@@ -538,7 +582,7 @@ extern "C" int qora_hip_destroy(qora_hip_ctx* c) {
         if (w.w) (void)hipFree(w.w);
         if (w.scales) (void)hipFree(w.scales);
     }
-    for (void* p : {(void*)c->ws_acc, (void*)c->ws_attn_part, c->ws_pf, (void*)c->smp_work, (void*)c->smp_cand,
+    for (void* p : {(void*)c->ws_acc, (void*)c->ws_part, (void*)c->ws_count, (void*)c->ws_attn_part, c->ws_pf, (void*)c->smp_work, (void*)c->smp_cand,
                     (void*)c->smp_rng, (void*)c->smp_pen, c->smp_sort})
         if (p) (void)hipFree(p);
     if (c->h_pin) (void)hipHostFree(c->h_pin);
@@ -1659,13 +1703,12 @@ extern "C" int qora_hip_graph_destroy(qora_hip_ctx* c, void* graph_exec) {
 
 namespace {
 
-// Argument checks and launch plan of acc[0:n] (+ acc[n:2n] when paired) +=
-// W x; nothing is launched, so a refused call leaves the device untouched.
-int gemv_acc_prepare(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, const void* w1, const void* s1,
-                     const float* x, long long* acc, uint64_t k, uint64_t n, bool paired, GemvPlan* plan,
-                     GemvParams* params) {
-    if (!c) return QORA_HIP_E_INVALID;
-    if (!w0 || !x || !acc || (fmt == FMT_Q4 && !s0) || (paired && (!w1 || (fmt == FMT_Q4 && !s1))))
+// Argument checks and launch plan of W x (paired: Wg x and Wu x) on the
+// reference layout; nothing is launched, so a refused call leaves the device
+// untouched.
+int gemv_prepare_launch(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, const void* w1, const void* s1,
+                        const float* x, uint64_t k, uint64_t n, bool paired, GemvPlan* plan, GemvParams* params) {
+    if (!w0 || !x || (fmt == FMT_Q4 && !s0) || (paired && (!w1 || (fmt == FMT_Q4 && !s1))))
         return fail(c, QORA_HIP_E_INVALID, "null argument");
     if (k == 0 || n == 0 || n % 32 != 0 || k > 0xFFFFFFFFull || n / 32 > 0xFFFFFFFFull)
         return fail(c, QORA_HIP_E_INVALID, "GEMV needs k > 0 and n % 32 == 0");
@@ -1685,10 +1728,20 @@ int gemv_acc_prepare(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, c
     p.k = (uint32_t)k;
     p.pro = PRO_PLAIN;
     p.x = x;
-    p.acc = acc;
     apply_plan(pl, &p);
     *plan = pl;
     *params = p;
+    return QORA_HIP_OK;
+}
+
+// The same for acc[0:n] (+ acc[n:2n] when paired) += W x.
+int gemv_acc_prepare(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, const void* w1, const void* s1,
+                     const float* x, long long* acc, uint64_t k, uint64_t n, bool paired, GemvPlan* plan,
+                     GemvParams* params) {
+    if (!c) return QORA_HIP_E_INVALID;
+    if (!acc) return fail(c, QORA_HIP_E_INVALID, "null argument");
+    if (int rc = gemv_prepare_launch(c, fmt, w0, s0, w1, s1, x, k, n, paired, plan, params)) return rc;
+    params->acc = acc;
     return QORA_HIP_OK;
 }
 
@@ -1703,16 +1756,42 @@ int gemv_acc_entry(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, con
     return QORA_HIP_OK;
 }
 
-// y = W x (paired: y = silu(Wg x) * (Wu x)) through the context accumulator:
-// clear, accumulate, convert.
+// Whether a kernel-level call may use scratch that has to be zero between
+// launches: on the context's own stream, outside a capture, calls run one
+// behind the other; a caller's stream or a captured graph could overlap them.
+bool in_order(qora_hip_ctx* c, hipStream_t s) {
+    if (s != c->stream || c->capturing) return false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+}
+
+// y = W x (paired: y = silu(Wg x) * (Wu x)). On the context's stream one
+// launch: the last workgroup of each column tile sums the K slices (2048 ->
+// 512 in Q4: 4.1 us a call against 9.4 for three launches, which the host's
+// ~2.8 us a launch bounds). In a capture or on a caller's stream through the
+// context accumulator (clear, accumulate, convert): the same terms summed in
+// the same fixed point, so the same bits.
 int gemv_entry(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, const void* w1, const void* s1,
                const float* x, float* y, uint64_t k, uint64_t n, bool paired, void* stream) {
     if (!c) return QORA_HIP_E_INVALID;
     if (!y) return fail(c, QORA_HIP_E_INVALID, "null argument");
     if (n == 0 || n > 0x7FFFFFFFull) return fail(c, QORA_HIP_E_INVALID, "GEMV needs 0 < n < 2^31");
+    const hipStream_t s = pick_stream(c, stream);
+    // (an eager call also sizes what a captured one will need)
     const uint64_t accn = paired ? 2 * n : n;
     if (int rc = ensure_acc_ws(c, accn)) return rc;
-    const hipStream_t s = pick_stream(c, stream);
+    if (in_order(c, s)) {
+        GemvPlan pl;
+        GemvParams p{};
+        if (int rc = gemv_prepare_launch(c, fmt, w0, s0, w1, s1, x, k, n, paired, &pl, &p)) return rc;
+        if (pl.wgs() > 1)
+            if (int rc = ensure_gemv_ws(c, (uint64_t)pl.tiles * pl.wgs() * (uint64_t)pl.gt * 32u, pl.tiles)) return rc;
+        p.y = y;
+        p.part = c->ws_part;
+        p.count = c->ws_count;
+        HIP_TRY(c, launch_gemv(fmt, pl, p, s));
+        return QORA_HIP_OK;
+    }
     HIP_TRY(c, launch_fill_zero(c->ws_acc, accn, s));
     if (int rc = gemv_acc_entry(c, fmt, w0, s0, w1, s1, x, c->ws_acc, k, n, paired, stream)) return rc;
     HIP_TRY(c, launch_acc_to_f32(c->ws_acc, (uint32_t)n, paired ? 1 : 0, y, s));

@@ -14,9 +14,10 @@
 //   * A workgroup (256 lanes) covers a column tile of GT groups and a slice of
 //     KR = (256/GT)*RPL input rows. Lanes t = rl*GT + gi: the GT lanes of a
 //     row read GT*16 contiguous bytes (128 B or 256 B row segments).
-//   * The row lanes of a group are summed through LDS; each column's sum is
-//     then added to a fixed-point int64 accumulator with one fire-and-forget
-//     64-bit atomic. Integer addition is exact, so the result does not
+//   * The row lanes of a group are summed in registers and the waves through
+//     LDS; each column's sum is then added to a fixed-point int64 accumulator
+//     with one fire-and-forget 64-bit atomic (or, for the kernel-level entries
+//     that return y, left for the tile's last workgroup: OUT below). Integer addition is exact, so the result does not
 //     depend on the order the K slices land in (deterministic), and no
 //     fence or counter is needed: the kernel boundary publishes the sums.
 //   * The prologue builds the K slice of the input in LDS: plain x, RMSNorm
@@ -38,6 +39,9 @@
 #include "params.hpp"
 
 namespace qora {
+
+// v as a fixed-point term; a value of 2^20 or more (or NaN) gives 0.
+__device__ __forceinline__ long long fixed_term(float v) { return fabsf(v) < 1048576.0f ? to_fixed(v) : 0LL; }
 
 // acc += v in fixed point; a contribution of 2^20 or more (or NaN) sets *flag
 // instead of wrapping the accumulator.
@@ -165,11 +169,10 @@ __device__ __forceinline__ LaneSrc lane_source(const GemvParams& p, uint32_t til
     return s;
 }
 
-// Tile-layout packer: one workgroup per (GEMV workgroup b, row step j)
-// copies what lane t of GEMV workgroup b loads at step j (16 B of Q4 or 64 B
-// of F16, and the Q4 scale) into load order. grid = blocks * rpl, 256 lanes.
-template <int FMT>
-__global__ __launch_bounds__(256) void gemv_tile_kernel(GemvParams p, int gt, int rpl, uint8_t* tw, uint16_t* ts) {
+// Tile-layout packer (F16): one workgroup per (GEMV workgroup b, row step j)
+// copies the 64 B that lane t of GEMV workgroup b loads at step j into load
+// order. grid = blocks * rpl, 256 lanes.
+__global__ __launch_bounds__(256) void gemv_tile_kernel(GemvParams p, int gt, int rpl, uint8_t* tw) {
     const int t = threadIdx.x;
     const uint32_t b = blockIdx.x / (uint32_t)rpl;
     const uint32_t j = blockIdx.x % (uint32_t)rpl;
@@ -177,204 +180,207 @@ __global__ __launch_bounds__(256) void gemv_tile_kernel(GemvParams p, int gt, in
     const uint32_t RL = 256u / (uint32_t)gt;
     const LaneSrc src = lane_source(p, tile, t % gt, gt);
     const uint32_t r = min(split * p.rows_per_split + (uint32_t)(t / gt) + j * RL, p.k - 1u);
-    if constexpr (FMT == FMT_Q4) {
-        const uint4 v = *reinterpret_cast<const uint4*>(src.sg.w + ((uint64_t)r * src.sg.groups + src.grp_c) * 16u);
-        *reinterpret_cast<uint4*>(tw + (((uint64_t)b * rpl + j) * 256u + t) * 16u) = v;
-        ts[((uint64_t)b * 256u + t) * rpl + j] = src.sg.scales[(uint64_t)r * src.sg.groups + src.grp_c];
-    } else {
-        const uint4* s = reinterpret_cast<const uint4*>(src.sg.w + ((uint64_t)r * src.sg.groups + src.grp_c) * 64u);
+    const uint4* s = reinterpret_cast<const uint4*>(src.sg.w + ((uint64_t)r * src.sg.groups + src.grp_c) * 64u);
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-            *reinterpret_cast<uint4*>(tw + ((((uint64_t)b * rpl + j) * 4u + v) * 256u + t) * 16u) = s[v];
-    }
+    for (int v = 0; v < 4; ++v)
+        *reinterpret_cast<uint4*>(tw + ((((uint64_t)b * rpl + j) * 4u + v) * 256u + t) * 16u) = s[v];
 }
 
-template <int FMT, int GT, int RPL, int PRO, bool TILED>
-__global__ __launch_bounds__(256) void gemv_kernel(const uint8_t* tw, const uint16_t* ts, const void* xin,
+// Sum of acc[0..31] over the 64 / GT row lanes of a wave (lane = row lane * GT
+// + group), scattered: lane l ends with GT / 2 columns of its group,
+// out[0 .. GT / 2) = the sums of columns base .. base + GT / 2 - 1, base as
+// returned. Each stage halves a lane's columns by adding its partner's copy of
+// the half it keeps (lane-swap instructions for lanes ^ 32 and ^ 16, a DPP row
+// rotate for ^ 8), so no stage goes through LDS.
+template <int GT>
+__device__ __forceinline__ int reduce_row_lanes(const float (&acc)[32], float (&out)[GT / 2]) {
+    static_assert(GT == 8 || GT == 16, "8 or 4 row lanes a wave");
+    const int lane = threadIdx.x & (kWave - 1);
+    float a[16], b[8];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[i]), __float_as_uint(acc[i + 16]), false, false);
+        a[i] = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(a[i]), __float_as_uint(a[i + 8]), false, false);
+        b[i] = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+    }
+    int base = ((lane & 32) ? 16 : 0) + ((lane & 16) ? 8 : 0);
+    if constexpr (GT == 16) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) out[i] = b[i];
+    } else {
+        const bool hi = (lane & 8) != 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[i] = (hi ? b[i + 4] : b[i]) + dpp_f32<0x128>(hi ? b[i] : b[i + 4]);   // row_ror:8
+        base += hi ? 4 : 0;
+    }
+    return base;
+}
+
+// OUT: 0 adds the slice's sums to the fixed-point accumulator p.acc with
+// atomics. 1 leaves them (the same fixed-point terms) in p.part and the last
+// workgroup of a column tile to arrive (p.count, one counter per tile) sums the
+// tile's terms and writes y, SiLU(gate) * up when paired: clear, accumulate
+// and convert in one launch. The terms travel by agent-scope stores and loads
+// (each wave waits for its stores' acknowledgement before the tile's count),
+// so no L2 write-back is needed; the last arriver sets the counter back to 0.
+//
+// What bounds it: F16 the weight stream (2048 -> 2 x 11008 at 4.9 TB/s, a large
+// copy's rate), Q4 the unpacking on the VALU (17 instructions per 8 weights;
+// the same pair at 2.0 TB/s), small shapes the launch and the hand-over (1.5 us
+// of a 4.1 us call). Batches of B rows are loaded by global instructions with
+// their inputs, every load of a batch in flight; the row lanes are summed in
+// registers (reduce_row_lanes) and the four waves through 4 or 8 KB of LDS.
+// Before, weights came by flat loads (each wait drained every load), each lane
+// put 32 sums into 34 KB of LDS (four workgroups a CU), and a call took three
+// launches: one token's MLP (norm, gate|up, down) 22.0 -> 13.8 us in Q4 and 32.3
+// -> 27.5 us in F16, 2048 -> 512 9.4 -> 4.1 us a call.
+template <int FMT, int GT, int B, bool LOOP, int PRO, bool TILED, int OUT>
+__global__ __launch_bounds__(256) void gemv_kernel(const uint8_t* tw, const void* xin,
                                                    const void* xaux, uint32_t k, uint32_t tiles_a, uint32_t rps,
                                                    uint32_t ss_nn, GemvParams p) {
     // (the arguments of the first loads come ahead of the parameter block and
     // are preloaded into scalar registers at wave launch: tile-layout
-    // weights and scales, the input and its second operand, K, the tile
-    // count, the rows per K slice, ss_n | norm_n << 8)
+    // weights, the input and its second operand, K, the tile count, the rows
+    // per K slice, ss_n | norm_n << 8)
+    static_assert(FMT == FMT_F16 || !TILED, "the Q4 tile layout runs on the matrix cores");
+    static_assert(OUT == 0 || (PRO == PRO_PLAIN && !TILED), "y is written by the kernel-level entries only");
     const uint32_t ss_n = ss_nn & 0xFFu, norm_n = ss_nn >> 8;
     const long long* xacc = static_cast<const long long*>(xin);
     constexpr int NT = 256;
+    constexpr int NW = NT / kWave;
     constexpr int RL = NT / GT;          // row lanes
     constexpr int COLS = GT * 32;        // columns per tile
-    constexpr int KR = RL * RPL;         // rows per workgroup
-    constexpr int RED_STRIDE = 33;       // padded group stride in LDS
     constexpr int CPT = COLS / NT;       // columns per thread in the reduction
-    constexpr int MAXH = KR / 32 + 1;    // heads a K slice can touch (head_dim >= 32)
     constexpr bool kStage = PRO == PRO_ATTN;   // only the attention merge stages x in LDS
+    constexpr int MAXH = kGemvAttnRows / 32 + 1;   // heads a K slice can touch (head_dim >= 32)
 
-    __shared__ float xs[kStage ? KR : 1];
-    __shared__ float red[NT * RED_STRIDE];
-    __shared__ float wred[NT / kWave];
+    __shared__ float xs[kStage ? kGemvAttnRows : 1];
+    __shared__ __align__(16) float red[OUT ? 2 : 1][NW][COLS];   // (OUT 1: alternating by slice)
+    __shared__ float wred[NW];
     __shared__ float aw[kStage ? kAttnMaxSplits * MAXH : 1];
 
     const int t = threadIdx.x;
     const int gi = t % GT;
-    const int rl = t / GT;
+    const uint32_t rl = (uint32_t)(t / GT);
     const uint32_t tile = blockIdx.x % tiles_a;
-    const uint32_t split = blockIdx.x / tiles_a;
-    const uint32_t k0 = split * rps;
-    const uint32_t k1 = min(k, k0 + rps);
     const uint32_t klast = k - 1u;
+    const uint32_t rpl = rps / RL;       // rows per lane and slice: a multiple of B (LOOP), or B
     // (the accumulator this launch clears is cleared at the end: stores issued
     // first would count in vmcnt ahead of the input and weight loads)
 
     // ---- which segment / group this lane reads ----
     const LaneSrc src = lane_source(p, tile, gi, GT);
     const GemvSeg& sg = src.sg;
-    // Every load is unconditional, so all of a lane's loads are in flight
-    // together and the math on row j starts when row j arrives: rows past
-    // the slice read a valid row and get a zero input; lanes past the
-    // segment read group 0 and their columns are never written.
-    const uint32_t grp_c = src.grp_c;
 
-    // ---- 1. input values of this lane's rows (direct loads, no LDS) ----
-    float xv[RPL];
-    long long xa[PRO == PRO_PLAIN || PRO == PRO_ATTN ? 1 : RPL];
-    long long ua[PRO == PRO_SILU_FIXED ? RPL : 1];
-    uint32_t gm[PRO == PRO_GAMMA_FIXED ? RPL : 1];
+    // ---- one batch of B rows: weights, scales, inputs ----
+    // Every load is unconditional, so all of a batch's loads are in flight
+    // together: rows past the slice read a valid row and get a zero input;
+    // lanes past the segment read group 0 and their columns are never written.
+    constexpr int WV = FMT == FMT_Q4 ? 1 : 4;
+    struct Batch {
+        v4u32 w[B][WV];
+        uint32_t s[FMT == FMT_Q4 ? B : 1];
+        float x[PRO == PRO_PLAIN ? B : 1];
+        long long xa[PRO == PRO_GAMMA_FIXED || PRO == PRO_SILU_FIXED ? B : 1];
+        long long ua[PRO == PRO_SILU_FIXED ? B : 1];
+        uint32_t gm[PRO == PRO_GAMMA_FIXED ? B : 1];
+    };
+    const uint32_t row_bytes = FMT == FMT_Q4 ? 16u : 64u;
+    const uint8_t* wbase = TILED ? tw + (uint64_t)blockIdx.x * rpl * 16384u + (uint32_t)t * 16u
+                                 : sg.w + (uint64_t)src.grp_c * row_bytes;
+    const uint64_t wrow = (uint64_t)sg.groups * row_bytes;
+    auto load = [&](uint32_t k0, uint32_t j0) {
+        Batch b;
 #pragma unroll
-    for (int j = 0; j < RPL; ++j) {
-        const uint32_t rc = min(k0 + rl + j * RL, klast);
-        if constexpr (PRO == PRO_PLAIN) xv[j] = static_cast<const float*>(xin)[rc];
-        if constexpr (PRO == PRO_GAMMA_FIXED) {
-            xa[j] = xacc[rc];
-            gm[j] = static_cast<const uint16_t*>(xaux)[rc];
+        for (int j = 0; j < B; ++j) {
+            const uint32_t r = min(k0 + rl + (j0 + (uint32_t)j) * RL, klast);
+            if constexpr (PRO == PRO_PLAIN) b.x[j] = static_cast<const float*>(xin)[r];
+            if constexpr (PRO == PRO_GAMMA_FIXED) {
+                b.xa[j] = xacc[r];
+                b.gm[j] = static_cast<const uint16_t*>(xaux)[r];
+            }
+            if constexpr (PRO == PRO_SILU_FIXED) {
+                b.xa[j] = xacc[r];
+                b.ua[j] = xacc[k + r];
+            }
         }
-        if constexpr (PRO == PRO_SILU_FIXED) {
-            xa[j] = xacc[rc];
-            ua[j] = xacc[k + rc];
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            const uint32_t r = min(k0 + rl + (j0 + (uint32_t)j) * RL, klast);
+            const uint8_t* wp = TILED ? wbase + (uint64_t)(j0 + (uint32_t)j) * 16384u : wbase + r * wrow;
+#pragma unroll
+            for (int v = 0; v < WV; ++v) b.w[j][v] = ld_global<v4u32>(wp + v * (TILED ? 4096 : 16));
+            if constexpr (FMT == FMT_Q4) b.s[j] = ld_global<uint16_t>(sg.scales + (uint64_t)r * sg.groups + src.grp_c);
         }
-    }
+        return b;
+    };
+
+    float inv = 1.f;   // PRO_SILU_FIXED: the RMSNorm factor of the gate and up sums
     float ss_part = 0.f;
     if constexpr (PRO == PRO_SILU_FIXED) ss_part = static_cast<const float*>(xaux)[min((uint32_t)(t & (kWave - 1)), ss_n - 1u)];
+    const NibbleConsts nk = nibble_consts();
 
-    // ---- 2. weight loads ----
+    // ---- the workgroup's K slices: one, or with OUT 1 p.spw of them ----
+    const uint32_t split = blockIdx.x / tiles_a;
+    const uint32_t s0 = OUT ? split * p.spw : split;
+    const uint32_t s1 = OUT ? min(p.splits, s0 + p.spw) : s0 + 1u;
+    long long sum[CPT];
+#pragma unroll
+    for (int cc = 0; cc < CPT; ++cc) sum[cc] = 0;
+#pragma unroll 1
+    for (uint32_t sl = s0; sl < s1; ++sl) {
+    const uint32_t k0 = sl * rps, k1 = min(k, k0 + rps);
+    if constexpr (PRO == PRO_ATTN) attn_merge_rows<NT>(p, k0, k1, rps, xs, aw);
     float acc[32];
 #pragma unroll
     for (int c = 0; c < 32; ++c) acc[c] = 0.f;
-    uint4 wq[FMT == FMT_Q4 ? RPL : 1];
-    uint32_t sq[FMT == FMT_Q4 ? RPL : 1];
-    if constexpr (FMT == FMT_Q4 && TILED) {
-        // one contiguous block per workgroup: step j reads 4 KB, lane t 16 B
-        const uint8_t* bw = tw + (uint64_t)blockIdx.x * (RPL * 4096u) + (uint32_t)t * 16u;
-#pragma unroll
-        for (int j = 0; j < RPL; ++j) wq[j] = *reinterpret_cast<const uint4*>(bw + j * 4096u);
-        // the lane's RPL scales are adjacent
-        const uint16_t* bs = ts + ((uint64_t)blockIdx.x * 256u + (uint32_t)t) * RPL;
-        if constexpr (RPL >= 8) {
-#pragma unroll
-            for (int h = 0; h < RPL / 8; ++h) {
-                const uint4 v = reinterpret_cast<const uint4*>(bs)[h];
-                const uint32_t v4[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    sq[8 * h + 2 * e] = v4[e] & 0xFFFFu;
-                    sq[8 * h + 2 * e + 1] = v4[e] >> 16;
-                }
-            }
-        } else if constexpr (RPL == 4) {
-            const uint2 v = *reinterpret_cast<const uint2*>(bs);
-            sq[0] = v.x & 0xFFFFu; sq[1] = v.x >> 16; sq[2] = v.y & 0xFFFFu; sq[3] = v.y >> 16;
-        } else if constexpr (RPL == 2) {
-            const uint32_t v = *reinterpret_cast<const uint32_t*>(bs);
-            sq[0] = v & 0xFFFFu; sq[1] = v >> 16;
-        } else {
-            sq[0] = bs[0];
-        }
-    } else if constexpr (FMT == FMT_Q4) {
-        const uint64_t row_bytes = (uint64_t)sg.groups * 16u;
-#pragma unroll
-        for (int j = 0; j < RPL; ++j) {
-            const uint32_t r = min(k0 + rl + j * RL, klast);
-            wq[j] = *reinterpret_cast<const uint4*>(sg.w + r * row_bytes + (uint64_t)grp_c * 16u);
-            sq[j] = sg.scales[(uint64_t)r * sg.groups + grp_c];
-        }
-    }
-
-    // ---- 3. the input values ----
     float ssq = 0.f;   // PRO_GAMMA_FIXED: sum of x^2 over this lane's rows
-    if constexpr (PRO == PRO_GAMMA_FIXED) {
+#pragma unroll 1
+    for (uint32_t j0 = 0; j0 < (LOOP ? rpl : (uint32_t)B); j0 += B) {
+        const Batch b = load(k0, j0);
+        if constexpr (PRO == PRO_SILU_FIXED)
+            if (j0 == 0) inv = 1.0f / sqrtf(wave_sum(t % kWave < (int)ss_n ? ss_part : 0.f) / (float)norm_n + 1e-6f);
 #pragma unroll
-        for (int j = 0; j < RPL; ++j) {
-            const bool ok = k0 + rl + j * RL < k1;
-            const float xf = ok ? from_fixed(xa[j]) : 0.f;
-            fix_flag(p.range_flag, ok && fix_out_of_range(xa[j], kFixReadLimit));
-            ssq += xf * xf;
-            xv[j] = xf * h2f((uint16_t)gm[j]);
-        }
-    } else if constexpr (PRO == PRO_SILU_FIXED) {
-        const float inv = 1.0f / sqrtf(wave_sum(t % kWave < (int)ss_n ? ss_part : 0.f) / (float)norm_n + 1e-6f);
-#pragma unroll
-        for (int j = 0; j < RPL; ++j) {
-            const bool ok = k0 + rl + j * RL < k1;
-            xv[j] = ok ? silu_mul(inv * from_fixed(xa[j]), inv * from_fixed(ua[j])) : 0.f;
-        }
-    } else if constexpr (PRO == PRO_PLAIN) {
-#pragma unroll
-        for (int j = 0; j < RPL; ++j) xv[j] = (k0 + rl + j * RL < k1) ? xv[j] : 0.f;
-    } else {
-        attn_merge_rows<NT>(p, k0, k1, KR, xs, aw);
-#pragma unroll
-        for (int j = 0; j < RPL; ++j) xv[j] = xs[rl + j * RL];
-    }
-
-    if constexpr (FMT == FMT_Q4) {
-        const NibbleConsts nk = nibble_consts();
-#pragma unroll
-        for (int j = 0; j < RPL; ++j) {
-            const float sx = h2f((uint16_t)sq[j]) * xv[j];
-            const uint32_t w4[4] = {wq[j].x, wq[j].y, wq[j].z, wq[j].w};
-#pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                const Nib8 nb = unpack_nibbles(w4[d], nk);
-                acc[d * 8 + 0] = fmaf(f16lo(nb.c04), sx, acc[d * 8 + 0]);
-                acc[d * 8 + 4] = fmaf(f16hi(nb.c04), sx, acc[d * 8 + 4]);
-                acc[d * 8 + 1] = fmaf(f16lo(nb.c15), sx, acc[d * 8 + 1]);
-                acc[d * 8 + 5] = fmaf(f16hi(nb.c15), sx, acc[d * 8 + 5]);
-                acc[d * 8 + 2] = fmaf(f16lo(nb.c26), sx, acc[d * 8 + 2]);
-                acc[d * 8 + 6] = fmaf(f16hi(nb.c26), sx, acc[d * 8 + 6]);
-                acc[d * 8 + 3] = fmaf(f16lo(nb.c37), sx, acc[d * 8 + 3]);
-                acc[d * 8 + 7] = fmaf(f16hi(nb.c37), sx, acc[d * 8 + 7]);
+        for (int j = 0; j < B; ++j) {
+            const uint32_t jr = j0 + (uint32_t)j;
+            const bool ok = k0 + rl + jr * RL < k1;
+            float xr = 0.f;
+            if constexpr (PRO == PRO_PLAIN) xr = ok ? b.x[j] : 0.f;
+            if constexpr (PRO == PRO_GAMMA_FIXED) {
+                const float xf = ok ? from_fixed(b.xa[j]) : 0.f;
+                fix_flag(p.range_flag, ok && fix_out_of_range(b.xa[j], kFixReadLimit));
+                ssq += xf * xf;
+                xr = xf * h2f((uint16_t)b.gm[j]);
             }
-        }
-    } else {
-        const uint64_t row_bytes = (uint64_t)sg.groups * 64u;
-        constexpr int B = RPL < 4 ? RPL : 4;   // rows of 64 B in flight per batch
+            if constexpr (PRO == PRO_SILU_FIXED) xr = ok ? silu_mul(inv * from_fixed(b.xa[j]), inv * from_fixed(b.ua[j])) : 0.f;
+            if constexpr (PRO == PRO_ATTN) xr = xs[rl + jr * RL];
+            if constexpr (FMT == FMT_Q4) {
+                const float sx = h2f((uint16_t)b.s[j]) * xr;
 #pragma unroll
-        for (int j0 = 0; j0 < RPL; j0 += B) {
-            uint4 wv[B][4];
-#pragma unroll
-            for (int j = 0; j < B; ++j) {
-                if constexpr (TILED) {
-                    const uint8_t* bw = tw + ((uint64_t)blockIdx.x * RPL + (uint32_t)(j0 + j)) * 16384u +
-                                        (uint32_t)t * 16u;
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) wv[j][v] = *reinterpret_cast<const uint4*>(bw + v * 4096u);
-                } else {
-                    const uint32_t r = min(k0 + rl + (j0 + j) * RL, klast);
-                    const uint4* wsrc = reinterpret_cast<const uint4*>(sg.w + r * row_bytes + (uint64_t)grp_c * 64u);
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) wv[j][v] = wsrc[v];
+                for (int d = 0; d < 4; ++d) {
+                    const Nib8 nb = unpack_nibbles(b.w[j][0][d], nk);
+                    acc[d * 8 + 0] = fmaf(f16lo(nb.c04), sx, acc[d * 8 + 0]);
+                    acc[d * 8 + 4] = fmaf(f16hi(nb.c04), sx, acc[d * 8 + 4]);
+                    acc[d * 8 + 1] = fmaf(f16lo(nb.c15), sx, acc[d * 8 + 1]);
+                    acc[d * 8 + 5] = fmaf(f16hi(nb.c15), sx, acc[d * 8 + 5]);
+                    acc[d * 8 + 2] = fmaf(f16lo(nb.c26), sx, acc[d * 8 + 2]);
+                    acc[d * 8 + 6] = fmaf(f16hi(nb.c26), sx, acc[d * 8 + 6]);
+                    acc[d * 8 + 3] = fmaf(f16lo(nb.c37), sx, acc[d * 8 + 3]);
+                    acc[d * 8 + 7] = fmaf(f16hi(nb.c37), sx, acc[d * 8 + 7]);
                 }
-            }
+            } else {
 #pragma unroll
-            for (int j = 0; j < B; ++j) {
-                const float xr = xv[j0 + j];
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const uint32_t w4[4] = {wv[j][v].x, wv[j][v].y, wv[j][v].z, wv[j][v].w};
+                for (int v = 0; v < 4; ++v)
 #pragma unroll
                     for (int d = 0; d < 4; ++d) {
-                        acc[v * 8 + d * 2 + 0] = fmaf(xr, h2f((uint16_t)(w4[d] & 0xFFFFu)), acc[v * 8 + d * 2 + 0]);
-                        acc[v * 8 + d * 2 + 1] = fmaf(xr, h2f((uint16_t)(w4[d] >> 16)), acc[v * 8 + d * 2 + 1]);
+                        const uint32_t w = b.w[j][v][d];
+                        acc[v * 8 + d * 2 + 0] = fmaf(xr, h2f((uint16_t)(w & 0xFFFFu)), acc[v * 8 + d * 2 + 0]);
+                        acc[v * 8 + d * 2 + 1] = fmaf(xr, h2f((uint16_t)(w >> 16)), acc[v * 8 + d * 2 + 1]);
                     }
-                }
             }
         }
     }
@@ -385,46 +391,109 @@ __global__ __launch_bounds__(256) void gemv_kernel(const uint8_t* tw, const uint
         if ((t & (kWave - 1)) == 0) wred[t / kWave] = ws;
     }
 
-    // ---- reduce the RL row lanes of each group through LDS ----
+    // ---- sum the row lanes of each group: in registers, then the waves through LDS ----
+    const uint32_t rb = OUT ? (sl & 1u) : 0u;
     {
-        float* dst = red + (rl * GT + gi) * RED_STRIDE;
+        float o[GT / 2];
+        const int base = reduce_row_lanes<GT>(acc, o);
+        float4* dst = reinterpret_cast<float4*>(&red[rb][t / kWave][gi * 32 + base]);
 #pragma unroll
-        for (int c = 0; c < 32; ++c) dst[c] = acc[c];
+        for (int i = 0; i < GT / 8; ++i) dst[i] = make_float4(o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]);
     }
     __syncthreads();
     if constexpr (PRO == PRO_GAMMA_FIXED) {
         if (t == 0 && tile == 0) {
             float ws = 0.f;
 #pragma unroll
-            for (int w = 0; w < NT / kWave; ++w) ws += wred[w];
-            p.ss_out[split] = ws;
+            for (int w = 0; w < NW; ++w) ws += wred[w];
+            p.ss_out[sl] = ws;
         }
     }
 #pragma unroll
     for (int cc = 0; cc < CPT; ++cc) {
         const int col = t + cc * NT;
-        const int g = col / 32, c = col % 32;
-        float s = 0.f;
-#pragma unroll 8
-        for (int r = 0; r < RL; ++r) s += red[(r * GT + g) * RED_STRIDE + c];
-        // tile column -> (segment, local column) -> accumulator slot
-        uint32_t local, lim, col0;
-        if (p.paired) {
-            const bool up = g >= GT / 2;
-            local = tile * (COLS / 2) + (uint32_t)(col - (up ? COLS / 2 : 0));
-            lim = (up ? p.seg[1].groups : p.seg[0].groups) * 32u;
-            col0 = up ? p.seg[1].col0 : p.seg[0].col0;
+        const float s = (red[rb][0][col] + red[rb][1][col]) + (red[rb][2][col] + red[rb][3][col]);
+        if constexpr (OUT == 0) {
+            // tile column -> (segment, local column) -> accumulator slot
+            uint32_t local, lim, col0;
+            if (p.paired) {
+                const bool up = col / 32 >= GT / 2;
+                local = tile * (COLS / 2) + (uint32_t)(col - (up ? COLS / 2 : 0));
+                lim = (up ? p.seg[1].groups : p.seg[0].groups) * 32u;
+                col0 = up ? p.seg[1].col0 : p.seg[0].col0;
+            } else {
+                local = (tile - sg.tile0) * COLS + (uint32_t)col;
+                lim = sg.groups * 32u;
+                col0 = sg.col0;
+            }
+            if (local < lim) fixed_add(p.acc + col0 + local, s, p.range_flag);
         } else {
-            local = (tile - sg.tile0) * COLS + (uint32_t)col;
-            lim = sg.groups * 32u;
-            col0 = sg.col0;
+            sum[cc] += fixed_term(s);
         }
-        if (local < lim) fixed_add(p.acc + col0 + local, s, p.range_flag);
     }
-    // the accumulator this launch clears (for a later kernel), after the
-    // launch's own loads
-    if (p.zero_ptr)
-        for (uint32_t i = blockIdx.x * NT + t; i < p.zero_n; i += gridDim.x * NT) p.zero_ptr[i] = 0;
+    }   // slices
+
+    if constexpr (OUT == 0) {
+        // the accumulator this launch clears (for a later kernel), after the
+        // launch's own loads
+        if (p.zero_ptr)
+            for (uint32_t i = blockIdx.x * NT + t; i < p.zero_n; i += gridDim.x * NT) p.zero_ptr[i] = 0;
+    } else {
+        __shared__ uint32_t s_arrived;
+        const uint32_t wgs = (p.splits + p.spw - 1) / p.spw;          // workgroups of the tile
+        if (wgs > 1) {
+            long long* tp = p.part + (uint64_t)tile * wgs * COLS;     // [workgroup][COLS]
+#pragma unroll
+            for (int cc = 0; cc < CPT; ++cc)
+                __hip_atomic_store(tp + split * COLS + (uint32_t)(t + cc * NT), sum[cc], __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's terms are in place
+            __syncthreads();
+            if (t == 0) {
+                uint32_t* cnt = p.count + tile * kGemvCountStride;
+                const uint32_t n = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (n == wgs - 1u) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                s_arrived = n;
+            }
+            __syncthreads();
+            if (s_arrived != wgs - 1u) return;
+            // every workgroup's terms are in place: sum them, 16 loads in
+            // flight a column (indexes clamped, the extra values not added)
+#pragma unroll
+            for (int cc = 0; cc < CPT; ++cc) sum[cc] = 0;
+#pragma unroll 1
+            for (uint32_t z = 0; z < wgs; z += 16) {
+                long long v[CPT][16];
+#pragma unroll
+                for (int u = 0; u < 16; ++u)
+#pragma unroll
+                    for (int cc = 0; cc < CPT; ++cc)
+                        v[cc][u] = __hip_atomic_load(tp + min(z + (uint32_t)u, wgs - 1u) * COLS + (uint32_t)(t + cc * NT),
+                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                for (int u = 0; u < 16; ++u)
+#pragma unroll
+                    for (int cc = 0; cc < CPT; ++cc) sum[cc] += z + (uint32_t)u < wgs ? v[cc][u] : 0;
+            }
+        }
+        if (p.paired) {
+            // gate columns in the tile's first half, up in the second
+            __syncthreads();
+#pragma unroll
+            for (int cc = 0; cc < CPT; ++cc) red[0][0][t + cc * NT] = from_fixed(sum[cc]);
+            __syncthreads();
+            for (int j = t; j < COLS / 2; j += NT) {
+                const uint32_t local = tile * (COLS / 2) + (uint32_t)j;
+                if (local < p.seg[0].groups * 32u) p.y[local] = silu_mul(red[0][0][j], red[0][0][j + COLS / 2]);
+            }
+        } else {
+#pragma unroll
+            for (int cc = 0; cc < CPT; ++cc) {
+                const uint32_t local = tile * COLS + (uint32_t)(t + cc * NT);
+                if (local < p.seg[0].groups * 32u) p.y[local] = from_fixed(sum[cc]);
+            }
+        }
+    }
 }
 
 // acc (fixed point) -> y (fp32); paired: y[j] = silu(acc[j]) * acc[n + j].

@@ -9,6 +9,7 @@
 #include "sample.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <cstdlib>
 
@@ -26,40 +27,56 @@ static int env_int(const char* name, int dflt) {
     return v ? std::atoi(v) : dflt;
 }
 
+// Rows a lane loads at a time in gemv_kernel: four (2048 -> 2048 in F16 4.1
+// against 4.4 us with two at a time).
+static int plan_batch(int rpl) { return std::min(rpl, 4); }
+
 bool plan_gemv(int fmt, uint32_t k, const uint32_t* seg_groups, int nseg, bool paired, int cus,
                GemvPlan* plan, uint32_t row_align) {
     if (k == 0 || nseg < 1 || nseg > 3 || row_align == 0) return false;
     if (paired && (nseg != 2 || seg_groups[0] != seg_groups[1])) return false;
     GemvPlan pl;
-    pl.gt = paired ? 16 : 8;
+    uint64_t groups = 0;
+    for (int i = 0; i < nseg; ++i) groups += seg_groups[i];
+    pl.gt = (paired && fmt == FMT_Q4 && groups >= 512) ? 16 : 8;
     const int forced_gt = env_int("QORA_GEMV_GT", 0);
-    if (!paired && (forced_gt == 8 || forced_gt == 16)) pl.gt = forced_gt;
+    if (forced_gt == 8 || forced_gt == 16) pl.gt = forced_gt;
     if (paired) {
         pl.tiles = (seg_groups[0] + pl.gt / 2 - 1) / (pl.gt / 2);
     } else {
         pl.tiles = 0;
         for (int i = 0; i < nseg; ++i) pl.tiles += (seg_groups[i] + pl.gt - 1) / pl.gt;
     }
-    const uint32_t rl = 256 / pl.gt;
-    const int max_rpl = (fmt == FMT_Q4) ? 16 : 8;
-    const uint32_t target = (uint32_t)std::max(1, cus) * 2;   // ~2 workgroups per CU
-    const uint32_t s_des = std::max(1u, (target + pl.tiles / 2) / pl.tiles);
-    const uint32_t kr_des = (k + s_des - 1) / s_des;
-    const uint32_t rpl_des = std::max(1u, (kr_des + rl - 1) / rl);
-    int rpl = 1;
-    while (rpl < max_rpl && (uint32_t)rpl * 3 / 2 < rpl_des) rpl *= 2;   // nearest power of two
+    const uint32_t rl = 256u / (uint32_t)pl.gt;
+    // K slices of 128 rows (64 where K is short, 256 for a long Q4 one): enough
+    // workgroups without more than the hand-over or the atomics bear. Calls
+    // of the one-launch entry, rows 64 / 128 / 256: 512 -> 512 Q4 4.6 / 4.8 /
+    // 5.7 us, 2048 -> 512 5.4 / 5.0 / 5.8, 11008 -> 2048 - / 11.9 / 10.1; the
+    // decode step's F16 11008 -> 2048 9.9 / 9.7 / 10.7 (gt 8), its gate|up
+    // pair 18.3 / 18.4 / 19.0. Tiles of 16 groups pay for wide Q4 pairs only
+    // (2048 -> 2 x 11008: 12.4 against 14.3 us; F16 18.8 against 18.6).
+    int rpl = (k <= 1024u ? 64 : (fmt == FMT_Q4 && pl.gt == 8 && k > 4096u) ? 256 : 128) / (int)rl;
     const int forced_rpl = env_int("QORA_GEMV_RPL", 0);
-    if ((forced_rpl == 1 || forced_rpl == 2 || forced_rpl == 4 || forced_rpl == 8 || forced_rpl == 16) &&
-        forced_rpl <= max_rpl)
-        rpl = forced_rpl;
-    while (rpl < max_rpl && ((rl * (uint32_t)rpl) % row_align) != 0) rpl *= 2;
+    if (forced_rpl == 1 || forced_rpl == 2 || (forced_rpl > 0 && forced_rpl % 4 == 0)) rpl = forced_rpl;
+    if (row_align > 1) {
+        // the attention merge: whole heads in a slice of at most kGemvAttnRows
+        rpl = 1;
+        while (rpl < 8 && ((rl * (uint32_t)rpl) % row_align != 0 || (rl * (uint32_t)rpl < 128u))) rpl *= 2;
+        if ((rl * (uint32_t)rpl) % row_align != 0 || rl * (uint32_t)rpl > kGemvAttnRows) return false;
+    }
     // at most kFixMaxTerms split-K terms per accumulator between two reads
     // (the fixed-point range guard, params.hpp)
-    while (rpl < max_rpl && (k + rl * (uint32_t)rpl - 1) / (rl * (uint32_t)rpl) > kFixMaxTerms) rpl *= 2;
-    if ((rl * (uint32_t)rpl) % row_align != 0) return false;
+    while ((k + rl * (uint32_t)rpl - 1) / (rl * (uint32_t)rpl) > kFixMaxTerms) {
+        if (row_align > 1 && (rpl >= 8 || 2 * rl * (uint32_t)rpl > kGemvAttnRows)) break;
+        rpl *= 2;
+    }
     pl.rpl = rpl;
     pl.kr = rl * (uint32_t)rpl;
     pl.splits = (k + pl.kr - 1) / pl.kr;
+    // slices per workgroup of a one-launch GEMV: about 2.5 sqrt(k) rows, since
+    // the last workgroup's sum grows with their number (11008 -> 2048 in F16,
+    // 86 slices: 14.9 us one by one, 13.3 two by two, 13.5 three by three)
+    pl.spw = (uint32_t)std::max(1.0, 2.5 * std::sqrt((double)k) / pl.kr + 0.5);
     *plan = pl;
     return true;
 }
@@ -140,6 +157,7 @@ void apply_plan(const GemvPlan& plan, GemvParams* p) {
     p->tiles = plan.tiles;
     p->splits = plan.splits;
     p->rows_per_split = plan.kr;
+    p->spw = plan.spw;
     // XCD order for the prologues that read a previous kernel's output (bit
     // = prologue): each XCD's L2 then fetches the inputs of its own K slices
     // only. The plain prologue's input is one small vector; it keeps launch
@@ -149,9 +167,9 @@ void apply_plan(const GemvPlan& plan, GemvParams* p) {
     p->xcd_order = (uint32_t)(xcd_mask >> p->pro) & 1u;
 }
 
-template <int FMT, int GT, int PRO, bool TILED>
+template <int FMT, int GT, int PRO, bool TILED, int OUT>
 static hipError_t launch_gemv_pro(const GemvPlan& plan, const GemvParams& p, hipStream_t stream) {
-    const dim3 grid(plan.blocks()), block(256);
+    const dim3 grid(OUT ? plan.tiles * plan.wgs() : plan.blocks()), block(256);
     // the first loads' arguments ahead of the parameter block (preloaded into
     // scalar registers at wave launch); ss_n | norm_n << 8 in one word
     if (p.ss_n > 0xFFu || p.norm_n >= (1u << 24)) return hipErrorInvalidValue;
@@ -159,21 +177,18 @@ static hipError_t launch_gemv_pro(const GemvPlan& plan, const GemvParams& p, hip
     const void* xaux = PRO == PRO_GAMMA_FIXED ? static_cast<const void*>(p.gamma)
                                               : static_cast<const void*>(p.ss_in);
     const uint32_t ss_nn = p.ss_n | (p.norm_n << 8);
-#define QORA_GEMV_ARGS p.tw, p.ts, xin, xaux, p.k, p.tiles, p.rows_per_split, ss_nn, p
-    switch (plan.rpl) {
-    case 1: hipLaunchKernelGGL((gemv_kernel<FMT, GT, 1, PRO, TILED>), grid, block, 0, stream, QORA_GEMV_ARGS); break;
-    case 2: hipLaunchKernelGGL((gemv_kernel<FMT, GT, 2, PRO, TILED>), grid, block, 0, stream, QORA_GEMV_ARGS); break;
-    case 4: hipLaunchKernelGGL((gemv_kernel<FMT, GT, 4, PRO, TILED>), grid, block, 0, stream, QORA_GEMV_ARGS); break;
-    case 8: hipLaunchKernelGGL((gemv_kernel<FMT, GT, 8, PRO, TILED>), grid, block, 0, stream, QORA_GEMV_ARGS); break;
-    case 16:
-        if constexpr (FMT == FMT_Q4) {
-            hipLaunchKernelGGL((gemv_kernel<FMT, GT, 16, PRO, TILED>), grid, block, 0, stream, QORA_GEMV_ARGS);
-            break;
-        }
+#define QORA_GEMV_B(B_, LOOP_)                                                                                     \
+    hipLaunchKernelGGL((gemv_kernel<FMT, GT, B_, LOOP_, PRO, TILED, OUT>), grid, block, 0, stream, p.tw, xin, xaux, p.k, \
+                       p.tiles, p.rows_per_split, ss_nn, p)
+    const int b = plan_batch(plan.rpl);
+    if (plan.rpl < 1 || plan.rpl % b != 0 || p.rows_per_split != (256u / GT) * (uint32_t)plan.rpl ||
+        (PRO == PRO_ATTN && p.rows_per_split > kGemvAttnRows))
         return hipErrorInvalidValue;
-    default: return hipErrorInvalidValue;
-    }
-#undef QORA_GEMV_ARGS
+    if (b == 1) QORA_GEMV_B(1, false);
+    else if (b == 2) QORA_GEMV_B(2, false);
+    else if (plan.rpl == 4) QORA_GEMV_B(4, false);
+    else QORA_GEMV_B(4, true);
+#undef QORA_GEMV_B
     return hipGetLastError();
 }
 
@@ -182,16 +197,20 @@ static hipError_t launch_gemv_gt(const GemvPlan& plan, const GemvParams& p, hipS
     if (!p.tw) {
         // reference layout: the kernel-level plain GEMV entry points only
         if (p.pro != PRO_PLAIN) return hipErrorInvalidValue;
-        return launch_gemv_pro<FMT, GT, PRO_PLAIN, false>(plan, p, stream);
+        if (p.y) {
+            if (p.spw != plan.spw || p.spw == 0 || (plan.wgs() > 1 && (!p.part || !p.count))) return hipErrorInvalidValue;
+            return launch_gemv_pro<FMT, GT, PRO_PLAIN, false, 1>(plan, p, stream);
+        }
+        return launch_gemv_pro<FMT, GT, PRO_PLAIN, false, 0>(plan, p, stream);
     }
     if constexpr (FMT == FMT_Q4) {
         return hipErrorInvalidValue;   // the Q4 tile layout runs on the matrix cores (launch_q4m_*)
     } else {
         switch (p.pro) {
-        case PRO_PLAIN: return launch_gemv_pro<FMT, GT, PRO_PLAIN, true>(plan, p, stream);
-        case PRO_GAMMA_FIXED: return launch_gemv_pro<FMT, GT, PRO_GAMMA_FIXED, true>(plan, p, stream);
-        case PRO_SILU_FIXED: return launch_gemv_pro<FMT, GT, PRO_SILU_FIXED, true>(plan, p, stream);
-        case PRO_ATTN: return launch_gemv_pro<FMT, GT, PRO_ATTN, true>(plan, p, stream);
+        case PRO_PLAIN: return launch_gemv_pro<FMT, GT, PRO_PLAIN, true, 0>(plan, p, stream);
+        case PRO_GAMMA_FIXED: return launch_gemv_pro<FMT, GT, PRO_GAMMA_FIXED, true, 0>(plan, p, stream);
+        case PRO_SILU_FIXED: return launch_gemv_pro<FMT, GT, PRO_SILU_FIXED, true, 0>(plan, p, stream);
+        case PRO_ATTN: return launch_gemv_pro<FMT, GT, PRO_ATTN, true, 0>(plan, p, stream);
         default: return hipErrorInvalidValue;
         }
     }
@@ -287,9 +306,9 @@ void gemv_tile_bytes(int fmt, const GemvPlan& plan, uint64_t* w_bytes, uint64_t*
         *e_bytes = waves * (uint64_t)plan.gw;
         return;
     }
-    const uint64_t steps = (uint64_t)plan.blocks() * (uint64_t)plan.rpl;
-    *w_bytes = steps * 256u * (fmt == FMT_Q4 ? 16u : 64u);
-    *s_bytes = fmt == FMT_Q4 ? steps * 256u * 2u : 0u;
+    // F16 (the Q4 VALU kernel reads the reference layout)
+    *w_bytes = (uint64_t)plan.blocks() * (uint64_t)plan.rpl * 256u * 64u;
+    *s_bytes = 0;
     *e_bytes = 0;
 }
 
@@ -305,14 +324,8 @@ hipError_t launch_gemv_tile(int fmt, const GemvPlan& plan, const GemvParams& p, 
     }
     const uint64_t grid = (uint64_t)plan.blocks() * (uint64_t)plan.rpl;
     if (grid == 0 || grid > 0x7FFFFFFFull) return hipErrorInvalidValue;
-    if (fmt == FMT_Q4) {
-        if (!ts) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(gemv_tile_kernel<FMT_Q4>, dim3((uint32_t)grid), dim3(256), 0, stream, p, plan.gt, plan.rpl,
-                           tw, ts);
-    } else {
-        hipLaunchKernelGGL(gemv_tile_kernel<FMT_F16>, dim3((uint32_t)grid), dim3(256), 0, stream, p, plan.gt,
-                           plan.rpl, tw, ts);
-    }
+    if (fmt == FMT_Q4) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(gemv_tile_kernel, dim3((uint32_t)grid), dim3(256), 0, stream, p, plan.gt, plan.rpl, tw);
     return hipGetLastError();
 }
 

@@ -22,8 +22,10 @@ struct GemvPlan {
     uint32_t kr = 0;      // rows per K slice
     int mfma = 0;         // 1: Q4 on the matrix cores (gemv_q4m_kernel): gt = 4*gw, kr = kw
     int gw = 0;           // groups per wave (MFMA kernel)
+    uint32_t spw = 1;     // K slices per workgroup of a one-launch GEMV (p.y)
     int ipw = 1;          // work items (tile, K slice) per workgroup (MFMA kernel)
     uint32_t blocks() const { return tiles * splits; }                // work items
+    uint32_t wgs() const { return (splits + spw - 1) / spw; }        // workgroups per column tile (p.y)
     uint32_t grid() const { return (blocks() + (uint32_t)ipw - 1) / (uint32_t)ipw; }
 };
 
@@ -49,7 +51,9 @@ bool plan_gemv_q4m(uint32_t k, const uint32_t* seg_groups, int nseg, bool paired
 void apply_plan(const GemvPlan& plan, GemvParams* p);
 
 // p.tw == nullptr: reference layout, plain prologue only (kernel-level
-// entry points). Otherwise the tile layout written by launch_gemv_tile.
+// entry points); with p.y set the launch writes y itself (p.part and p.count
+// when the plan splits K) instead of adding to p.acc. Otherwise the tile
+// layout written by launch_gemv_tile.
 hipError_t launch_gemv(int fmt, const GemvPlan& plan, const GemvParams& p, hipStream_t stream);
 // Size of the tile layout of a planned GEMV (scales, exponent bounds: Q4 only).
 void gemv_tile_bytes(int fmt, const GemvPlan& plan, uint64_t* w_bytes, uint64_t* s_bytes, uint64_t* e_bytes);

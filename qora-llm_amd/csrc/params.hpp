@@ -33,6 +33,9 @@ constexpr long long kFixReadLimit = 1LL << 61;
 constexpr long long kFixAddLimit = 1LL << 56;
 constexpr uint32_t kFixMaxTerms = 96;
 
+constexpr uint32_t kGemvAttnRows = 256;      // most rows per K slice of gemv_kernel's attention-merge prologue
+constexpr uint32_t kGemvCountStride = 16;   // gemv_kernel's tile counters, u32 words apart (64 bytes)
+
 struct GemvSeg {
     const uint8_t* w;         // Q4 packed bytes or F16 words (as bytes), reference layout
     const uint16_t* scales;   // Q4 only
@@ -67,8 +70,8 @@ struct GemvParams {
     uint32_t zero_n;
     // Tile layout (set by gemv_tile_kernel): the bytes every workgroup loads,
     // stored in load order so each workgroup streams one contiguous block.
-    //   Q4 : tw[block][j < RPL][lane < 256] x 16 B, ts[block][lane][j] scales
-    //   F16: tw[block][j][v < 4][lane] x 16 B
+    //   F16: tw[block][j < RPL][v < 4][lane < 256] x 16 B
+    //   Q4 (matrix cores): gemv_q4m_pack_kernel
     // The segment pointers then only describe the shape.
     const uint8_t* tw;
     const uint16_t* ts;
@@ -76,6 +79,14 @@ struct GemvParams {
     // exponent bound of the K slice's scales, max |s| <= 2^tes.
     const int8_t* tes;
     int* range_flag;          // optional: set when a fixed-point value leaves its range
+    // gemv_kernel with OUT 1 (y instead of acc): K slices per workgroup, the
+    // workgroups' fixed-point terms [tiles][ceil(splits / spw)][gt * 32], one
+    // arrival counter per column tile (0 before and after every launch), the
+    // output
+    uint32_t spw;
+    long long* part;
+    uint32_t* count;
+    float* y;
     // 1: the matrix-core kernels run item xcd_item(b, G) in workgroup b
     // (each XCD takes a contiguous run of items); 0: item b
     uint32_t xcd_order;
