@@ -191,13 +191,13 @@ struct qora_hip_ctx {
     std::vector<DevWeight> weights;
     long long* ws_acc = nullptr;         // kernel-level fixed-point accumulator
     uint64_t ws_acc_n = 0;
-    // one-launch GEMV entries: the K slices' terms, and the column tiles'
-    // arrival counters (0 between calls; only calls on the context's own
-    // stream outside a capture use them, one behind the other)
-    long long* ws_part = nullptr;
-    uint64_t ws_part_n = 0;
+    // one-launch GEMV entries: the column tiles' sums behind the accumulator and
+    // their arrival counters ahead of it, all 0 between calls, used only by calls
+    // on the context's own stream outside a capture (one behind the other)
+    long long* ws_sum = nullptr;
     uint32_t* ws_count = nullptr;
-    uint64_t ws_count_n = 0;
+    uint64_t ws_tiles = 0;
+    std::vector<void*> ws_old;           // outgrown ones: a captured graph may still use them
     // on-device sampling scratch (grown to the largest vocab seen)
     float* smp_work = nullptr;
     unsigned long long* smp_cand = nullptr;
@@ -260,54 +260,29 @@ int dalloc(qora_hip_ctx* c, size_t bytes, void** p) {
 
 hipStream_t pick_stream(qora_hip_ctx* c, void* s) { return s ? reinterpret_cast<hipStream_t>(s) : c->stream; }
 
-// Grow the kernel-level scratch (fixed-point accumulator, attention partials).
-int ensure_acc_ws(qora_hip_ctx* c, uint64_t n) {
-    if (n <= c->ws_acc_n) return QORA_HIP_OK;
+// Grow the kernel-level scratch: one allocation of tile counters, the
+// fixed-point accumulator (n words) and the one-launch GEMVs' sums (a tile has
+// at most 512 columns, the last one partly past n).
+int ensure_acc_ws(qora_hip_ctx* c, uint64_t n, uint64_t tiles = 0) {
+    if (n <= c->ws_acc_n && tiles <= c->ws_tiles) return QORA_HIP_OK;
     if (c->capturing) return fail(c, QORA_HIP_E_STATE, "scratch must be sized by an eager call before capture");
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    if (c->ws_acc) (void)hipFree(c->ws_acc);
-    c->ws_acc = nullptr;
-    c->ws_acc_n = 0;
+    // (each growth at least doubles: the outgrown ones together stay below the current)
+    const uint64_t nn = std::max<uint64_t>({n, 2 * c->ws_acc_n, 32768});
+    const uint64_t nt = std::max<uint64_t>({tiles, 2 * c->ws_tiles, (nn + 255) / 256 + 8});
+    const uint64_t cb = nt * kGemvCountStride * sizeof(uint32_t), sw = nn + 512;
     void* p;
-    const uint64_t nn = n < 65536 ? 65536 : n;
-    if (int rc = dalloc(c, nn * sizeof(long long), &p)) return rc;
-    c->ws_acc = (long long*)p;
+    if (int rc = dalloc(c, cb + (nn + sw) * sizeof(long long), &p)) return rc;
+    const hipError_t e = hipMemsetAsync(p, 0, cb + (nn + sw) * sizeof(long long), c->stream);
+    if (e != hipSuccess) {
+        (void)hipFree(p);
+        return fail(c, QORA_HIP_E_DEVICE, std::string("GEMV scratch: ") + hipGetErrorString(e));
+    }
+    if (c->ws_count) c->ws_old.push_back(c->ws_count);
+    c->ws_count = (uint32_t*)p;
+    c->ws_tiles = nt;
+    c->ws_acc = (long long*)((uint8_t*)p + cb);
     c->ws_acc_n = nn;
-    return QORA_HIP_OK;
-}
-
-// Terms and counters of a one-launch GEMV of `terms` int64 words and `tiles`
-// column tiles. qora_hip_create asks for kGemvWsTerms and kGemvWsTiles once
-// (the largest GEMV of SmolLM3-3B takes 352256 terms), so that a first call
-// allocates nothing here.
-constexpr uint64_t kGemvWsTerms = 1u << 19, kGemvWsTiles = 256;
-
-int ensure_gemv_ws(qora_hip_ctx* c, uint64_t terms, uint64_t tiles) {
-    const uint64_t words = tiles * kGemvCountStride;
-    if (terms <= c->ws_part_n && words <= c->ws_count_n) return QORA_HIP_OK;
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    void* p;
-    if (terms > c->ws_part_n) {
-        if (c->ws_part) (void)hipFree(c->ws_part);
-        c->ws_part = nullptr;
-        c->ws_part_n = 0;
-        if (int rc = dalloc(c, terms * sizeof(long long), &p)) return rc;
-        c->ws_part = (long long*)p;
-        c->ws_part_n = terms;
-    }
-    if (words > c->ws_count_n) {
-        if (c->ws_count) (void)hipFree(c->ws_count);
-        c->ws_count = nullptr;
-        c->ws_count_n = 0;
-        if (int rc = dalloc(c, words * sizeof(uint32_t), &p)) return rc;
-        const hipError_t e = hipMemsetAsync(p, 0, words * sizeof(uint32_t), c->stream);
-        if (e != hipSuccess) {
-            (void)hipFree(p);
-            return fail(c, QORA_HIP_E_DEVICE, std::string("GEMV counters: ") + hipGetErrorString(e));
-        }
-        c->ws_count = (uint32_t*)p;
-        c->ws_count_n = words;
-    }
+    c->ws_sum = c->ws_acc + nn;
     return QORA_HIP_OK;
 }
 
@@ -564,8 +539,6 @@ extern "C" int qora_hip_create(int device, qora_hip_ctx** out) {
     } else {
         c->h_tok = nullptr;
     }
-    // (without room for it here the first GEMV call asks again and reports it)
-    (void)ensure_gemv_ws(c, kGemvWsTerms, kGemvWsTiles);
     *out = c;
     return QORA_HIP_OK;
 }
@@ -582,9 +555,10 @@ extern "C" int qora_hip_destroy(qora_hip_ctx* c) {
         if (w.w) (void)hipFree(w.w);
         if (w.scales) (void)hipFree(w.scales);
     }
-    for (void* p : {(void*)c->ws_acc, (void*)c->ws_part, (void*)c->ws_count, (void*)c->ws_attn_part, c->ws_pf, (void*)c->smp_work, (void*)c->smp_cand,
+    for (void* p : {(void*)c->ws_count, (void*)c->ws_attn_part, c->ws_pf, (void*)c->smp_work, (void*)c->smp_cand,
                     (void*)c->smp_rng, (void*)c->smp_pen, c->smp_sort})
         if (p) (void)hipFree(p);
+    for (void* p : c->ws_old) (void)hipFree(p);
     if (c->h_pin) (void)hipHostFree(c->h_pin);
     if (c->h_pen) (void)hipHostFree(c->h_pen);
     if (c->h_tok) (void)hipHostFree(c->h_tok);
@@ -1777,21 +1751,20 @@ int gemv_entry(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, const v
     if (!y) return fail(c, QORA_HIP_E_INVALID, "null argument");
     if (n == 0 || n > 0x7FFFFFFFull) return fail(c, QORA_HIP_E_INVALID, "GEMV needs 0 < n < 2^31");
     const hipStream_t s = pick_stream(c, stream);
-    // (an eager call also sizes what a captured one will need)
     const uint64_t accn = paired ? 2 * n : n;
-    if (int rc = ensure_acc_ws(c, accn)) return rc;
     if (in_order(c, s)) {
         GemvPlan pl;
         GemvParams p{};
         if (int rc = gemv_prepare_launch(c, fmt, w0, s0, w1, s1, x, k, n, paired, &pl, &p)) return rc;
-        if (pl.wgs() > 1)
-            if (int rc = ensure_gemv_ws(c, (uint64_t)pl.tiles * pl.wgs() * (uint64_t)pl.gt * 32u, pl.tiles)) return rc;
+        // (also sizes what the same call needs in a capture)
+        if (int rc = ensure_acc_ws(c, accn, pl.tiles)) return rc;
         p.y = y;
-        p.part = c->ws_part;
+        p.part = c->ws_sum;
         p.count = c->ws_count;
         HIP_TRY(c, launch_gemv(fmt, pl, p, s));
         return QORA_HIP_OK;
     }
+    if (int rc = ensure_acc_ws(c, accn)) return rc;
     HIP_TRY(c, launch_fill_zero(c->ws_acc, accn, s));
     if (int rc = gemv_acc_entry(c, fmt, w0, s0, w1, s1, x, c->ws_acc, k, n, paired, stream)) return rc;
     HIP_TRY(c, launch_acc_to_f32(c->ws_acc, (uint32_t)n, paired ? 1 : 0, y, s));

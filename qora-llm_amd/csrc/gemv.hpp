@@ -221,13 +221,12 @@ __device__ __forceinline__ int reduce_row_lanes(const float (&acc)[32], float (&
 }
 
 // OUT: 0 adds the slice's sums to the fixed-point accumulator p.acc with
-// atomics. 1 leaves them (the same fixed-point terms) in p.part and the last
-// workgroup of a column tile to arrive (p.count, one counter per tile) sums the
-// tile's terms and writes y, SiLU(gate) * up when paired: clear, accumulate
-// and convert in one launch. The terms travel by agent-scope stores and loads
-// (each wave waits for its stores' acknowledgement before the tile's count),
-// so no L2 write-back is needed; the last arriver sets the counter back to 0.
-//
+// atomics. 1 adds them to the column tile's sums in p.part, and the last
+// workgroup of the tile to arrive (p.count, one counter per tile) reads the sums,
+// writes y, SiLU(gate) * up when paired, and sets the sums and the counter back
+// to 0: clear, accumulate and convert in one launch. The sums travel by
+// agent-scope atomics only (each wave waits for its own before the tile's count),
+// so no L2 write-back is needed.
 // What bounds it: F16 the weight stream (2048 -> 2 x 11008 at 4.9 TB/s, a large
 // copy's rate), Q4 the unpacking on the VALU (17 instructions per 8 weights;
 // the same pair at 2.0 TB/s), small shapes the launch and the hand-over (1.5 us
@@ -442,12 +441,11 @@ __global__ __launch_bounds__(256) void gemv_kernel(const uint8_t* tw, const void
         __shared__ uint32_t s_arrived;
         const uint32_t wgs = (p.splits + p.spw - 1) / p.spw;          // workgroups of the tile
         if (wgs > 1) {
-            long long* tp = p.part + (uint64_t)tile * wgs * COLS;     // [workgroup][COLS]
+            long long* tp = p.part + (uint64_t)tile * COLS;           // the tile's sums
 #pragma unroll
             for (int cc = 0; cc < CPT; ++cc)
-                __hip_atomic_store(tp + split * COLS + (uint32_t)(t + cc * NT), sum[cc], __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's terms are in place
+                atomicAdd(reinterpret_cast<unsigned long long*>(tp + t + cc * NT), (unsigned long long)sum[cc]);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's terms are added
             __syncthreads();
             if (t == 0) {
                 uint32_t* cnt = p.count + tile * kGemvCountStride;
@@ -457,24 +455,12 @@ __global__ __launch_bounds__(256) void gemv_kernel(const uint8_t* tw, const void
             }
             __syncthreads();
             if (s_arrived != wgs - 1u) return;
-            // every workgroup's terms are in place: sum them, 16 loads in
-            // flight a column (indexes clamped, the extra values not added)
 #pragma unroll
-            for (int cc = 0; cc < CPT; ++cc) sum[cc] = 0;
-#pragma unroll 1
-            for (uint32_t z = 0; z < wgs; z += 16) {
-                long long v[CPT][16];
+            for (int cc = 0; cc < CPT; ++cc)
+                sum[cc] = __hip_atomic_load(tp + t + cc * NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-                for (int u = 0; u < 16; ++u)
-#pragma unroll
-                    for (int cc = 0; cc < CPT; ++cc)
-                        v[cc][u] = __hip_atomic_load(tp + min(z + (uint32_t)u, wgs - 1u) * COLS + (uint32_t)(t + cc * NT),
-                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-                for (int u = 0; u < 16; ++u)
-#pragma unroll
-                    for (int cc = 0; cc < CPT; ++cc) sum[cc] += z + (uint32_t)u < wgs ? v[cc][u] : 0;
-            }
+            for (int cc = 0; cc < CPT; ++cc)
+                __hip_atomic_store(tp + t + cc * NT, 0LL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (p.paired) {
             // gate columns in the tile's first half, up in the second

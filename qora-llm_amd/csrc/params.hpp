@@ -80,9 +80,8 @@ struct GemvParams {
     const int8_t* tes;
     int* range_flag;          // optional: set when a fixed-point value leaves its range
     // gemv_kernel with OUT 1 (y instead of acc): K slices per workgroup, the
-    // workgroups' fixed-point terms [tiles][ceil(splits / spw)][gt * 32], one
-    // arrival counter per column tile (0 before and after every launch), the
-    // output
+    // column tiles' fixed-point sums [tiles][gt * 32] and one arrival counter per
+    // tile (both 0 before and after every launch), the output
     uint32_t spw;
     long long* part;
     uint32_t* count;
