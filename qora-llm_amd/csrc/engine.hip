@@ -2078,15 +2078,38 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
     if (T == 0 || T > 0x7FFFFFFFull) return fail(c, QORA_HIP_E_INVALID, "bad row count");
     if (!pf_gemm_supported((uint32_t)w->k, (uint32_t)w->n)) return fail(c, QORA_HIP_E_INVALID, "k must be a multiple of 32");
     const uint32_t K = (uint32_t)w->k, N = (uint32_t)w->n;
-    // Q4 with n % 128 == 0 runs the prefill's packed-weight GEMM (the weight
-    // packed into the workspace for this call), anything else pf_gemm_kernel
-    const bool packed = w->fmt == FMT_Q4 && pf_gemm2_supported(K, N);
-    // scratch: xh, xl [T][k] binary16, xe [T], wf [n/32], exponent partials,
-    // then the packed weight (wq, sc) or nothing, then the split-K partials
-    // (each part 256-byte aligned)
+    const hipStream_t s = pick_stream(c, stream);
     auto al = [](uint64_t b) { return (b + 255) & ~uint64_t(255); };
-    const uint64_t bx = al(T * K * 2), be = al(T * 4), bf = al(N / 32 + 1);
-    const uint64_t bs = al(pf_weight_exp_scratch(K, N / 32));
+    if (T <= kPfSmallT) {
+        // a few tokens: straight from the weight as it was uploaded
+        PfSmallParams q{};
+        q.x = x;
+        q.T = (uint32_t)T;
+        q.k = K;
+        q.n = N;
+        q.w = (const uint8_t*)w->w;
+        q.scales = (const uint16_t*)w->scales;
+        q.y = y;
+        const PfSmallShape sh = pf_small_shape(q.T, K, N, c->cus);
+        q.splits = sh.splits;
+        q.kper = sh.kper;
+        if (sh.splits > 1) {
+            if (int rc = ensure_pf_ws(c, al((uint64_t)sh.splits * T * N * 4))) return rc;
+            q.part = (float*)c->ws_pf;
+        }
+        HIP_TRY(c, launch_pf_gemm_small(w->fmt, q, s));
+        return QORA_HIP_OK;
+    }
+    // Q4 with n % 128 == 0 runs the prefill's packed-weight GEMM (the weight
+    // packed into the workspace for this call, with its own scales), anything
+    // else pf_gemm_kernel
+    const bool packed = w->fmt == FMT_Q4 && pf_gemm2_supported(K, N);
+    const bool exps = w->fmt == FMT_Q4 && !packed;
+    // scratch: xh, xl [T][k] binary16, xe [T], then the packed weight (wq, sc)
+    // or wf [n/32] and the exponent partials, then the split-K partials (each
+    // part 256-byte aligned)
+    const uint64_t bx = al(T * K * 2), be = al(T * 4), bf = exps ? al(N / 32 + 1) : 0;
+    const uint64_t bs = exps ? al(pf_weight_exp_scratch(K, N / 32)) : 0;
     const uint64_t bq = packed ? al((uint64_t)K * N / 2) : 0, bc = packed ? al((uint64_t)K * N / 16) : 0;
     const PfGemmShape sh = pf_gemm_shape((uint32_t)T, K, N, c->cus);
     const PfGemm2Shape s2 = packed ? pf_gemm2_shape((uint32_t)T, K, N, c->cus) : PfGemm2Shape{};
@@ -2096,20 +2119,15 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
     uint8_t* base = (uint8_t*)c->ws_pf;
     uint8_t* wq = base + 2 * bx + be + bf + bs;
     float* part = splits > 1 ? (float*)(wq + bq + bc) : nullptr;
-    const hipStream_t s = pick_stream(c, stream);
     PrefillRowParams r{};
     r.x = const_cast<float*>(x);
     r.n = K;
     r.xh = (uint16_t*)base;
     r.xl = (uint16_t*)(base + bx);
     r.xe = (int32_t*)(base + 2 * bx);
-    HIP_TRY(c, launch_pf_rows(PF_ROW_SPLIT, r, (uint32_t)T, s));
-    int8_t* wf = (int8_t*)(base + 2 * bx + be);
-    if (w->fmt == FMT_Q4)
-        HIP_TRY(c, launch_pf_weight_exp((const uint16_t*)w->scales, K, N / 32, wf, (uint32_t*)(base + 2 * bx + be + bf), s));
     if (packed) {
-        HIP_TRY(c, launch_pf_pack_q4((const uint8_t*)w->w, (const uint16_t*)w->scales, wf, K, N, (uint2*)wq,
-                                     (uint16_t*)(wq + bq), s));
+        HIP_TRY(c, launch_pf_gemm_prep(x, (uint32_t)T, r.xh, r.xl, r.xe, (const uint8_t*)w->w, (const uint16_t*)w->scales,
+                                       K, N, (uint2*)wq, (uint16_t*)(wq + bq), s));
         PfGemm2Params h{};
         h.xh = r.xh;
         h.xl = r.xl;
@@ -2118,13 +2136,17 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
         h.k = K;
         h.nseg = 1;
         h.ntot = N;
-        h.seg[0] = PfGemm2Seg{(const uint2*)wq, (const uint16_t*)(wq + bq), wf, N, 0, y, N, 0};
+        h.seg[0] = PfGemm2Seg{(const uint2*)wq, (const uint16_t*)(wq + bq), nullptr, N, 0, y, N, 0};
         h.splits = s2.splits;
         h.kper = s2.kper;
         h.part = part;
-        HIP_TRY(c, launch_pf_gemm2(s2.bm, h, s));
+        HIP_TRY(c, launch_pf_gemm2(s2.bm, h, s, true, true));
         return QORA_HIP_OK;
     }
+    HIP_TRY(c, launch_pf_rows(PF_ROW_SPLIT, r, (uint32_t)T, s));
+    int8_t* wf = (int8_t*)(base + 2 * bx + be);
+    if (exps)
+        HIP_TRY(c, launch_pf_weight_exp((const uint16_t*)w->scales, K, N / 32, wf, (uint32_t*)(base + 2 * bx + be + bf), s));
     PrefillGemmParams g{};
     g.xh = r.xh;
     g.xl = r.xl;
@@ -2134,7 +2156,7 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
     g.n = N;
     g.w = (const uint8_t*)w->w;
     g.scales = (const uint16_t*)w->scales;
-    g.wf = w->fmt == FMT_Q4 ? wf : nullptr;
+    g.wf = exps ? wf : nullptr;
     g.y = y;
     g.ldy = N;
     g.nt = sh.nt;

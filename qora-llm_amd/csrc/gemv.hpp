@@ -235,8 +235,8 @@ __device__ __forceinline__ int reduce_row_lanes(const float (&acc)[32], float (&
 // registers (reduce_row_lanes) and the four waves through 4 or 8 KB of LDS.
 // Before, weights came by flat loads (each wait drained every load), each lane
 // put 32 sums into 34 KB of LDS (four workgroups a CU), and a call took three
-// launches: one token's MLP (norm, gate|up, down) 22.0 -> 13.8 us in Q4 and 32.3
-// -> 27.5 us in F16, 2048 -> 512 9.4 -> 4.1 us a call.
+// launches: one token's MLP (norm, gate|up, down) 22.3 -> 13.2 us in Q4 and 32.4
+// -> 26.3 us in F16, 2048 -> 512 9.4 -> 4.1 us a call.
 template <int FMT, int GT, int B, bool LOOP, int PRO, bool TILED, int OUT>
 __global__ __launch_bounds__(256) void gemv_kernel(const uint8_t* tw, const void* xin,
                                                    const void* xaux, uint32_t k, uint32_t tiles_a, uint32_t rps,

@@ -728,6 +728,54 @@ hipError_t launch_pf_pack_q4(const uint8_t* w, const uint16_t* scales, const int
     return hipGetLastError();
 }
 
+hipError_t launch_pf_gemm_prep(const float* x, uint32_t T, uint16_t* xh, uint16_t* xl, int32_t* xe, const uint8_t* w,
+                               const uint16_t* scales, uint32_t k, uint32_t n, uint2* wq, uint16_t* sc,
+                               hipStream_t stream) {
+    if (!pf_gemm2_supported(k, n) || T == 0) return hipErrorInvalidValue;
+    const uint64_t grid = (uint64_t)T + (uint64_t)(n / 128u) * ((k / 32u + 1u) / 2u);
+    if (grid > 0x7FFFFFFFull) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(pf_gemm_prep_kernel, dim3((uint32_t)grid), dim3(256), 0, stream, x, xh, xl, xe, T, w, scales, k,
+                       n, wq, sc);
+    return hipGetLastError();
+}
+
+// K slices of pf_gemm_small_kernel: the longest its LDS takes (512 rows, 256
+// above 32 tokens), halved down to 128 while the blocks do not fill the CUs
+// (each slice adds T n partial sums to write and read).
+PfSmallShape pf_small_shape(uint32_t T, uint32_t k, uint32_t n, int cus) {
+    PfSmallShape sh{};
+    const uint32_t blocks = (n + 127u) / 128u;
+    uint32_t kper = T > 32u ? 256u : 512u;
+    while (kper > 128u && (uint64_t)blocks * ((k + kper - 1u) / kper) < (uint64_t)std::max(1, cus)) kper /= 2u;
+    sh.kper = kper;
+    sh.splits = (k + kper - 1u) / kper;
+    return sh;
+}
+
+hipError_t launch_pf_gemm_small(int fmt, const PfSmallParams& p, hipStream_t stream) {
+    if (p.T == 0 || p.T > kPfSmallT || !pf_gemm_supported(p.k, p.n) || p.n % 32 != 0 || p.kper % 32 != 0 || p.kper == 0 ||
+        p.kper > (p.T > 32u ? 256u : 512u) || (uint64_t)p.splits * p.kper < p.k ||
+        (uint64_t)(p.splits - 1u) * p.kper >= p.k || p.splits > 65535u || (p.splits > 1 && !p.part))
+        return hipErrorInvalidValue;
+    const dim3 grid((p.n + 127u) / 128u, p.splits);
+#define QORA_PF_SMALL(TM_)                                                                                    \
+    do {                                                                                                      \
+        if (fmt == FMT_Q4) hipLaunchKernelGGL((pf_gemm_small_kernel<TM_, true>), grid, dim3(256), 0, stream, p); \
+        else hipLaunchKernelGGL((pf_gemm_small_kernel<TM_, false>), grid, dim3(256), 0, stream, p);           \
+    } while (0)
+    if (p.T <= 16u) QORA_PF_SMALL(1);
+    else if (p.T <= 32u) QORA_PF_SMALL(2);
+    else QORA_PF_SMALL(4);
+#undef QORA_PF_SMALL
+    if (p.splits > 1) {
+        const uint64_t total = (uint64_t)p.T * p.n;
+        const uint32_t blocks = (uint32_t)std::min<uint64_t>(2048, (total / 4 + 255) / 256);
+        hipLaunchKernelGGL(pf_sum_splits_kernel, dim3(blocks), dim3(256), 0, stream, (const float*)p.part, p.splits,
+                           total, p.y);
+    }
+    return hipGetLastError();
+}
+
 // Tile height (32 or 64 tokens), then the K split.
 PfGemm2Shape pf_gemm2_shape(uint32_t T, uint32_t k, uint32_t ntot, int cus) {
     PfGemm2Shape sh{};
@@ -774,21 +822,23 @@ PfGemm2Shape pf_gemm2_shape(uint32_t T, uint32_t k, uint32_t ntot, int cus) {
     return sh;
 }
 
-hipError_t launch_pf_gemm2(uint32_t bm, const PfGemm2Params& p, hipStream_t stream, bool reduce) {
+hipError_t launch_pf_gemm2(uint32_t bm, const PfGemm2Params& p, hipStream_t stream, bool reduce, bool raw) {
     if (p.T == 0 || p.k % 32 != 0 || p.nseg < 1 || p.nseg > 3 || p.ntot % 128 != 0 || p.splits == 0 ||
         p.kper % 32 != 0 || (uint64_t)p.splits * p.kper < p.k || (p.splits > 1 && !p.part))
         return hipErrorInvalidValue;
     uint32_t nb = 0;
     for (int i = 0; i < p.nseg; ++i) {
-        if (p.seg[i].nb0 != nb || p.seg[i].n % 128 != 0 || !p.seg[i].wq || !p.seg[i].sc || !p.seg[i].wf) return hipErrorInvalidValue;
+        if (p.seg[i].nb0 != nb || p.seg[i].n % 128 != 0 || !p.seg[i].wq || !p.seg[i].sc || (!raw && !p.seg[i].wf)) return hipErrorInvalidValue;
         nb += p.seg[i].n / 128;
     }
     if (nb * 128u != p.ntot) return hipErrorInvalidValue;
     if (p.swiglu && (p.nseg != 2 || p.seg[0].n != p.seg[1].n || p.splits != 1 || !p.seg[0].y || p.seg[0].accumulate))
         return hipErrorInvalidValue;
     const dim3 grid(nb, (p.T + bm - 1) / bm, p.splits);
-    if (bm == 64) hipLaunchKernelGGL((pf_gemm2_kernel<64>), grid, dim3(256), 0, stream, p);
-    else if (bm == 32) hipLaunchKernelGGL((pf_gemm2_kernel<32>), grid, dim3(256), 0, stream, p);
+    if (bm == 64 && raw) hipLaunchKernelGGL((pf_gemm2_kernel<64, true>), grid, dim3(256), 0, stream, p);
+    else if (bm == 64) hipLaunchKernelGGL((pf_gemm2_kernel<64, false>), grid, dim3(256), 0, stream, p);
+    else if (bm == 32 && raw) hipLaunchKernelGGL((pf_gemm2_kernel<32, true>), grid, dim3(256), 0, stream, p);
+    else if (bm == 32) hipLaunchKernelGGL((pf_gemm2_kernel<32, false>), grid, dim3(256), 0, stream, p);
     else return hipErrorInvalidValue;
     if (p.splits > 1 && reduce) {
         const uint64_t total = (uint64_t)p.T * p.ntot;

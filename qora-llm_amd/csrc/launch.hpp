@@ -135,7 +135,20 @@ struct PfGemm2Shape {
 PfGemm2Shape pf_gemm2_shape(uint32_t T, uint32_t k, uint32_t ntot, int cus);
 // p.splits, p.kper from pf_gemm2_shape (bm too); p.part holds splits * T * ntot floats when splits > 1.
 // reduce = false leaves the split partials for the consumer to sum (pf_rmsnorm_split_reg_kernel).
-hipError_t launch_pf_gemm2(uint32_t bm, const PfGemm2Params& p, hipStream_t stream, bool reduce = true);
+// raw: the packed scales are the weight's own (launch_pf_gemm_prep), seg.wf is not read.
+hipError_t launch_pf_gemm2(uint32_t bm, const PfGemm2Params& p, hipStream_t stream, bool reduce = true,
+                           bool raw = false);
+// x [T][k] split into xh, xl, xe and a Q4 weight packed with its own scales, in one launch
+hipError_t launch_pf_gemm_prep(const float* x, uint32_t T, uint16_t* xh, uint16_t* xl, int32_t* xe, const uint8_t* w,
+                               const uint16_t* scales, uint32_t k, uint32_t n, uint2* wq, uint16_t* sc,
+                               hipStream_t stream);
+// GEMM of at most kPfSmallT tokens on the reference layout; p.part holds splits * T * n floats when splits > 1
+constexpr uint32_t kPfSmallT = 64;
+struct PfSmallShape {
+    uint32_t splits, kper;
+};
+PfSmallShape pf_small_shape(uint32_t T, uint32_t k, uint32_t n, int cus);
+hipError_t launch_pf_gemm_small(int fmt, const PfSmallParams& p, hipStream_t stream);
 hipError_t launch_pf_rope_cache(const PrefillAttnParams& p, hipStream_t stream);
 hipError_t launch_pf_attn(const PrefillAttnParams& p, hipStream_t stream);
 

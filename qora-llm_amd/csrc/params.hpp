@@ -205,6 +205,19 @@ struct PfGemm2Params {
     int swiglu;
 };
 
+// GEMM of a few tokens on an unprepared weight (pf_gemm_small_kernel).
+struct PfSmallParams {
+    const float* x;            // [T][k]
+    uint32_t T, k, n;
+    const uint8_t* w;          // reference layout: Q4 packed [k][n/2] or f16 [k][n]
+    const uint16_t* scales;    // Q4 [k][n/32]
+    float* y;                  // [T][n]
+    // split K: grid.y = splits, split z takes rows [z kper, (z + 1) kper) and
+    // writes part[z][T][n], summed in split order by pf_sum_splits_kernel
+    uint32_t splits, kper;
+    float* part;
+};
+
 struct PrefillAttnParams {
     const float* qkv;          // GEMM output rows [T][qd + 2 kvd]
     float* q;                  // rotated q [T][qd]

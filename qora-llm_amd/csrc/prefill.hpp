@@ -422,6 +422,15 @@ __global__ __launch_bounds__(256) void pf_weight_exp_kernel(const uint32_t* part
     wf[g] = (int8_t)(eb - 12);
 }
 
+// The exponent f of the scales of one K slice, from their largest magnitude
+// bits: s 2^-f < 2^12 as above, f kept between -5 and 5 so that 2^-f, 1032 2^-f
+// and (q - 8) 2^-f are binary16 values (s is a multiple of 2^-24, so
+// s (q - 8) 2^5 still splits exactly into two of them).
+__device__ __forceinline__ int pf_scale_exp(uint32_t mx) {
+    const int e = (int)((mx >> 10) & 0x1F);
+    return max((e == 0 ? -14 : e - 14) - 12, -5);
+}
+
 // ---------------------------------------------------------------------------
 // The GEMM. Grid (n / NT column tiles, ceil(T / 64) token tiles).
 // ---------------------------------------------------------------------------
@@ -679,7 +688,317 @@ __global__ __launch_bounds__(256) void pf_pack_q4_kernel(const uint8_t* w, const
     }
 }
 
-template <int BM>
+// One launch before the GEMM of a call on an unprepared Q4 weight: blocks
+// 0 .. T - 1 split a row of x each (pf_split_kernel's values), the others
+// pack the weight with its own scales (pf_pack_q4_kernel's layout, for
+// pf_gemm2_kernel<.., RAW>), one 128-column block and 64 rows each. Both are
+// bound by their memory traffic (512 x 2048 -> 11008: 4.2 + 8.4 MB of x and
+// 28.5 MB of weights); as separate launches behind two that found the
+// groups' largest scales they took half as long as the GEMM.
+__global__ __launch_bounds__(256) void pf_gemm_prep_kernel(const float* x, uint16_t* xh_, uint16_t* xl_, int32_t* xe, uint32_t T,
+                                                           const uint8_t* w, const uint16_t* scales, uint32_t k,
+                                                           uint32_t n, uint2* wq, uint16_t* sc) {
+    __shared__ float red[4];
+    const uint32_t t = threadIdx.x;
+    if (blockIdx.x < T) {
+        const float* xr = x + (uint64_t)blockIdx.x * k;
+        _Float16* xh = reinterpret_cast<_Float16*>(xh_) + (uint64_t)blockIdx.x * k;
+        _Float16* xl = reinterpret_cast<_Float16*>(xl_) + (uint64_t)blockIdx.x * k;
+        const bool vec = pf_al(x, 16);              // k % 32 == 0, the workspace rows are aligned
+        float v[8][4];
+        float amax = 0.f;
+        for (uint32_t j0 = 0; j0 < k; j0 += 8192u) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t j = j0 + 4u * (t + 256u * (uint32_t)i);
+                if (vec) pf_load4<true>(xr, j, k, v[i]);
+                else pf_load4<false>(xr, j, k, v[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) amax = fmaxf(amax, fabsf(v[i][c]));
+        }
+        const int e = pf_row_exponent(pf_block_max<256>(amax, red));
+        for (uint32_t j0 = 0; j0 < k; j0 += 8192u) {
+            if (k > 8192u) {                        // (a shorter row is still in registers)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const uint32_t j = j0 + 4u * (t + 256u * (uint32_t)i);
+                    if (vec) pf_load4<true>(xr, j, k, v[i]);
+                    else pf_load4<false>(xr, j, k, v[i]);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) pf_split4<true>(v[i], e, xh, xl, j0 + 4u * (t + 256u * (uint32_t)i), k);
+        }
+        if (t == 0) xe[blockIdx.x] = e;
+        return;
+    }
+    const uint32_t KS = k / 32u, kb2 = (KS + 1u) / 2u;
+    const uint32_t b = blockIdx.x - T, nb = b / kb2, ks0 = (b % kb2) * 2u;
+    const uint32_t bc = t % 64u, rg = t / 64u;
+    const uint32_t c0 = nb * 128u + (bc / 16u) * 32u + bc % 16u, c1 = c0 + 16u;
+    const uint32_t sh = (c0 & 1u) * 4u;             // column c is the low nibble of byte c / 2 when c is even
+#pragma unroll
+    for (uint32_t u = 0; u < 2; ++u) {
+        const uint32_t ks = min(ks0 + u, KS - 1u);  // (an odd last step is packed twice, with the same values)
+        uint32_t b0[8], b1[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const uint64_t row = (uint64_t)(ks * 32u + rg * 8u + (uint32_t)r) * (n / 2u);
+            b0[r] = w[row + c0 / 2u];
+            b1[r] = w[row + c1 / 2u];
+        }
+        uint32_t w0 = 0, w1 = 0;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const int slot = (r >> 1) + 4 * (r & 1);
+            w0 |= ((b0[r] >> sh) & 0xFu) << (4 * slot);
+            w1 |= ((b1[r] >> sh) & 0xFu) << (4 * slot);
+        }
+        wq[((uint64_t)nb * KS + ks) * 256u + t] = make_uint2(w0, w1);
+        if (t < 128u) {
+            const uint32_t g = t / 32u, r = t % 32u;
+            sc[(((uint64_t)nb * KS + ks) * 4u + g) * 32u + r] = scales[(uint64_t)(ks * 32u + r) * (n / 32u) + nb * 4u + g];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// GEMM of a few tokens (T <= 16 TM) on the reference layout, x in fp32: one
+// launch and, when K is split, a sum over the slices. The numerics are those of
+// pf_gemm2_kernel (x and w in two binary16 parts, three products, fp32 sums),
+// with the row and group exponents taken per K slice.
+// Block: 4 waves over every token x 128 columns x one K slice of at most KP
+// rows. The block splits its x slice into LDS itself (rows padded by 16 bytes:
+// conflict-free fragment reads) and never synchronises again: each wave runs
+// over its 32 columns with D steps of weights in flight, a lane holding
+//   Q4:  dword li / 4 of rows 8 kq + 2 (li % 4), + 1 (64 B a row per block); the
+//        quad exchanges them (DPP broadcasts), so that byte li of the 8 rows
+//        gives the B fragments of columns 2 li and 2 li + 1;
+//   F16: columns 2 li, 2 li + 1 of rows 8 kq .. + 7.
+// What bounds it: at 24 tokens, 11008 -> 2048, the weight stream's latency (352
+// blocks of 33 KB) and two launches: 13.9 us a call against 30.7 on the packed
+// path, which split x, found the groups' exponents (two launches), packed,
+// multiplied and summed in six.
+// ---------------------------------------------------------------------------
+template <int TM, bool Q4>
+__global__ __launch_bounds__(256) void pf_gemm_small_kernel(PfSmallParams p) {
+    constexpr int BM = 16 * TM;
+    constexpr int KP = TM == 4 ? 256 : 512;
+    constexpr int TPR = 256 / BM;                   // threads per x row
+    constexpr int NF = KP / (4 * TPR);              // float4 per thread
+    constexpr int XS = KP + 8;                      // halves per LDS row
+    constexpr int D = Q4 ? 8 : 4;                   // steps of weights in flight
+    __shared__ __align__(16) _Float16 xs[2][BM * XS];
+    __shared__ __align__(16) _Float16 ss[Q4 ? 4 : 1][Q4 ? KP : 8];
+    __shared__ int xes[BM];
+
+    const int t = threadIdx.x;
+    const int lane = t & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
+    const uint32_t li = (uint32_t)lane % 16u, kq = (uint32_t)lane / 16u;
+    const uint32_t K = p.k, N = p.n, G = N / 32u;
+    const uint32_t grp = blockIdx.x * 4u + (uint32_t)wave;
+    const uint32_t gc = min(grp, G - 1u);           // (a wave past the last group works on it and stores nothing)
+    const uint32_t kb = blockIdx.y * p.kper;
+    const uint32_t ke = min(K, kb + p.kper);
+    const uint32_t steps = (ke - kb) / 32u;
+
+    struct WStep {
+        uint32_t w[Q4 ? 2 : 8];
+    };
+    auto load_w = [&](uint32_t s) {
+        WStep q;
+        const uint32_t r0 = kb + min(s, steps - 1u) * 32u + 8u * kq;
+        if constexpr (Q4) {
+            const uint8_t* b = p.w + (uint64_t)(r0 + 2u * (li % 4u)) * (N / 2u) + gc * 16u + (li / 4u) * 4u;
+            q.w[0] = *reinterpret_cast<const uint32_t*>(b);
+            q.w[1] = *reinterpret_cast<const uint32_t*>(b + N / 2u);
+        } else {
+            const uint8_t* b = p.w + ((uint64_t)r0 * N + gc * 32u + 2u * li) * 2u;
+#pragma unroll
+            for (int r = 0; r < 8; ++r) q.w[r] = *reinterpret_cast<const uint32_t*>(b + (uint64_t)r * N * 2u);
+        }
+        return q;
+    };
+    WStep wr[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) wr[d] = load_w((uint32_t)d);
+
+    // the slice's scales of the wave's group, and x (rows past T read row T - 1)
+    uint32_t sv[Q4 ? KP / 64 : 1];
+    if constexpr (Q4) {
+#pragma unroll
+        for (int i = 0; i < KP / 64; ++i) {
+            const uint32_t r = kb + (uint32_t)lane + 64u * (uint32_t)i;
+            sv[i] = p.scales[(uint64_t)min(r, ke - 1u) * G + gc];
+            if (r >= ke) sv[i] = 0;
+        }
+    }
+    const uint32_t xr = (uint32_t)t / TPR, xq = (uint32_t)t % TPR;
+    const float* xp = p.x + (uint64_t)min(xr, p.T - 1u) * K + kb;
+    const uint32_t kn = ke - kb;
+    float xv[NF][4];
+    const bool vec = pf_al(p.x, 16);                // K and kb are multiples of 32
+#pragma unroll
+    for (int i = 0; i < NF; ++i) {
+        const uint32_t j = 4u * (xq + (uint32_t)TPR * (uint32_t)i);
+        if (vec) pf_load4<true>(xp, j, kn, xv[i]);
+        else pf_load4<false>(xp, j, kn, xv[i]);
+    }
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < NF; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) amax = fmaxf(amax, fabsf(xv[i][c]));
+#pragma unroll
+    for (int o = 1; o < TPR; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, kWave));
+    const int xe = pf_row_exponent(amax);
+    if (xq == 0) xes[xr] = xe;
+#pragma unroll
+    for (int i = 0; i < NF; ++i)
+        pf_split4<true>(xv[i], xe, &xs[0][xr * XS], &xs[1][xr * XS], 4u * (xq + (uint32_t)TPR * (uint32_t)i), kn);
+    int fw = 0;
+    if constexpr (Q4) {
+        uint32_t mx = 0;
+#pragma unroll
+        for (int i = 0; i < KP / 64; ++i) mx = max(mx, sv[i] & 0x7FFFu);
+        fw = pf_scale_exp(wave_max_u32(mx));
+        const float f = ldexpf(1.0f, -fw);
+#pragma unroll
+        for (int i = 0; i < KP / 64; ++i) ss[wave][lane + 64 * i] = (_Float16)(h2f((uint16_t)sv[i]) * f);
+    }
+    __syncthreads();
+
+    f32x4v acc[TM][2];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    const uint32_t bsel = (li % 4u) | 0x0C000C00u | ((4u + li % 4u) << 16);
+    auto compute = [&](const WStep& q, uint32_t s) {
+        half8v bh[2], bl[2];
+        if constexpr (Q4) {
+            const half8v s8 = *reinterpret_cast<const half8v*>(&ss[wave][s * 32u + 8u * kq]);
+            const v4u32 s4 = __builtin_bit_cast(v4u32, s8);
+            const half2v b_lo = {(_Float16)1032.0f, (_Float16)1032.0f}, b_hi = {(_Float16)72.0f, (_Float16)72.0f};
+            v4u32 h0, h1, l0, l1;
+            auto pair = [&](int j, uint32_t e0, uint32_t e1) {
+                const uint32_t by = __builtin_amdgcn_perm(e1, e0, bsel);    // byte li of rows 2 j and 2 j + 1
+                const half2v q0 = __builtin_bit_cast(half2v, (by & 0x000F000Fu) | 0x64006400u) - b_lo;
+                const half2v q1 = __builtin_bit_cast(half2v, (by & 0x00F000F0u) | 0x54005400u) - b_hi;
+                const uint32_t sj = s4[j];
+                const half2v sc = __builtin_bit_cast(half2v, sj);
+                const half2v a0 = q0 * sc, a1 = q1 * sc;
+                h0[j] = __builtin_bit_cast(uint32_t, a0);
+                h1[j] = __builtin_bit_cast(uint32_t, a1);
+                l0[j] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(q0, sc, -a0));
+                l1[j] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(q1, sc, -a1));
+            };
+            // lane j of each quad holds rows 8 kq + 2 j, + 1
+            pair(0, dpp_u32<0x00>(q.w[0]), dpp_u32<0x00>(q.w[1]));
+            pair(1, dpp_u32<0x55>(q.w[0]), dpp_u32<0x55>(q.w[1]));
+            pair(2, dpp_u32<0xAA>(q.w[0]), dpp_u32<0xAA>(q.w[1]));
+            pair(3, dpp_u32<0xFF>(q.w[0]), dpp_u32<0xFF>(q.w[1]));
+            bh[0] = __builtin_bit_cast(half8v, h0);
+            bh[1] = __builtin_bit_cast(half8v, h1);
+            bl[0] = __builtin_bit_cast(half8v, l0);
+            bl[1] = __builtin_bit_cast(half8v, l1);
+        } else {
+            v4u32 h0, h1;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                h0[j] = __builtin_amdgcn_perm(q.w[2 * j + 1], q.w[2 * j], 0x05040100u);
+                h1[j] = __builtin_amdgcn_perm(q.w[2 * j + 1], q.w[2 * j], 0x07060302u);
+            }
+            bh[0] = __builtin_bit_cast(half8v, h0);
+            bh[1] = __builtin_bit_cast(half8v, h1);
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const uint32_t o = ((uint32_t)i * 16u + li) * XS + s * 32u + 8u * kq;
+            const half8v ah = *reinterpret_cast<const half8v*>(&xs[0][o]);
+            const half8v al = *reinterpret_cast<const half8v*>(&xs[1][o]);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh[j], acc[i][j], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh[j], acc[i][j], 0, 0, 0);
+                if constexpr (Q4) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl[j], acc[i][j], 0, 0, 0);
+            }
+        }
+    };
+    // D steps a round, the next round's loads going out as a slot is used
+    // (past the slice the last step is loaded again and not used)
+    for (uint32_t s0 = 0; s0 < steps; s0 += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const uint32_t s = s0 + (uint32_t)d;
+            if (s < steps) compute(wr[d], s);
+            if (s0 + D < steps) wr[d] = load_w(s + D);
+        }
+    }
+
+    if (grp >= G) return;
+    const uint32_t c = grp * 32u + 2u * li;
+    float* y = p.splits > 1 ? p.part + (uint64_t)blockIdx.y * p.T * N : p.y;
+    const bool al8 = pf_al(y, 8);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t row = (uint32_t)i * 16u + kq * 4u + (uint32_t)r;
+            if (row >= p.T) continue;
+            const int e = xes[row] + fw;
+            const float v0 = ldexpf(acc[i][0][r], e), v1 = ldexpf(acc[i][1][r], e);
+            float* d = y + (uint64_t)row * N + c;
+            if (al8) {
+                *reinterpret_cast<float2*>(d) = make_float2(v0, v1);
+            } else {
+                d[0] = v0;
+                d[1] = v1;
+            }
+        }
+}
+
+// part[z][total] summed over z in order into y (total a multiple of 4, part
+// 16-byte aligned): four elements a thread, four slices in flight.
+__global__ __launch_bounds__(256) void pf_sum_splits_kernel(const float* part, uint32_t splits, uint64_t total, float* y) {
+    const bool vec = pf_al(y, 16);
+    for (uint64_t e = 4u * ((uint64_t)blockIdx.x * 256u + threadIdx.x); e < total; e += 1024ull * gridDim.x) {
+        float4 a = *reinterpret_cast<const float4*>(part + e);
+        for (uint32_t z = 1; z < splits; z += 4) {
+            float4 q[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) q[u] = *reinterpret_cast<const float4*>(part + (uint64_t)min(z + u, splits - 1u) * total + e);
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u)
+                if (z + u < splits) {
+                    a.x += q[u].x;
+                    a.y += q[u].y;
+                    a.z += q[u].z;
+                    a.w += q[u].w;
+                }
+        }
+        if (vec) {
+            *reinterpret_cast<float4*>(y + e) = a;
+        } else {
+            y[e] = a.x;
+            y[e + 1] = a.y;
+            y[e + 2] = a.z;
+            y[e + 3] = a.w;
+        }
+    }
+}
+
+// RAW: sc holds the weight's own scales and sg.wf is not read; each wave takes
+// the exponent f of its column group over its K slice from a first look at the
+// slice's scales (pf_scale_exp) and forms (q - 8) 2^-f with the multiply-add
+// that takes the bias off (scaling the scales instead cost four instructions a
+// step: 63.4 against 62.5 us a call). A call on an unprepared weight then packs
+// it without a pass over the scales of the whole matrix first.
+template <int BM, bool RAW>
 __global__ __launch_bounds__(256, 2) void pf_gemm2_kernel(PfGemm2Params p) {
     constexpr int BN = 128, KC = 32;
     // LDS rows of 64 B (32 halves, no padding); the 16-byte chunk c of row r
@@ -759,6 +1078,22 @@ __global__ __launch_bounds__(256, 2) void pf_gemm2_kernel(PfGemm2Params p) {
         *reinterpret_cast<v4u32*>(&xs[buf][0][xc0]) = q.xh0;
         *reinterpret_cast<v4u32*>(&xs[buf][1][xc0]) = q.xl0;
     };
+    int fw = 0;                                     // RAW: the wave's weight exponent
+    half2v qf = {(_Float16)1.0f, (_Float16)1.0f}, qb = qf;   // RAW: 2^-f and -1032 2^-f
+    if constexpr (RAW) {
+        // 64 bytes of scales (32 rows) per step: four lanes a step
+        const uint16_t* sl = sg.sc + ((uint64_t)lnb * KS * 4u + grp) * 32u + (uint64_t)(kb / 32u) * 128u;
+        uint32_t mx = 0;
+        for (uint32_t s = (uint32_t)lane / 4u; s < steps; s += 16u) {
+            const v4u32 v = *reinterpret_cast<const v4u32*>(sl + (uint64_t)s * 128u + 8u * ((uint32_t)lane % 4u));
+#pragma unroll
+            for (int c = 0; c < 4; ++c) mx = max(mx, max(v[c] & 0x7FFFu, (v[c] >> 16) & 0x7FFFu));
+        }
+        fw = pf_scale_exp(wave_max_u32(mx));
+        const _Float16 f = (_Float16)ldexpf(1.0f, -fw), b = (_Float16)ldexpf(-1032.0f, -fw);
+        qf = half2v{f, f};
+        qb = half2v{b, b};
+    }
     // wh, wl of the lane's two columns, two rows per binary16 pair: the B
     // fragments (k = 8 kq + b, column li) of tiles 0 and 1
     auto dequant = [&](const Slice& q, half8v* bh, half8v* bl) {
@@ -769,7 +1104,8 @@ __global__ __launch_bounds__(256, 2) void pf_gemm2_kernel(PfGemm2Params p) {
             v4u32 wh, wl;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const half2v qv = __builtin_bit_cast(half2v, ((wv >> (4 * j)) & 0x000F000Fu) | 0x64006400u) - bias;
+                const half2v q1 = __builtin_bit_cast(half2v, ((wv >> (4 * j)) & 0x000F000Fu) | 0x64006400u);
+                const half2v qv = RAW ? __builtin_elementwise_fma(q1, qf, qb) : q1 - bias;
                 const uint32_t sj = q.sc[j];        // (a bit_cast of a vector element would read element 0)
                 const half2v sv = __builtin_bit_cast(half2v, sj);
                 const half2v h = qv * sv;
@@ -865,7 +1201,7 @@ __global__ __launch_bounds__(256, 2) void pf_gemm2_kernel(PfGemm2Params p) {
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
                     const uint32_t c = lnb * (uint32_t)BN + grp * 32u + (uint32_t)j * 16u + li;
-                    const int fg = (int)sg.wf[c / 32u];
+                    const int fg = RAW ? fw : (int)sg.wf[c / 32u];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const uint32_t rl = (uint32_t)i * 16u + kq * 4u + (uint32_t)r;
@@ -881,7 +1217,7 @@ __global__ __launch_bounds__(256, 2) void pf_gemm2_kernel(PfGemm2Params p) {
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 const uint32_t c = lnb * (uint32_t)BN + grp * 32u + (uint32_t)j * 16u + li;
-                const int fg = (int)sg.wf[c / 32u];
+                const int fg = RAW ? fw : (int)sg.wf[c / 32u];
                 const uint32_t hc = 64u * nb + ((uint32_t)wave - 2u) * 32u + (uint32_t)j * 16u + li;   // h column
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
@@ -903,7 +1239,7 @@ __global__ __launch_bounds__(256, 2) void pf_gemm2_kernel(PfGemm2Params p) {
         for (int j = 0; j < TN; ++j) {
             const uint32_t cl = (uint32_t)wave * 32u + (uint32_t)j * 16u + li;  // column in the block
             const uint32_t c = lnb * (uint32_t)BN + cl;                        // column in the segment
-            const int fg = (int)sg.wf[c / 32u];
+            const int fg = RAW ? fw : (int)sg.wf[c / 32u];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const uint32_t row = m0 + (uint32_t)i * 16u + kq * 4u + (uint32_t)r;

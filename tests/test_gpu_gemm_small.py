@@ -1,0 +1,85 @@
+"""qora_hip_gemm at the edges of its routes: the few-token kernel (16, 32 and 64
+token tiles, K slices of 128 to 512 rows, column blocks partly past the last
+group, x and y off the 16- and 8-byte boundaries) and the packed path just above
+it, against float64. The bound is the other GEMM tests': fp32 sums of products
+exact to 22 bits."""
+import numpy as np
+import pytest
+
+from helpers import device, elem_err, dequant_np, rel_err, rng
+
+pytestmark = pytest.mark.gpu
+
+TRUTH_TOL = 1e-5
+
+
+def _weight(pkg, fmt, k, n, seed, spread):
+    if fmt == "f16":
+        w = pkg.synth_f16(seed, 1, k * n, 0.02)
+        return pkg.Weight(k=k, n=n, data=w), w.view(np.float16).astype(np.float64).reshape(k, n)
+    packed, scales = pkg.synth_q4(seed, 2, k, n)
+    if spread:      # scales over a range of exponents, both signs
+        r = rng(seed)
+        scales = (r.choice([-1.0, 1.0], scales.size) * 2.0 ** r.integers(*spread, scales.size)).astype(np.float16)
+        scales = scales.view(np.uint16)
+    return pkg.Weight(k=k, n=n, packed=packed, scales=scales), dequant_np(packed, scales, k, n)
+
+
+@pytest.mark.parametrize("fmt", ["q4", "f16"])
+@pytest.mark.parametrize("T,k,n", [(1, 32, 32), (15, 544, 96), (16, 2048, 512), (17, 1056, 160), (32, 11008, 256),
+                                   (33, 4096, 2080), (64, 2048, 2048), (65, 2080, 256), (66, 8224, 384)])
+def test_gemm_few_tokens_vs_truth(ctx, pkg, fmt, T, k, n):
+    print(f"case gemm {fmt} T={T} k={k} n={n}", flush=True)
+    wt, W = _weight(pkg, fmt, k, n, T + k, None)
+    wid = ctx.upload(wt)
+    x = (rng(T).standard_normal((T, k)) * 2.0 ** rng(k).integers(-6, 6, (T, 1))).astype(np.float32)
+    truth = x.astype(np.float64) @ W
+    mag = np.abs(x.astype(np.float64)) @ np.abs(W)
+    with device(ctx) as d:
+        for off in (0, 4):          # bytes past an aligned address, of x and of y
+            xd, yd = d.empty(x.nbytes + 16), d.empty(T * n * 4 + 16)
+            ctx.h2d(xd + off, x)
+            ctx.check(ctx.lib.qora_hip_gemm(ctx.h, wid, xd + off, yd + off, T, None))
+            y = d.get(yd + off, (T, n), np.float32)
+            assert rel_err(y, truth) <= TRUTH_TOL
+            assert elem_err(y, truth, mag) <= TRUTH_TOL
+    ctx.lib.qora_hip_release_weight(ctx.h, wid)
+
+
+@pytest.mark.parametrize("spread", [(-24, 15), (-24, -18)])
+@pytest.mark.parametrize("T", [5, 64, 65])
+def test_gemm_scale_extremes(ctx, pkg, T, spread):
+    """Scales from subnormal to 2^14 in one matrix, and subnormal ones only:
+    the slice exponents keep every weight's two parts finite and exact."""
+    k, n = 1024, 256
+    wt, W = _weight(pkg, "q4", k, n, 77, spread)
+    wid = ctx.upload(wt)
+    x = rng(T).standard_normal((T, k)).astype(np.float32)
+    with device(ctx) as d:
+        y = d.empty(T * n * 4)
+        ctx.check(ctx.lib.qora_hip_gemm(ctx.h, wid, d.put(x), y, T, None))
+        got = d.get(y, (T, n), np.float32)
+    assert elem_err(got, x.astype(np.float64) @ W, np.abs(x.astype(np.float64)) @ np.abs(W)) <= TRUTH_TOL
+    ctx.lib.qora_hip_release_weight(ctx.h, wid)
+
+
+def test_gemm_non_finite_row_stays_in_its_row(ctx, pkg):
+    """A row of x with an infinity or NaN gives non-finite outputs in that row
+    and leaves the others as they are."""
+    k, n, T = 544, 160, 20
+    wt, _ = _weight(pkg, "q4", k, n, 5, None)
+    wid = ctx.upload(wt)
+    x = rng(3).standard_normal((T, k)).astype(np.float32)
+    with device(ctx) as d:
+        y = d.empty(T * n * 4)
+        ctx.check(ctx.lib.qora_hip_gemm(ctx.h, wid, d.put(x), y, T, None))
+        want = d.get(y, (T, n), np.float32)
+        for bad in (np.inf, np.nan):
+            xb = x.copy()
+            xb[7, 100] = bad
+            ctx.check(ctx.lib.qora_hip_gemm(ctx.h, wid, d.put(xb), y, T, None))
+            got = d.get(y, (T, n), np.float32)
+            rows = np.arange(T) != 7
+            assert np.array_equal(got[rows], want[rows])
+            assert not np.isfinite(got[7]).all()
+    ctx.lib.qora_hip_release_weight(ctx.h, wid)
