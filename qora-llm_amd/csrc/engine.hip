@@ -11,7 +11,6 @@
 #include <cstring>
 #include <cstdio>
 #include <string>
-#include <unordered_map>
 #include <initializer_list>
 #include <vector>
 
@@ -197,12 +196,16 @@ struct qora_hip_ctx {
     long long* ws_sum = nullptr;
     uint32_t* ws_count = nullptr;
     uint64_t ws_tiles = 0;
+    std::vector<SamplePenalty> pen;      // sampling: the call's penalty list and its look-up table
+    std::vector<uint32_t> pen_at;
     std::vector<void*> ws_old;           // outgrown ones: a captured graph may still use them
-    // on-device sampling scratch (grown to the largest vocab seen)
-    float* smp_work = nullptr;
-    unsigned long long* smp_cand = nullptr;
+    // on-device sampling scratch (grown to the largest vocab seen), one
+    // allocation that smp_rng starts
     unsigned long long* smp_rng = nullptr;
     int32_t* smp_tok = nullptr;
+    uint32_t* smp_count = nullptr;       // blocks arrived (smp_topk_draw_kernel)
+    unsigned long long* smp_cand = nullptr;
+    float* smp_work = nullptr;
     SamplePenalty* smp_pen = nullptr;
     SamplePenalty* h_pen = nullptr;      // pinned staging of the penalty list
     uint64_t h_pen_n = 0;
@@ -555,8 +558,7 @@ extern "C" int qora_hip_destroy(qora_hip_ctx* c) {
         if (w.w) (void)hipFree(w.w);
         if (w.scales) (void)hipFree(w.scales);
     }
-    for (void* p : {(void*)c->ws_count, (void*)c->ws_attn_part, c->ws_pf, (void*)c->smp_work, (void*)c->smp_cand,
-                    (void*)c->smp_rng, (void*)c->smp_pen, c->smp_sort})
+    for (void* p : {(void*)c->ws_count, (void*)c->ws_attn_part, c->ws_pf, (void*)c->smp_rng, (void*)c->smp_pen, c->smp_sort})
         if (p) (void)hipFree(p);
     for (void* p : c->ws_old) (void)hipFree(p);
     if (c->h_pin) (void)hipHostFree(c->h_pin);
@@ -2222,45 +2224,55 @@ int sample_device(qora_hip_ctx* c, const float* logits, uint64_t vocab, const ui
     const bool rep = !greedy && sp->repetition_penalty > 1.0f;
     const bool pres = !greedy && sp->presence_penalty > 0.0f;
     // distinct history tokens with their penalties (apply_repetition_penalty walks the last 64
-    // tokens, apply_presence_penalty every token; ids >= vocab are skipped, generate.rs:68, 85)
-    std::vector<SamplePenalty> pen;
-    {
-        std::unordered_map<uint32_t, size_t> at;
-        auto entry = [&](uint32_t t) -> SamplePenalty& {
-            auto it = at.find(t);
-            if (it != at.end()) return pen[it->second];
-            at.emplace(t, pen.size());
-            pen.push_back(SamplePenalty{t, 0, 0, 0});
-            return pen.back();
-        };
-        if (rep)
-            for (uint64_t i = n_history - std::min<uint64_t>(64, n_history); i < n_history; ++i)
-                if (history[i] < vocab) entry(history[i]).rep_count += 1;
-        if (pres)
-            for (uint64_t i = 0; i < n_history; ++i)
-                if (history[i] < vocab) entry(history[i]).seen = 1;
+    // tokens, apply_presence_penalty every token; ids >= vocab are skipped, generate.rs:68, 85),
+    // found through an open-addressing table of pen indexes + 1 kept in the context
+    std::vector<SamplePenalty>& pen = c->pen;
+    pen.clear();
+    if (rep || pres) {
+        const uint64_t first = pres ? 0 : n_history - std::min<uint64_t>(64, n_history);
+        size_t cap = 64;
+        while (cap < 2 * (n_history - first)) cap *= 2;
+        std::vector<uint32_t>& at = c->pen_at;
+        at.assign(cap, 0);
+        for (uint64_t i = first; i < n_history; ++i) {
+            const uint32_t t = history[i];
+            if (t >= vocab) continue;
+            size_t h = (t * 2654435761u) & (cap - 1);
+            while (at[h] && pen[at[h] - 1].token != t) h = (h + 1) & (cap - 1);
+            if (!at[h]) {
+                pen.push_back(SamplePenalty{t, 0, 0, 0});
+                at[h] = (uint32_t)pen.size();
+            }
+            SamplePenalty& e = pen[at[h] - 1];
+            if (rep && i + 64 >= n_history) e.rep_count += 1;
+            if (pres) e.seen = 1;
+        }
     }
     const uint32_t V = (uint32_t)vocab, blocks = smp_blocks(V);
     if (V > c->smp_vocab || !c->smp_rng) {
         HIP_TRY(c, hipStreamSynchronize(c->stream));
-        for (void* q : {(void*)c->smp_work, (void*)c->smp_cand, (void*)c->smp_rng})   // smp_tok lies in smp_rng
-            if (q) (void)hipFree(q);
-        c->smp_work = nullptr;
-        c->smp_cand = nullptr;
+        if (c->smp_rng) (void)hipFree(c->smp_rng);
         c->smp_rng = nullptr;
-        c->smp_tok = nullptr;
         c->smp_vocab = 0;
+        // one allocation: state, token and count; candidates; the penalised copy
+        const size_t cb = (size_t)blocks * 64 * 8;
         void* q = nullptr;
-        if (int rc = dalloc(c, (size_t)V * 4, &q)) return rc;
-        c->smp_work = (float*)q;
-        if (int rc = dalloc(c, (size_t)blocks * 64 * 8, &q)) return rc;
-        c->smp_cand = (unsigned long long*)q;
-        if (int rc = dalloc(c, 256, &q)) return rc;
+        if (int rc = dalloc(c, 256 + cb + (size_t)V * 4, &q)) return rc;
+        const hipError_t e = hipMemsetAsync(q, 0, 256, c->stream);
+        if (e != hipSuccess) {
+            (void)hipFree(q);
+            return fail(c, QORA_HIP_E_DEVICE, std::string("sampling scratch: ") + hipGetErrorString(e));
+        }
         c->smp_rng = (unsigned long long*)q;
         c->smp_tok = (int32_t*)((uint8_t*)q + 64);
+        c->smp_count = (uint32_t*)((uint8_t*)q + 128);
+        c->smp_cand = (unsigned long long*)((uint8_t*)q + 256);
+        c->smp_work = (float*)((uint8_t*)q + 256 + cb);
         c->smp_vocab = V;
     }
-    if (pen.size() > c->smp_pen_n) {
+    const bool few = sp->top_k >= 1 && sp->top_k <= 64 && smp_supported(V);
+    const bool args = few && pen.size() <= kSmpPenaltyArgs;   // the list goes with the launch
+    if (!args && pen.size() > c->smp_pen_n) {
         HIP_TRY(c, hipStreamSynchronize(c->stream));
         if (c->smp_pen) (void)hipFree(c->smp_pen);
         c->smp_pen = nullptr;
@@ -2271,7 +2283,7 @@ int sample_device(qora_hip_ctx* c, const float* logits, uint64_t vocab, const ui
         c->smp_pen = (SamplePenalty*)q;
         c->smp_pen_n = n;
     }
-    if (pen.size() > c->h_pen_n) {
+    if (!args && pen.size() > c->h_pen_n) {
         HIP_TRY(c, hipStreamSynchronize(s));
         if (c->h_pen) (void)hipHostFree(c->h_pen);
         c->h_pen = nullptr;
@@ -2283,7 +2295,7 @@ int sample_device(qora_hip_ctx* c, const float* logits, uint64_t vocab, const ui
         }
         c->h_pen_n = n;
     }
-    if (!pen.empty()) {
+    if (!args && !pen.empty()) {
         // through pinned memory: the copy may run after this call returns
         std::memcpy(c->h_pen, pen.data(), pen.size() * sizeof(SamplePenalty));
         HIP_TRY(c, hipMemcpyAsync(c->smp_pen, c->h_pen, pen.size() * sizeof(SamplePenalty), hipMemcpyHostToDevice, s));
@@ -2299,7 +2311,7 @@ int sample_device(qora_hip_ctx* c, const float* logits, uint64_t vocab, const ui
     p.dev_token = dev_token;
     p.work = c->smp_work;
     p.vocab = V;
-    p.pen = c->smp_pen;
+    p.pen = args ? nullptr : c->smp_pen;
     p.n_pen = (uint32_t)pen.size();
     p.repetition = sp->repetition_penalty;
     p.presence = sp->presence_penalty;
@@ -2310,9 +2322,12 @@ int sample_device(qora_hip_ctx* c, const float* logits, uint64_t vocab, const ui
     p.top_k = sp->top_k;
     p.rng = c->smp_rng;
     p.token_out = c->smp_tok;
-    const bool few = sp->top_k >= 1 && sp->top_k <= 64 && smp_supported(V);
     if (few) {
-        HIP_TRY(c, launch_sample(logits, p, s));
+        SmpPenaltyArgs l;
+        if (args)
+            for (size_t i = 0; i < pen.size(); ++i) l.e[i] = pen[i].token | (pen[i].rep_count << 17) | (pen[i].seen << 24);
+        p.count = c->smp_count;
+        HIP_TRY(c, launch_sample(logits, p, l, in_order(c, s), s));
     } else {
         const uint32_t k = sp->top_k > 0 ? std::min<uint32_t>(sp->top_k, V) : V;
         const uint32_t ns = smp_sort_keys(V);

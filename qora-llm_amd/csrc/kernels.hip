@@ -923,14 +923,20 @@ hipError_t launch_pf_attn(const PrefillAttnParams& p, hipStream_t stream) {
 uint32_t smp_blocks(uint32_t vocab) { return (vocab + kSmpBlock - 1) / kSmpBlock; }
 bool smp_supported(uint32_t vocab) { return vocab > 0 && smp_blocks(vocab) * kSmpKeep <= kSmpFinal; }
 
-hipError_t launch_sample(const float* logits, const SampleParams& p, hipStream_t stream) {
-    if (!smp_supported(p.vocab) || p.blocks != smp_blocks(p.vocab) || p.top_k == 0 || p.top_k > kSmpKeep)
+hipError_t launch_sample(const float* logits, const SampleParams& p, const SmpPenaltyArgs& pen, bool one,
+                         hipStream_t stream) {
+    if (!smp_supported(p.vocab) || p.blocks != smp_blocks(p.vocab) || p.top_k == 0 || p.top_k > kSmpKeep ||
+        (!p.pen && p.n_pen > kSmpPenaltyArgs) || (one && !p.count))
         return hipErrorInvalidValue;
     // the block kernel reads the logits and applies the penalties itself
     SampleParams q = p;
     q.logits = logits;
-    hipLaunchKernelGGL(smp_block_topk_kernel, dim3(p.blocks), dim3(kSmpTopkThreads), 0, stream, q);
-    hipLaunchKernelGGL(smp_final_kernel, dim3(1), dim3(kSmpFinalThreads), 0, stream, q);
+    if (one) {
+        hipLaunchKernelGGL(smp_topk_draw_kernel, dim3(p.blocks), dim3(kSmpThreads), 0, stream, q, pen);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(smp_block_topk_kernel, dim3(p.blocks), dim3(kSmpThreads), 0, stream, q, pen);
+    hipLaunchKernelGGL(smp_final_kernel, dim3(1), dim3(kSmpThreads), 0, stream, q);
     return hipGetLastError();
 }
 

@@ -155,7 +155,9 @@ hipError_t launch_pf_attn(const PrefillAttnParams& p, hipStream_t stream);
 // on-device sampling (sample.hpp): vocab <= 131072, 1 <= top_k <= 64
 uint32_t smp_blocks(uint32_t vocab);
 bool smp_supported(uint32_t vocab);
-hipError_t launch_sample(const float* logits, const SampleParams& p, hipStream_t stream);
+// one: a single launch, whose count word no other launch may share while it runs.
+hipError_t launch_sample(const float* logits, const SampleParams& p, const SmpPenaltyArgs& pen, bool one,
+                         hipStream_t stream);
 // The full-sort path (any top_k, vocabularies up to 4M): n_sort keys per
 // sort buffer, and the kernels over the first k sorted candidates.
 uint32_t smp_sort_keys(uint32_t vocab);

@@ -263,14 +263,22 @@ struct SamplePenalty {
     uint32_t pad_;
 };
 
+// The same entries as kernel arguments (vocabularies up to 131072): token |
+// rep_count << 17 | seen << 24. 3 KiB of the 4 KiB a launch can pass.
+constexpr uint32_t kSmpPenaltyArgs = 768;
+struct SmpPenaltyArgs {
+    uint32_t e[kSmpPenaltyArgs];
+};
+
 struct SampleParams {
     float* work;               // [vocab] penalised copy of the logits
     uint32_t vocab;
-    const SamplePenalty* pen;  // distinct history tokens
+    const SamplePenalty* pen;  // distinct history tokens; null: n_pen entries of the SmpPenaltyArgs
     uint32_t n_pen;
     float repetition, presence;
     unsigned long long* cand;  // [blocks][kSmpKeep] per-block best keys
     uint32_t blocks;
+    uint32_t* count;           // smp_topk_draw_kernel: blocks arrived (0 between launches)
     float temperature, top_p;
     uint32_t top_k;
     unsigned long long rng_in; // xorshift64 state before the draw

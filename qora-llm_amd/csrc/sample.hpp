@@ -15,9 +15,10 @@
 //    NaN ranks last. Each wave sorts runs of 64 keys, one key per lane, with
 //    cross-lane exchanges (a bitonic network in registers), and sorted runs
 //    are merged pairwise keeping the 64 smallest keys (smp_wave_merge_low).
-// 3. smp_final_kernel: one block merges the blocks' sorted candidate runs the
-//    same way down to the best 64; the softmax terms of the top k are computed
-//    one per lane, and one thread runs the reference's sums in the reference's
+// 3. smp_final_kernel (or, when calls run in order, the last block of 2:
+//    smp_topk_draw_kernel) merges the blocks' sorted candidate runs the same
+//    way down to the best 64; the softmax terms of the top k are computed
+//    one per lane, and one wave runs the reference's sums in the reference's
 //    order (softmax normaliser, nucleus cut-off, one xorshift64 draw, linear
 //    scan). Greedy (temperature <= 0) takes the first candidate: the
 //    first-max rule.
@@ -33,8 +34,7 @@ namespace qora {
 constexpr uint32_t kSmpBlock = 2048;    // logits per block in the first pass
 constexpr uint32_t kSmpKeep = 64;       // candidates kept per block (top_k <= kSmpKeep)
 constexpr uint32_t kSmpFinal = 4096;    // candidate keys merged by the final block (64 runs of 64)
-constexpr uint32_t kSmpTopkThreads = 512;    // 8 waves: 4 runs of 64 keys each
-constexpr uint32_t kSmpFinalThreads = 1024;  // 16 waves: two merges each in the first round
+constexpr uint32_t kSmpThreads = 1024;  // 16 waves: two runs of 64 keys each, two merges in the final's first round
 constexpr uint32_t kSmpSortMax = 1u << 22;   // keys of the full-sort path (vocabularies up to 4M)
 
 // Orderable key: ascending key = value descending, then index ascending.
@@ -187,16 +187,71 @@ __global__ __launch_bounds__(256) void smp_penalty_kernel(SampleParams p) {
     p.work[e.token] = smp_penalise(p, e, p.work[e.token]);
 }
 
-__global__ __launch_bounds__(kSmpTopkThreads) void smp_block_topk_kernel(SampleParams p) {
-    constexpr uint32_t NWV = kSmpTopkThreads / kWave;
-    static_assert(kSmpKeep == 64 && kSmpBlock % (NWV * 64) == 0, "64-key runs, NWV waves");
+// Softmax, nucleus cut-off and draw over the sorted candidates keys[0..63];
+// publishes the token and the state. Wave 0 alone: lane i holds candidate i's
+// term (each the expression the reference evaluates for it, generate.rs:360-366)
+// and the reference's sums run in its order over v_readlane, the same in every
+// lane (on one thread over LDS each addition waited for its own read).
+__device__ __forceinline__ void smp_draw(const SampleParams& p, const unsigned long long* keys) {
+    if (threadIdx.x >= kWave) return;
+    const uint32_t lane = threadIdx.x;
+    const uint32_t k = min(p.top_k, min(p.vocab, kSmpKeep));
+    const unsigned long long key = keys[lane];
+    const uint32_t first = (uint32_t)keys[0];
+    uint32_t token = first;
+    unsigned long long state = p.rng_in;
+    if (p.temperature > 0.0f) {
+        const float inv_temp = 1.0f / p.temperature;
+        float prob = lane < k ? expf((smp_key_value(key) - smp_key_value(keys[0])) * inv_temp) : 0.0f;
+        // softmax over the top k (generate.rs:360-370)
+        float sum = 0.0f;
+        for (uint32_t i = 0; i < k; ++i) sum += lane_f32(prob, (int)i);
+        if (sum > 0.0f) {
+            prob *= 1.0f / sum;
+            // nucleus cut-off (generate.rs:372-380)
+            float cum = 0.0f;
+            uint32_t cutoff = k;
+            for (uint32_t i = 0; i < k; ++i) {
+                cum += lane_f32(prob, (int)i);
+                if (cum >= p.top_p) {
+                    cutoff = i + 1;
+                    break;
+                }
+            }
+            float total = 0.0f;
+            for (uint32_t i = 0; i < cutoff; ++i) total += lane_f32(prob, (int)i);
+            if (total > 0.0f) {
+                // one xorshift64 draw (Rng::next_f32, generate.rs:54-60) and the scan (382-393)
+                state ^= state << 13;
+                state ^= state >> 7;
+                state ^= state << 17;
+                const float rand_val = (float)(uint32_t)(state >> 40) / 16777216.0f * total;
+                float acc = 0.0f;
+                for (uint32_t i = 0; i < cutoff; ++i) {
+                    acc += lane_f32(prob, (int)i);
+                    if (acc >= rand_val) {
+                        token = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)key, (int)i);
+                        break;
+                    }
+                }
+            }
+        }
+    }
+    if (lane == 0) smp_publish(p, token, state);
+}
+
+// The best kSmpKeep keys of logits [2048 blockIdx.x, ..), ascending, in
+// runs[result]. Every load of the wave's runs first (the logits themselves),
+// the penalties of the block's tokens applied through LDS, then each run
+// sorted across the lanes and the runs merged.
+template <uint32_t N>
+__device__ __forceinline__ uint32_t smp_block_best(const SampleParams& p, const SmpPenaltyArgs& l,
+                                                   unsigned long long (*runs)[N]) {
+    constexpr uint32_t NWV = kSmpThreads / kWave;
+    static_assert(kSmpKeep == 64 && kSmpBlock % (NWV * 64) == 0 && N >= kSmpBlock, "64-key runs, NWV waves");
     constexpr uint32_t NR = kSmpBlock / 64, RPW = NR / NWV;   // runs, runs per wave
-    __shared__ unsigned long long runs[2][kSmpBlock];
     const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const uint32_t base = blockIdx.x * kSmpBlock;
-    // every load of the wave's runs first (the logits themselves), the
-    // penalties of the block's tokens applied through LDS, then each run
-    // sorted across the lanes
     float x[RPW];
 #pragma unroll
     for (uint32_t q = 0; q < RPW; ++q) x[q] = p.logits[min(base + (wave + NWV * q) * 64 + lane, p.vocab - 1)];
@@ -205,8 +260,16 @@ __global__ __launch_bounds__(kSmpTopkThreads) void smp_block_topk_kernel(SampleP
 #pragma unroll
         for (uint32_t q = 0; q < RPW; ++q) xs[(wave + NWV * q) * 64 + lane] = x[q];
         __syncthreads();
-        for (uint32_t j = threadIdx.x; j < p.n_pen; j += kSmpTopkThreads) {
-            const SamplePenalty e = p.pen[j];
+        for (uint32_t j = threadIdx.x; j < p.n_pen; j += kSmpThreads) {
+            SamplePenalty e;
+            if (p.pen) {
+                e = p.pen[j];
+            } else {
+                const uint32_t v = l.e[j];
+                e.token = v & 0x1FFFFu;
+                e.rep_count = (v >> 17) & 0x7Fu;
+                e.seen = v >> 24;
+            }
             if (e.token >= base && e.token - base < kSmpBlock) xs[e.token - base] = smp_penalise(p, e, xs[e.token - base]);
         }
         __syncthreads();
@@ -222,76 +285,57 @@ __global__ __launch_bounds__(kSmpTopkThreads) void smp_block_topk_kernel(SampleP
     }
 #pragma unroll
     for (uint32_t q = 0; q < RPW; ++q) runs[0][(wave + NWV * q) * 64 + lane] = smp_wave_sort(v[q]);
-    const uint32_t src = smp_merge_runs<kSmpBlock, NWV>(runs, NR, 0);
-    if (wave == 0) p.cand[blockIdx.x * kSmpKeep + lane] = runs[src][lane];
+    return smp_merge_runs<N, NWV>(runs, NR, 0);
 }
 
-__global__ __launch_bounds__(kSmpFinalThreads) void smp_final_kernel(SampleParams p) {
+__global__ __launch_bounds__(kSmpThreads) void smp_block_topk_kernel(SampleParams p, SmpPenaltyArgs l) {
+    __shared__ unsigned long long runs[2][kSmpBlock];
+    const uint32_t src = smp_block_best<kSmpBlock>(p, l, runs);
+    if (threadIdx.x < kSmpKeep) p.cand[blockIdx.x * kSmpKeep + threadIdx.x] = runs[src][threadIdx.x];
+}
+
+__global__ __launch_bounds__(kSmpThreads) void smp_final_kernel(SampleParams p) {
     static_assert(kSmpFinal % 64 == 0 && kSmpKeep == 64, "64-key runs");
     __shared__ unsigned long long runs[2][kSmpFinal];
-    __shared__ float prob[kSmpKeep];
-    __shared__ float s_inv;
     // the blocks' candidate runs (each ascending), then runs of ~0 padding
     const uint32_t nc = p.blocks * kSmpKeep;
-    for (uint32_t j = threadIdx.x; j < kSmpFinal; j += kSmpFinalThreads) runs[0][j] = j < nc ? p.cand[j] : ~0ull;
-    const uint32_t src = smp_merge_runs<kSmpFinal, kSmpFinalThreads / kWave>(runs, kSmpFinal / 64, 0);
-    const unsigned long long* keys = runs[src];
-    const uint32_t k = min(p.top_k, min(p.vocab, kSmpKeep));
-    const float inv_temp = p.temperature > 0.0f ? 1.0f / p.temperature : 0.0f;
-    // the softmax terms of the top k (generate.rs:360-366), one per lane of
-    // wave 0, each the expression the reference evaluates for it
-    if (p.temperature > 0.0f && threadIdx.x < k)
-        prob[threadIdx.x] = expf((smp_key_value(keys[threadIdx.x]) - smp_key_value(keys[0])) * inv_temp);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float sum = 0.0f;
-        if (p.temperature > 0.0f)
-            for (uint32_t i = 0; i < k; ++i) sum += prob[i];
-        s_inv = sum > 0.0f ? 1.0f / sum : 0.0f;
-    }
-    __syncthreads();
-    if (p.temperature > 0.0f && threadIdx.x < k && s_inv > 0.0f) prob[threadIdx.x] *= s_inv;
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    uint32_t token = (uint32_t)keys[0];
-    unsigned long long state = p.rng_in;
-    if (p.temperature > 0.0f) {
-        // softmax over the top k (generate.rs:360-370): the terms and their
-        // normalised values are in prob[]; the sum above ran in index order
-        if (s_inv > 0.0f) {
-            // nucleus cut-off (generate.rs:372-380)
-            float cum = 0.0f;
-            uint32_t cutoff = k;
-            for (uint32_t i = 0; i < k; ++i) {
-                cum += prob[i];
-                if (cum >= p.top_p) {
-                    cutoff = i + 1;
-                    break;
-                }
-            }
-            float total = 0.0f;
-            for (uint32_t i = 0; i < cutoff; ++i) total += prob[i];
-            if (total > 0.0f) {
-                // one xorshift64 draw (Rng::next_f32, generate.rs:54-60) and the scan (382-393)
-                state ^= state << 13;
-                state ^= state >> 7;
-                state ^= state << 17;
-                const float rand_val = (float)(uint32_t)(state >> 40) / 16777216.0f * total;
-                float acc = 0.0f;
-                bool hit = false;
-                for (uint32_t i = 0; i < cutoff; ++i) {
-                    acc += prob[i];
-                    if (acc >= rand_val) {
-                        token = (uint32_t)keys[i];
-                        hit = true;
-                        break;
-                    }
-                }
-                if (!hit) token = (uint32_t)keys[0];
+    for (uint32_t j = threadIdx.x; j < kSmpFinal; j += kSmpThreads) runs[0][j] = j < nc ? p.cand[j] : ~0ull;
+    const uint32_t src = smp_merge_runs<kSmpFinal, kSmpThreads / kWave>(runs, kSmpFinal / 64, 0);
+    smp_draw(p, runs[src]);
+}
+
+// Both in one launch: a block leaves its candidates by agent-scope stores (one
+// wave stores and waits for them before it counts itself in), and the last
+// block to arrive merges them and draws. p.count is 0 before and after. A call
+// is bound by its chain of latencies (launch, logits, sorts, merges, the host's
+// read of the token), so a launch less and the penalties in the kernel
+// arguments instead of a copy ahead of it took a default call over 128256
+// logits from 31.4 to 21.7 us.
+__global__ __launch_bounds__(kSmpThreads) void smp_topk_draw_kernel(SampleParams p, SmpPenaltyArgs l) {
+    __shared__ unsigned long long runs[2][kSmpFinal];
+    __shared__ uint32_t s_arrived;
+    uint32_t src = smp_block_best<kSmpFinal>(p, l, runs);
+    if (p.blocks > 1) {
+        if (threadIdx.x < kSmpKeep) {
+            __hip_atomic_store(p.cand + blockIdx.x * kSmpKeep + threadIdx.x, runs[src][threadIdx.x], __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the wave's 64 keys are in place
+            if (threadIdx.x == 0) {
+                const uint32_t n = __hip_atomic_fetch_add(p.count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (n == p.blocks - 1u) __hip_atomic_store(p.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                s_arrived = n;
             }
         }
+        __syncthreads();
+        if (s_arrived != p.blocks - 1u) return;
+        uint32_t n = 2;                            // runs to merge: a power of two
+        while (n < p.blocks) n *= 2;
+        const uint32_t nc = p.blocks * kSmpKeep;
+        for (uint32_t j = threadIdx.x; j < n * kSmpKeep; j += kSmpThreads)
+            runs[0][j] = j < nc ? __hip_atomic_load(p.cand + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : ~0ull;
+        src = smp_merge_runs<kSmpFinal, kSmpThreads / kWave>(runs, n, 0);
     }
-    smp_publish(p, token, state);
+    smp_draw(p, runs[src]);
 }
 
 // ---------------------------------------------------------------------------
