@@ -1786,7 +1786,8 @@ int rowdot_entry(qora_hip_ctx* c, int fmt, const void* w, const void* s, const f
     p.cols = (uint32_t)cols;
     p.x = x;
     p.y = y;
-    HIP_TRY(c, launch_rowdot(fmt, rowdot_blocks(p.rows, p.cols, c->cus), p, pick_stream(c, stream)));
+    if (fmt == FMT_Q4 && rowdot_q4m_supported(p)) HIP_TRY(c, launch_rowdot_q4m(p, c->cus, pick_stream(c, stream)));
+    else HIP_TRY(c, launch_rowdot(fmt, rowdot_blocks(p.rows, p.cols, c->cus), p, pick_stream(c, stream)));
     return QORA_HIP_OK;
 }
 

@@ -71,6 +71,9 @@ hipError_t launch_acc_to_f32(const long long* acc, uint32_t n, int paired, float
 // Row-dot GEMV (lm_head). blocks: grid size (also the argmax partial count).
 uint32_t rowdot_blocks(uint32_t rows, uint32_t cols, int cus);
 hipError_t launch_rowdot(int fmt, uint32_t blocks, const RowdotParams& p, hipStream_t stream);
+// Plain Q4 row-dot (x in fp32, no norm, no argmax) on the matrix cores.
+bool rowdot_q4m_supported(const RowdotParams& p);
+hipError_t launch_rowdot_q4m(const RowdotParams& p, int cus, hipStream_t stream);
 hipError_t launch_argmax_finish(const ArgmaxFinishParams& p, hipStream_t stream);
 
 // Tied lm_head on the matrix cores (Q4, cols in {128, 256, 512, 1024, 2048}).

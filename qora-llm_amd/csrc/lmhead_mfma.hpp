@@ -268,4 +268,130 @@ __global__ __launch_bounds__(256) void lmhead_q4m_kernel(LmHeadParams p) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// The same row-dot on the reference layout (qora_hip_gemv_q4_rowdot): y[r] =
+// sum_c x[c] W[r][c], cols = 256 NV. A lane's 16-byte load is one whole scale
+// group of one row, so the contraction of an MFMA pair (even columns, odd
+// columns) is split by group over the lanes' quarters and every A row is used:
+//   A[4 g' + limb][k of quarter g] = limb of x's group where g' == g, else 0
+//   C[4 g + limb][j]: lane (j, g) receives the four limb sums of its own row
+//   and group, one scale each.
+// Unit u of a tile of 16 rows: quarter kq holds group 4 u + kq of row l % 16.
+// The next tile's loads go out as a register is used. A byte of low nibbles is
+// 16 (q - 8) after shift, and, xor.
+// What bounds it: the weight stream. 128256 x 2048 (148 MB): 29.6 us, 5.0 TB/s
+// (a large copy's rate), against 32.6 on the VALU (rowdot_kernel: 17 instructions
+// per 8 weights against 5 and a quarter of an MFMA, and a 64-lane sum per row).
+// Two units share each 128-byte line, so the loads are ordinary ones:
+// non-temporal they took 42.8 us (33.4 with a quarter's two groups adjacent).
+// ---------------------------------------------------------------------------
+template <int NV>
+__global__ __launch_bounds__(256) void rowdot_q4m_kernel(RowdotParams p) {
+    kernarg_warm(p);
+    constexpr int NT = 256, NW = 4;
+    constexpr int COLS = 256 * NV, G = 8 * NV;
+    constexpr int XPT = COLS / NT;
+    __shared__ __align__(16) uint8_t xl[G * 128 + 16];   // [group][even, odd][limb][16], then a zero slot
+    __shared__ float red[NW];
+
+    const int t = threadIdx.x;
+    const int lane = t & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
+    const uint32_t li = (uint32_t)lane % 16u, kq = (uint32_t)lane / 16u;
+    const uint32_t tiles = (p.rows + 15u) / 16u, W = gridDim.x * NW;
+    uint32_t tile = blockIdx.x * NW + (uint32_t)wave;
+
+    float xv[XPT];
+#pragma unroll
+    for (int j = 0; j < XPT; ++j) xv[j] = p.x[t + NT * j];
+
+    // a tile's loads (rows and tiles past the end read the last row)
+    v4u32 wb[2 * NV];
+    uint16_t sb[2 * NV];
+    auto row_of = [&](uint32_t tl) { return min(tl * 16u + li, p.rows - 1u); };
+    auto wptr = [&](uint32_t r) { return p.w + (uint64_t)r * (COLS / 2) + kq * 16u; };
+    auto sptr = [&](uint32_t r) { return p.scales + (uint64_t)r * G + kq; };
+    {
+        const uint32_t r = row_of(tile);
+        const uint8_t* wp = wptr(r);
+        const uint16_t* sp = sptr(r);
+#pragma unroll
+        for (int u = 0; u < 2 * NV; ++u) {
+            wb[u] = *reinterpret_cast<const v4u32*>(wp + u * 64);
+            sb[u] = *reinterpret_cast<const uint16_t*>(sp + u * 4);
+        }
+    }
+
+    float mx = 0.f;
+#pragma unroll
+    for (int j = 0; j < XPT; ++j) mx = fmaxf(mx, fabsf(xv[j]) <= 3.4028235e38f ? fabsf(xv[j]) : INFINITY);   // (NaN too)
+    mx = block_max<NT>(mx, red);
+    if (mx == INFINITY) {
+        // an infinity or NaN in x: no common exponent; every row in fp32, as it was stored
+        for (; tile < tiles; tile += W)
+            for (uint32_t r = tile * 16u; r < min(tile * 16u + 16u, p.rows); ++r) {
+                float a = 0.f;
+                for (uint32_t c = (uint32_t)lane; c < (uint32_t)COLS; c += kWave) {
+                    const uint32_t b = p.w[((uint64_t)r * COLS + c) / 2u];
+                    const float q = (float)((int)((b >> (4u * (c & 1u))) & 0xFu) - 8);
+                    a = fmaf(p.x[c], h2f(p.scales[(uint64_t)r * G + c / 32u]) * q, a);
+                }
+                a = wave_sum(a);
+                if (lane == 0) p.y[r] = a;
+            }
+        return;
+    }
+    const int ex = mx > 0.f ? (int)((__float_as_uint(mx) >> 23) & 0xFFu) - 126 : 0;
+#pragma unroll
+    for (int j = 0; j < XPT; ++j) {
+        const uint32_t c = (uint32_t)(t + NT * j);
+        const int M = (int)rintf(ldexpf(xv[j], 30 - ex));
+        const uint32_t limbs = (uint32_t)(M + 0x808080) ^ 0x808080u;
+        uint8_t* dst = xl + (c / 32u) * 128u + (c & 1u) * 64u + (c % 32u) / 2u;
+        dst[0] = (uint8_t)(limbs & 0xFFu);
+        dst[16] = (uint8_t)((limbs >> 8) & 0xFFu);
+        dst[32] = (uint8_t)((limbs >> 16) & 0xFFu);
+        dst[48] = (uint8_t)(limbs >> 24);
+    }
+    if (t < 4) *reinterpret_cast<uint32_t*>(xl + G * 128 + t * 4) = 0u;
+    __syncthreads();
+
+    // lanes with li / 4 == kq read their group's limb li % 4, the others the
+    // zero slot (both parities and every unit at a fixed stride from there)
+    const bool nz = li / 4u == kq;
+    const uint32_t abase = nz ? kq * 128u + (li % 4u) * 16u : (uint32_t)(G * 128);
+    const uint32_t au = nz ? 512u : 0u, ap = nz ? 64u : 0u;
+    const v4i32 zero = (v4i32){0, 0, 0, 0};
+    for (; tile < tiles; tile += W) {
+        uint32_t ao = abase;
+        asm volatile("" : "+v"(ao));       // (A fragments from LDS every tile, not held in registers)
+        const uint32_t rn = row_of(tile + W);
+        const uint8_t* wp = wptr(rn);
+        const uint16_t* sp = sptr(rn);
+        float acc = 0.f;
+#pragma unroll
+        for (int u = 0; u < 2 * NV; ++u) {
+            const v4u32 w = wb[u];
+            const uint16_t s = sb[u];
+            wb[u] = *reinterpret_cast<const v4u32*>(wp + u * 64);
+            sb[u] = *reinterpret_cast<const uint16_t*>(sp + u * 4);
+            const uint32_t a = ao + (uint32_t)u * au;
+            const v4i32 ae = *reinterpret_cast<const v4i32*>(xl + a);
+            const v4i32 ad = *reinterpret_cast<const v4i32*>(xl + a + ap);
+            v4i32 be, bo;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                be[d] = (int)(((w[d] << 4) & 0xF0F0F0F0u) ^ 0x80808080u);
+                bo[d] = (int)((w[d] & 0xF0F0F0F0u) ^ 0x80808080u);
+            }
+            v4i32 c = __builtin_amdgcn_mfma_i32_16x16x64_i8(ae, be, zero, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_i32_16x16x64_i8(ad, bo, c, 0, 0, 0);
+            acc = fmaf(lm_limb_value(c), h2f(s), acc);
+        }
+        acc = sum_row_slots(acc);
+        const uint32_t r = tile * 16u + (uint32_t)lane;
+        if (lane < 16 && r < p.rows) p.y[r] = ldexpf(acc, ex - 34);
+    }
+}
+
 }  // namespace qora
