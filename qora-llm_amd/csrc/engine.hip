@@ -1199,7 +1199,7 @@ int pf_setup(qora_hip_ctx* c) {
             }
         }
         // the fused launches of the packed-weight GEMM: q|k|v, o, gate|up, down
-        m.pf2 = m.fmt == FMT_Q4 && pf_gemm2_supported(m.hidden, qd) && pf_gemm2_supported(m.hidden, kvd) &&
+        m.pf2 = pf_gemm2_supported(m.hidden, qd) && pf_gemm2_supported(m.hidden, kvd) &&
                 pf_gemm2_supported(qd, m.hidden) && pf_gemm2_supported(m.hidden, m.inter) &&
                 pf_gemm2_supported(m.inter, m.hidden);
         if (m.pf2) {
@@ -1237,7 +1237,7 @@ int pf_setup(qora_hip_ctx* c) {
                                                 scratch, c->stream));
             }
     }
-    if (m.pf2) {
+    if (m.pf2 && m.fmt == FMT_Q4) {
         m.pf_wq.assign((size_t)m.L * 7, nullptr);
         m.pf_sc.assign((size_t)m.L * 7, nullptr);
         for (uint32_t l = 0; l < m.L; ++l)
@@ -1330,9 +1330,13 @@ int pf_gemm2(qora_hip_ctx* c, uint32_t l, std::initializer_list<int> js, uint32_
         const DevWeight* w = get_weight(c, m.wids[wi]);
         if (!w) return fail(c, QORA_HIP_E_STATE, "model weight released");
         PfGemm2Seg& sg = g.seg[g.nseg++];
-        sg.wq = m.pf_wq[wi];
-        sg.sc = m.pf_sc[wi];
-        sg.wf = m.pf_wf[wi];
+        if (m.fmt == FMT_Q4) {
+            sg.wq = m.pf_wq[wi];
+            sg.sc = m.pf_sc[wi];
+            sg.wf = m.pf_wf[wi];
+        } else {
+            sg.wq = (const uint2*)w->w;             // binary16 weights are read as uploaded
+        }
         sg.n = (uint32_t)w->n;
         sg.nb0 = g.ntot / 128u;
         sg.y = *yi++;
@@ -1361,7 +1365,7 @@ int pf_gemm2(qora_hip_ctx* c, uint32_t l, std::initializer_list<int> js, uint32_
     bool side = ldy == g.ntot;
     for (int i = 0; i < g.nseg; ++i) side = side && g.seg[i].y == g.seg[0].y + (size_t)g.seg[i].nb0 * 128u;
     const bool leave = defer && g.splits > 1 && side;
-    HIP_TRY(c, launch_pf_gemm2(sh.bm, g, c->stream, !leave));
+    HIP_TRY(c, launch_pf_gemm2(sh.bm, g, c->stream, !leave, m.fmt == FMT_Q4 ? PF_W_PACKED : PF_W_F16));
     if (defer) *defer = leave ? PfDeferred{g.part, g.splits, (uint64_t)T * g.ntot} : PfDeferred{};
     return QORA_HIP_OK;
 }
@@ -2103,11 +2107,11 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
         HIP_TRY(c, launch_pf_gemm_small(w->fmt, q, s));
         return QORA_HIP_OK;
     }
-    // Q4 with n % 128 == 0 runs the prefill's packed-weight GEMM (the weight
-    // packed into the workspace for this call, with its own scales), anything
-    // else pf_gemm_kernel
-    const bool packed = w->fmt == FMT_Q4 && pf_gemm2_supported(K, N);
-    const bool exps = w->fmt == FMT_Q4 && !packed;
+    // n % 128 == 0 runs the prefill's GEMM (a Q4 weight packed into the
+    // workspace for this call, with its own scales), anything else
+    // pf_gemm_kernel
+    const bool q4 = w->fmt == FMT_Q4, wide = pf_gemm2_supported(K, N), packed = q4 && wide;
+    const bool exps = q4 && !wide;
     // scratch: xh, xl [T][k] binary16, xe [T], then the packed weight (wq, sc)
     // or wf [n/32] and the exponent partials, then the split-K partials (each
     // part 256-byte aligned)
@@ -2115,8 +2119,8 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
     const uint64_t bs = exps ? al(pf_weight_exp_scratch(K, N / 32)) : 0;
     const uint64_t bq = packed ? al((uint64_t)K * N / 2) : 0, bc = packed ? al((uint64_t)K * N / 16) : 0;
     const PfGemmShape sh = pf_gemm_shape((uint32_t)T, K, N, c->cus);
-    const PfGemm2Shape s2 = packed ? pf_gemm2_shape((uint32_t)T, K, N, c->cus) : PfGemm2Shape{};
-    const uint32_t splits = packed ? s2.splits : sh.splits;
+    const PfGemm2Shape s2 = wide ? pf_gemm2_shape((uint32_t)T, K, N, c->cus) : PfGemm2Shape{};
+    const uint32_t splits = wide ? s2.splits : sh.splits;
     const uint64_t bp = splits > 1 ? al((uint64_t)splits * T * N * 4) : 0;
     if (int rc = ensure_pf_ws(c, 2 * bx + be + bf + bs + bq + bc + bp)) return rc;
     uint8_t* base = (uint8_t*)c->ws_pf;
@@ -2128,9 +2132,10 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
     r.xh = (uint16_t*)base;
     r.xl = (uint16_t*)(base + bx);
     r.xe = (int32_t*)(base + 2 * bx);
-    if (packed) {
-        HIP_TRY(c, launch_pf_gemm_prep(x, (uint32_t)T, r.xh, r.xl, r.xe, (const uint8_t*)w->w, (const uint16_t*)w->scales,
+    if (wide) {
+        if (q4) HIP_TRY(c, launch_pf_gemm_prep(x, (uint32_t)T, r.xh, r.xl, r.xe, (const uint8_t*)w->w, (const uint16_t*)w->scales,
                                        K, N, (uint2*)wq, (uint16_t*)(wq + bq), s));
+        else HIP_TRY(c, launch_pf_rows(PF_ROW_SPLIT, r, (uint32_t)T, s));
         PfGemm2Params h{};
         h.xh = r.xh;
         h.xl = r.xl;
@@ -2139,11 +2144,11 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
         h.k = K;
         h.nseg = 1;
         h.ntot = N;
-        h.seg[0] = PfGemm2Seg{(const uint2*)wq, (const uint16_t*)(wq + bq), nullptr, N, 0, y, N, 0};
+        h.seg[0] = PfGemm2Seg{(const uint2*)(q4 ? wq : w->w), (const uint16_t*)(wq + bq), nullptr, N, 0, y, N, 0};
         h.splits = s2.splits;
         h.kper = s2.kper;
         h.part = part;
-        HIP_TRY(c, launch_pf_gemm2(s2.bm, h, s, true, true));
+        HIP_TRY(c, launch_pf_gemm2(s2.bm, h, s, true, q4 ? PF_W_RAW : PF_W_F16));
         return QORA_HIP_OK;
     }
     HIP_TRY(c, launch_pf_rows(PF_ROW_SPLIT, r, (uint32_t)T, s));

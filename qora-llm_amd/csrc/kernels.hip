@@ -844,24 +844,31 @@ PfGemm2Shape pf_gemm2_shape(uint32_t T, uint32_t k, uint32_t ntot, int cus) {
     return sh;
 }
 
-hipError_t launch_pf_gemm2(uint32_t bm, const PfGemm2Params& p, hipStream_t stream, bool reduce, bool raw) {
+hipError_t launch_pf_gemm2(uint32_t bm, const PfGemm2Params& p, hipStream_t stream, bool reduce, PfW wm) {
     if (p.T == 0 || p.k % 32 != 0 || p.nseg < 1 || p.nseg > 3 || p.ntot % 128 != 0 || p.splits == 0 ||
         p.kper % 32 != 0 || (uint64_t)p.splits * p.kper < p.k || (p.splits > 1 && !p.part))
         return hipErrorInvalidValue;
     uint32_t nb = 0;
     for (int i = 0; i < p.nseg; ++i) {
-        if (p.seg[i].nb0 != nb || p.seg[i].n % 128 != 0 || !p.seg[i].wq || !p.seg[i].sc || (!raw && !p.seg[i].wf)) return hipErrorInvalidValue;
+        if (p.seg[i].nb0 != nb || p.seg[i].n % 128 != 0 || !p.seg[i].wq ||
+            (wm != PF_W_F16 && !p.seg[i].sc) || (wm == PF_W_PACKED && !p.seg[i].wf))
+            return hipErrorInvalidValue;
         nb += p.seg[i].n / 128;
     }
     if (nb * 128u != p.ntot) return hipErrorInvalidValue;
     if (p.swiglu && (p.nseg != 2 || p.seg[0].n != p.seg[1].n || p.splits != 1 || !p.seg[0].y || p.seg[0].accumulate))
         return hipErrorInvalidValue;
     const dim3 grid(nb, (p.T + bm - 1) / bm, p.splits);
-    if (bm == 64 && raw) hipLaunchKernelGGL((pf_gemm2_kernel<64, true>), grid, dim3(256), 0, stream, p);
-    else if (bm == 64) hipLaunchKernelGGL((pf_gemm2_kernel<64, false>), grid, dim3(256), 0, stream, p);
-    else if (bm == 32 && raw) hipLaunchKernelGGL((pf_gemm2_kernel<32, true>), grid, dim3(256), 0, stream, p);
-    else if (bm == 32) hipLaunchKernelGGL((pf_gemm2_kernel<32, false>), grid, dim3(256), 0, stream, p);
-    else return hipErrorInvalidValue;
+    if (bm != 32 && bm != 64) return hipErrorInvalidValue;
+#define QORA_PF_GEMM2(WM_)                                                                              \
+    do {                                                                                                \
+        if (bm == 64) hipLaunchKernelGGL((pf_gemm2_kernel<64, WM_>), grid, dim3(256), 0, stream, p);    \
+        else hipLaunchKernelGGL((pf_gemm2_kernel<32, WM_>), grid, dim3(256), 0, stream, p);             \
+    } while (0)
+    if (wm == PF_W_PACKED) QORA_PF_GEMM2(PF_W_PACKED);
+    else if (wm == PF_W_RAW) QORA_PF_GEMM2(PF_W_RAW);
+    else QORA_PF_GEMM2(PF_W_F16);
+#undef QORA_PF_GEMM2
     if (p.splits > 1 && reduce) {
         const uint64_t total = (uint64_t)p.T * p.ntot;
         const uint32_t blocks = (uint32_t)std::min<uint64_t>(4096, (total + 255) / 256);

@@ -138,9 +138,9 @@ struct PfGemm2Shape {
 PfGemm2Shape pf_gemm2_shape(uint32_t T, uint32_t k, uint32_t ntot, int cus);
 // p.splits, p.kper from pf_gemm2_shape (bm too); p.part holds splits * T * ntot floats when splits > 1.
 // reduce = false leaves the split partials for the consumer to sum (pf_rmsnorm_split_reg_kernel).
-// raw: the packed scales are the weight's own (launch_pf_gemm_prep), seg.wf is not read.
+// wm: PF_W_RAW for scales as launch_pf_gemm_prep packs them, PF_W_F16 for binary16 weights.
 hipError_t launch_pf_gemm2(uint32_t bm, const PfGemm2Params& p, hipStream_t stream, bool reduce = true,
-                           bool raw = false);
+                           PfW wm = PF_W_PACKED);
 // x [T][k] split into xh, xl, xe and a Q4 weight packed with its own scales, in one launch
 hipError_t launch_pf_gemm_prep(const float* x, uint32_t T, uint16_t* xh, uint16_t* xl, int32_t* xe, const uint8_t* w,
                                const uint16_t* scales, uint32_t k, uint32_t n, uint2* wq, uint16_t* sc,

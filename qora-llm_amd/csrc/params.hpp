@@ -176,8 +176,11 @@ struct PrefillGemmParams {
 // nibbles of columns 2 bc, 2 bc + 1 of row 32 ks + 8 rg + r (the reference
 // byte); sc[((nb * KS + ks) * 4 + g) * 32 + r] the f16 scale of row 32 ks + r,
 // group g of the block. KS = k / 32.
+// How pf_gemm2_kernel's weights come (its comment has the details).
+enum PfW : int { PF_W_PACKED = 0, PF_W_RAW = 1, PF_W_F16 = 2 };
+
 struct PfGemm2Seg {
-    const uint2* wq;
+    const uint2* wq;           // (PF_W_F16: the binary16 weight [k][n])
     const uint16_t* sc;
     const int8_t* wf;          // per-group exponents [n/32]
     uint32_t n;                // columns (multiple of 128)

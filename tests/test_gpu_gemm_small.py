@@ -83,3 +83,20 @@ def test_gemm_non_finite_row_stays_in_its_row(ctx, pkg):
             assert np.array_equal(got[rows], want[rows])
             assert not np.isfinite(got[7]).all()
     ctx.lib.qora_hip_release_weight(ctx.h, wid)
+
+
+@pytest.mark.parametrize("T,k,n", [(65, 96, 128), (130, 2048, 512), (200, 4128, 256), (512, 512, 1152)])
+def test_gemm_f16_wide_vs_truth(ctx, pkg, T, k, n):
+    """F16 weights whose width is a multiple of 128 above 64 tokens: 32- and
+    64-token tiles, K split and unsplit."""
+    wt, W = _weight(pkg, "f16", k, n, T, None)
+    wid = ctx.upload(wt)
+    x = rng(T).standard_normal((T, k)).astype(np.float32)
+    with device(ctx) as d:
+        y = d.empty(T * n * 4)
+        ctx.check(ctx.lib.qora_hip_gemm(ctx.h, wid, d.put(x), y, T, None))
+        got = d.get(y, (T, n), np.float32)
+    truth = x.astype(np.float64) @ W
+    assert rel_err(got, truth) <= TRUTH_TOL
+    assert elem_err(got, truth, np.abs(x.astype(np.float64)) @ np.abs(W)) <= TRUTH_TOL
+    ctx.lib.qora_hip_release_weight(ctx.h, wid)
