@@ -1183,9 +1183,10 @@ int pf_setup(qora_hip_ctx* c) {
     PF_ALLOC(d_pf_xl, (size_t)tc * kmax * 2);
     PF_ALLOC(d_pf_xe, (size_t)tc * 4);
     PF_ALLOC(d_pf_ids, (size_t)m.cap * 4);
-    // attention key chunks: up to kPfAttnChunks per query block of >= 16 rows,
-    // 64 rows (4 waves x 16) of hd values plus (m, l) per block
-    PF_ALLOC(d_pf_apart, (size_t)((tc + 15) / 16) * kPfAttnChunks * m.KVH * 64 * (m.hd + 2) * 4);
+    // attention key chunks: up to kPfAttnChunks per query block, 16 rows a wave
+    // of hd values plus (m, l): 64 rows per 16 queries or more, the last block's
+    // 128 partly past the chunk
+    PF_ALLOC(d_pf_apart, (size_t)((tc + 15) / 16 + 1) * kPfAttnChunks * m.KVH * 64 * (m.hd + 2) * 4);
     {
         // the largest split-K partial set over every chunk length (the 7 shapes
         // repeat in every layer)

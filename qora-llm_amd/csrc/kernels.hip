@@ -900,7 +900,6 @@ hipError_t launch_pf_attn(const PrefillAttnParams& p, hipStream_t stream) {
     if (p.hd > (uint32_t)kAttnMaxHd || p.hd % 8 != 0 || p.H % p.KVH != 0) return hipErrorInvalidValue;
     const uint32_t G = p.H / p.KVH;
     if ((p.hd == 64 || p.hd == 128) && (G == 1 || G == 2 || G == 4)) {
-        const uint32_t qt = 16u * (4u / G);
         // Key chunks: a query block's keys split over up to part_nc blocks
         // (128 keys each, more when that would exceed part_nc) so that the
         // long rows of the causal triangle do not set the kernel's length;
@@ -921,13 +920,28 @@ hipError_t launch_pf_attn(const PrefillAttnParams& p, hipStream_t stream) {
                 q.ch = ch;
             }
         }
+        // Eight waves share a staged tile where four-wave blocks come near the CUs'
+        // number (16 heads over 4, f32, calls on three streams: 512 tokens 17.0 ->
+        // 12.4 us, behind 700 positions 36.7 -> 25.9), or where one four-wave tile
+        // holds every query and the other waves only help to stage (16 tokens
+        // behind 700 positions, one stream: 48.2 -> 38.8 us). Between the two, four
+        // waves on CUs of their own are as fast or faster (128 tokens, three
+        // streams 4.58 against 4.78; two heads of 64, 160 tokens: 12.1 against 12.7).
+        const uint32_t qt4 = 16u * (4u / G), nt4 = (p.T + qt4 - 1) / qt4;
+        q.nw = nt4 == 1 || (uint64_t)nt4 * p.KVH * q.nc >= 128u ? 8u : 4u;
+        const uint32_t qt = 16u * (q.nw / G);
         const dim3 grid((p.T + qt - 1) / qt * q.nc, p.KVH);
         // with split outputs and chunks, the merge writes the o GEMM's operand itself
         const bool merge_split = p.xh && q.nc > 1 && p.H * p.hd <= 2048u;
+#define QORA_PF_ATTN_NW(HD, F16, NW) \
+    hipLaunchKernelGGL((pf_attn_mfma_kernel<HD, F16, NW>), grid, dim3(64 * NW), 0, stream, q)
 #define QORA_PF_ATTN(HD)                                                                                     \
     do {                                                                                                    \
-        if (p.kv_f16) hipLaunchKernelGGL((pf_attn_mfma_kernel<HD, true>), grid, dim3(256), 0, stream, q);   \
-        else hipLaunchKernelGGL((pf_attn_mfma_kernel<HD, false>), grid, dim3(256), 0, stream, q);           \
+        if (p.kv_f16) {                                                                                     \
+            if (q.nw == 8) QORA_PF_ATTN_NW(HD, true, 8); else QORA_PF_ATTN_NW(HD, true, 4);                  \
+        } else {                                                                                            \
+            if (q.nw == 8) QORA_PF_ATTN_NW(HD, false, 8); else QORA_PF_ATTN_NW(HD, false, 4);                \
+        }                                                                                                   \
         if (merge_split)                                                                                    \
             hipLaunchKernelGGL((pf_attn_merge_split_kernel<HD>), dim3(p.T), dim3(256), 0, stream, q);        \
         else if (q.nc > 1)                                                                                  \
@@ -937,6 +951,7 @@ hipError_t launch_pf_attn(const PrefillAttnParams& p, hipStream_t stream) {
         if (p.hd == 128) QORA_PF_ATTN(128);
         else QORA_PF_ATTN(64);
 #undef QORA_PF_ATTN
+#undef QORA_PF_ATTN_NW
         if (p.xh && !merge_split) return launch_pf_attn_split(p, stream);
         return hipGetLastError();
     }

@@ -239,10 +239,11 @@ struct PrefillAttnParams {
     uint64_t kv_ps, kv_hs;     // cache addressing as in AttnParams (0: token-major)
     // key-range split of the matrix-core kernel: a workspace for up to part_nc
     // key chunks per query block (null / < 2: no split); nc and ch (keys per
-    // chunk, a multiple of 64) are set by the launcher
+    // chunk, a multiple of 64) are set by the launcher, as are its waves a block
     float* part;
     uint32_t part_nc;
     uint32_t nc, ch;
+    uint32_t nw;
     // pf_rope_cache_kernel: optional split-K partials of the q|k|v GEMM,
     // qkv_part[z][T][qd + 2 kvd] (z-stride qkv_part_stride), summed in split
     // order in place of the qkv rows (rows of at most kPfRopeRowMax floats)

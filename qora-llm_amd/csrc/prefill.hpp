@@ -1504,9 +1504,16 @@ __global__ __launch_bounds__(256) void pf_attn_vec_kernel(PrefillAttnParams p) {
 
 // ---------------------------------------------------------------------------
 // Causal prefill attention on the matrix cores. Block (query tile, KV head),
-// 4 waves; wave w takes query head kvh * G + w % G for 16 queries (sub-tile
-// w / G), so the G heads sharing a KV head share each K/V tile staged in LDS
-// (64 keys per step). Per wave and key tile:
+// NW = 4 or 8 waves; wave w takes query head kvh * G + w % G for 16 queries
+// (sub-tile w / G), so the G heads sharing a KV head, and NW / G query tiles,
+// share each K/V tile staged in LDS (64 keys per step). What bounds it: the chain of a tile
+// (loads, the split of K and V into two binary16 parts, two barriers, LDS reads
+// ahead of the MFMAs); the split takes a wave 400 VALU instructions a tile with
+// eight waves and 800 with four, against 320 and 96 MFMAs of attention.
+// 512 tokens, 16 heads over 4, f32 cache, calls on three streams: 13.2 -> 11.7 us
+// a call (12.5 without the reordered MFMAs and the mask's unconditional reads below).
+// Two key groups per block with 32-key tiles each measured 14.0. Per wave and key
+// tile:
 //   * S^T = K Q^T on the f16 matrix cores (v_mfma_f32_16x16x32_f16), K from
 //     LDS as the A operand and Q held in registers as B, each split into two
 //     binary16 parts on a power-of-two scale (per key row, per query: as the
@@ -1528,17 +1535,19 @@ __global__ __launch_bounds__(256) void pf_attn_vec_kernel(PrefillAttnParams p) {
 // 8 (l / 16) + b], B[k = 8 (l / 16) + b][j = l % 16], C[i = 4 (l / 16) + r]
 // [j = l % 16] in register r.
 // ---------------------------------------------------------------------------
-template <int HD, bool F16KV>
-__global__ __launch_bounds__(256, 2) void pf_attn_mfma_kernel(PrefillAttnParams p) {
+template <int HD, bool F16KV, uint32_t NW>
+__global__ __launch_bounds__(64 * NW) void pf_attn_mfma_kernel(PrefillAttnParams p) {
     constexpr int KT = 64;                          // keys per step
+    constexpr uint32_t NT = 64u * NW;
+    constexpr int NP = F16KV ? 1 : 2;               // binary16 parts of k and v (an f16 cache's are exact in one)
     constexpr int QC = HD / 32;                     // 32-deep contraction steps of K Q^T
     constexpr int OC = HD / 16;                     // 16-dim output tiles
     // K of the tile: kt[part][step st][key][32 dims] binary16 (dims 32 st ..),
     // 16-byte chunk c of key r at chunk c ^ ((r >> 1) & 3); ksc[key] = 2^e_k
-    __shared__ __align__(16) _Float16 kt[2][QC][KT * 32];
+    __shared__ __align__(16) _Float16 kt[NP][QC][KT * 32];
     __shared__ __align__(16) float ksc[KT];
     // V of the tile: vt[part][half s][lane group g][dim d][8 keys], binary16
-    __shared__ __align__(16) _Float16 vt[2][2 * 4 * HD * 8];
+    __shared__ __align__(16) _Float16 vt[NP][2 * 4 * HD * 8];
 
     const uint32_t t = threadIdx.x;
     const uint32_t lane = t % kWave, g4 = lane / 16u, li = lane % 16u;
@@ -1546,7 +1555,7 @@ __global__ __launch_bounds__(256, 2) void pf_attn_mfma_kernel(PrefillAttnParams 
     const uint32_t G = p.H / p.KVH, kvh = blockIdx.y;
     const uint32_t sub = wave / G;                  // query sub-tile of this wave
     const uint32_t h = kvh * G + wave % G;
-    const uint32_t QT = 16u * (4u / G);             // queries per block
+    const uint32_t QT = 16u * (NW / G);            // queries per block
     const uint32_t nc = p.nc > 1u ? p.nc : 1u;      // key chunks per query block
     const uint32_t q0 = (blockIdx.x / nc) * QT;     // chunk-relative first query of the block
     const uint32_t qd = p.H * HD, kvd = p.KVH * HD;
@@ -1604,8 +1613,8 @@ __global__ __launch_bounds__(256, 2) void pf_attn_mfma_kernel(PrefillAttnParams 
     // A tile's K and V are loaded into registers one tile ahead (thread e of
     // the K load: key e / (HD/4), dims 4 (e % (HD/4)) ..; of the V load: dim
     // e % HD, keys 4 (e / HD) .. + 3), then staged in LDS.
-    constexpr int KE = KT * HD / 4 / 256;           // K float4s per thread
-    constexpr int VE = HD * KT / 4 / 256;           // V key quads per thread
+    constexpr int KE = KT * HD / 4 / (int)NT;       // K float4s per thread
+    constexpr int VE = HD * KT / 4 / (int)NT;       // V key quads per thread
     float4 kreg[KE];
     float vreg[VE][4];
     // Cache rows addressed from the KV head's base (uniform) by 32-bit byte
@@ -1621,7 +1630,7 @@ __global__ __launch_bounds__(256, 2) void pf_attn_mfma_kernel(PrefillAttnParams 
         if (off32) {
 #pragma unroll
             for (int u = 0; u < KE; ++u) {
-                const uint32_t e = t + 256u * (uint32_t)u;
+                const uint32_t e = t + NT * (uint32_t)u;
                 const uint32_t r = e / (HD / 4), c4 = e % (HD / 4);
                 const uint32_t o = __umul24(min(k0 + r, last), rowb) + 4u * c4 * ES;
                 if constexpr (F16KV) {
@@ -1633,7 +1642,7 @@ __global__ __launch_bounds__(256, 2) void pf_attn_mfma_kernel(PrefillAttnParams 
             }
 #pragma unroll
             for (int u = 0; u < VE; ++u) {
-                const uint32_t e = t + 256u * (uint32_t)u;
+                const uint32_t e = t + NT * (uint32_t)u;
                 const uint32_t d = e % HD, quad = e / HD;
 #pragma unroll
                 for (int rr = 0; rr < 4; ++rr) {
@@ -1646,7 +1655,7 @@ __global__ __launch_bounds__(256, 2) void pf_attn_mfma_kernel(PrefillAttnParams 
         }
 #pragma unroll
         for (int u = 0; u < KE; ++u) {
-            const uint32_t e = t + 256u * (uint32_t)u;
+            const uint32_t e = t + NT * (uint32_t)u;
             const uint32_t r = e / (HD / 4), c4 = e % (HD / 4);
             const uint64_t idx = (uint64_t)min(k0 + r, last) * cps + (uint64_t)kvh * chs + 4u * c4;
             if constexpr (F16KV) {
@@ -1658,7 +1667,7 @@ __global__ __launch_bounds__(256, 2) void pf_attn_mfma_kernel(PrefillAttnParams 
         }
 #pragma unroll
         for (int u = 0; u < VE; ++u) {
-            const uint32_t e = t + 256u * (uint32_t)u;
+            const uint32_t e = t + NT * (uint32_t)u;
             const uint32_t d = e % HD, quad = e / HD;
 #pragma unroll
             for (int rr = 0; rr < 4; ++rr) {
@@ -1674,7 +1683,7 @@ __global__ __launch_bounds__(256, 2) void pf_attn_mfma_kernel(PrefillAttnParams 
         // (max |k| of the row, butterfly over those lanes), then two binary16 parts
 #pragma unroll
         for (int u = 0; u < KE; ++u) {
-            const uint32_t e = t + 256u * (uint32_t)u;
+            const uint32_t e = t + NT * (uint32_t)u;
             const uint32_t r = e / (HD / 4), c4 = e % (HD / 4);
             float4 kv = kreg[u];
             if constexpr (F16KV) {
@@ -1694,12 +1703,12 @@ __global__ __launch_bounds__(256, 2) void pf_attn_mfma_kernel(PrefillAttnParams 
             const uint32_t st = c4 / 8u, ch = ((c4 % 8u) / 2u) ^ ((r >> 1) & 3u);
             const uint32_t o4 = r * 32u + ch * 8u + (c4 % 2u) * 4u;
             *reinterpret_cast<half4v*>(&kt[0][st][o4]) = half4v{kh[0], kh[1], kh[2], kh[3]};
-            *reinterpret_cast<half4v*>(&kt[1][st][o4]) = half4v{kl[0], kl[1], kl[2], kl[3]};
+            if constexpr (NP == 2) *reinterpret_cast<half4v*>(&kt[1][st][o4]) = half4v{kl[0], kl[1], kl[2], kl[3]};
             if (c4 == 0) ksc[r] = ldexpf(1.0f, ek);
         }
 #pragma unroll
         for (int u = 0; u < VE; ++u) {
-            const uint32_t e = t + 256u * (uint32_t)u;
+            const uint32_t e = t + NT * (uint32_t)u;
             const uint32_t d = e % HD, quad = e / HD;   // keys 4 quad .. 4 quad + 3
             const uint32_t hs = quad / 8u, cq = (quad % 8u) / 4u, gq = quad % 4u;
             _Float16 vh[4], vl[4];
@@ -1711,7 +1720,7 @@ __global__ __launch_bounds__(256, 2) void pf_attn_mfma_kernel(PrefillAttnParams 
             }
             const uint32_t o8 = ((hs * 4u + gq) * (uint32_t)HD + d) * 8u + cq * 4u;
             *reinterpret_cast<half4v*>(&vt[0][o8]) = half4v{vh[0], vh[1], vh[2], vh[3]};
-            *reinterpret_cast<half4v*>(&vt[1][o8]) = half4v{vl[0], vl[1], vl[2], vl[3]};
+            if constexpr (NP == 2) *reinterpret_cast<half4v*>(&vt[1][o8]) = half4v{vl[0], vl[1], vl[2], vl[3]};
         }
     };
 
@@ -1725,32 +1734,50 @@ __global__ __launch_bounds__(256, 2) void pf_attn_mfma_kernel(PrefillAttnParams 
         // a wave with no visible key in the tile skips the work, not the barriers
         if (!(wave_on && k0 <= p.pos0 + wq0 + 15u)) continue;
         // ---- S^T = K Q^T: four 16-key x 16-query tiles, three binary16 products
-        // (kh qh + kl qh + kh ql) per 32-deep step ----
+        // (kh qh + kl qh + kh ql; two for an f16 cache) per 32-deep step ----
+        // (each product goes over the four tiles before the next: consecutive
+        // MFMAs then add to different accumulators instead of waiting)
         f32x4v sacc[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            sacc[c] = f32x4v{0.f, 0.f, 0.f, 0.f};
-            const uint32_t o8 = (16u * c + li) * 32u + (g4 ^ ((li >> 1) & 3u)) * 8u;
+        for (int c = 0; c < 4; ++c) sacc[c] = f32x4v{0.f, 0.f, 0.f, 0.f};
+        const uint32_t ko = li * 32u + (g4 ^ ((li >> 1) & 3u)) * 8u;
 #pragma unroll
-            for (int st = 0; st < QC; ++st) {
-                const half8v kh = *reinterpret_cast<const half8v*>(&kt[0][st][o8]);
-                const half8v kl = *reinterpret_cast<const half8v*>(&kt[1][st][o8]);
-                sacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[st], sacc[c], 0, 0, 0);
-                sacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[st], sacc[c], 0, 0, 0);
-                sacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[st], sacc[c], 0, 0, 0);
+        for (int st = 0; st < QC; ++st) {
+            half8v kh[4], kl[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                kh[c] = *reinterpret_cast<const half8v*>(&kt[0][st][512u * c + ko]);
+                if constexpr (NP == 2) kl[c] = *reinterpret_cast<const half8v*>(&kt[1][st][512u * c + ko]);
             }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) sacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[c], qh[st], sacc[c], 0, 0, 0);
+            if constexpr (NP == 2) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) sacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl[c], qh[st], sacc[c], 0, 0, 0);
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) sacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[c], ql[st], sacc[c], 0, 0, 0);
         }
         // ---- online softmax of query li over keys 16 c + 4 g4 + r ----
+        // (the keys' factors read ahead of the masks: under them each became a
+        // branch with its own LDS read)
+        float kf[4][4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float4 v = *reinterpret_cast<const float4*>(&ksc[16u * c + 4u * g4]);
+            kf[c][0] = v.x; kf[c][1] = v.y; kf[c][2] = v.z; kf[c][3] = v.w;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(kf[c][r]));
+        }
         float sv[4][4];
         float mx = -INFINITY;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const float4 kf = *reinterpret_cast<const float4*>(&ksc[16u * c + 4u * g4]);
-            const float kfa[4] = {kf.x, kf.y, kf.z, kf.w};
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const uint32_t kp = k0 + 16u * c + 4u * g4 + (uint32_t)r;
-                sv[c][r] = kp <= qpos ? sacc[c][r] * (kfa[r] * qf) : -INFINITY;
+                const float v = sacc[c][r] * (kf[c][r] * qf);
+                sv[c][r] = kp <= qpos ? v : -INFINITY;
                 mx = fmaxf(mx, sv[c][r]);
             }
         }
@@ -1780,14 +1807,28 @@ __global__ __launch_bounds__(256, 2) void pf_attn_mfma_kernel(PrefillAttnParams 
             for (int r = 0; r < 4; ++r) o[c][r] *= f;
 #pragma unroll
         for (int hs = 0; hs < 2; ++hs) {
+            constexpr int CB = 4;                   // dim tiles per round (as above)
+            static_assert(OC % CB == 0, "whole rounds");
 #pragma unroll
-            for (int c = 0; c < OC; ++c) {
-                const uint32_t o8 = (((uint32_t)hs * 4u + g4) * (uint32_t)HD + 16u * c + li) * 8u;
-                const half8v ah = *reinterpret_cast<const half8v*>(&vt[0][o8]);
-                const half8v al = *reinterpret_cast<const half8v*>(&vt[1][o8]);
-                o[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, ph[hs], o[c], 0, 0, 0);
-                o[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, ph[hs], o[c], 0, 0, 0);
-                o[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, pl[hs], o[c], 0, 0, 0);
+            for (int c0 = 0; c0 < OC; c0 += CB) {
+                half8v ah[CB], al[CB];
+#pragma unroll
+                for (int c = 0; c < CB; ++c) {
+                    const uint32_t o8 = (((uint32_t)hs * 4u + g4) * (uint32_t)HD + 16u * (c0 + c) + li) * 8u;
+                    ah[c] = *reinterpret_cast<const half8v*>(&vt[0][o8]);
+                    if constexpr (NP == 2) al[c] = *reinterpret_cast<const half8v*>(&vt[1][o8]);
+                }
+#pragma unroll
+                for (int c = 0; c < CB; ++c)
+                    o[c0 + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[c], ph[hs], o[c0 + c], 0, 0, 0);
+                if constexpr (NP == 2) {
+#pragma unroll
+                    for (int c = 0; c < CB; ++c)
+                        o[c0 + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[c], ph[hs], o[c0 + c], 0, 0, 0);
+                }
+#pragma unroll
+                for (int c = 0; c < CB; ++c)
+                    o[c0 + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[c], pl[hs], o[c0 + c], 0, 0, 0);
             }
         }
     }
@@ -1799,8 +1840,8 @@ __global__ __launch_bounds__(256, 2) void pf_attn_mfma_kernel(PrefillAttnParams 
         // partial state of the chunk: unnormalised o, running max m and sum l
         // per row, merged by pf_attn_merge_kernel / pf_attn_merge_split_kernel
         const uint64_t blk = (uint64_t)blockIdx.x * p.KVH + kvh;
-        float* po = p.part + (blk * 64u + wave * 16u) * HD;
-        float* pml = p.part + (uint64_t)gridDim.x * p.KVH * 64u * HD + (blk * 64u + wave * 16u) * 2u;
+        float* po = p.part + (blk * 16u * NW + wave * 16u) * HD;
+        float* pml = p.part + (uint64_t)gridDim.x * p.KVH * 16u * NW * HD + (blk * 16u * NW + wave * 16u) * 2u;
 #pragma unroll
         for (int c = 0; c < OC; ++c)
             *reinterpret_cast<float4*>(&po[row * HD + 16 * c + 4 * g4]) = make_float4(o[c][0], o[c][1], o[c][2], o[c][3]);
@@ -1826,14 +1867,14 @@ template <int HD>
 __global__ __launch_bounds__(256) void pf_attn_merge_kernel(PrefillAttnParams p) {
     constexpr uint32_t MC = 8;                      // most chunks (the workspace's bound)
     const uint32_t t = blockIdx.x;
-    const uint32_t G = p.H / p.KVH, QT = 16u * (4u / G), nc = p.nc;
+    const uint32_t G = p.H / p.KVH, QT = 16u * (p.nw / G), nc = p.nc;
     const uint32_t qb = t / QT, qloc = t % QT, sub = qloc / 16u, row = qloc % 16u;
     const uint32_t q0 = qb * QT, nq = min(QT, p.T - q0);
     const uint32_t last = p.pos0 + q0 + nq - 1u;
     const uint32_t nlive = min(min(nc, MC), last / p.ch + 1u);
     const uint64_t nblk = (uint64_t)((p.T + QT - 1u) / QT) * nc * p.KVH;
     const float* po = p.part;
-    const float* pml = p.part + nblk * 64u * HD;
+    const float* pml = p.part + nblk * (16u * p.nw) * HD;
     const uint32_t qd = p.H * HD;
     // thread: element e = head * HD + d of the row (grid.y covers the row in
     // 256-element pieces); every chunk's (m, l, o) requested before any is used
@@ -1845,7 +1886,7 @@ __global__ __launch_bounds__(256) void pf_attn_merge_kernel(PrefillAttnParams p)
 #pragma unroll
         for (uint32_t kc = 0; kc < MC; ++kc) {
             const uint32_t kk = min(kc, nlive - 1u);
-            const uint64_t r = (((uint64_t)qb * nc + kk) * p.KVH + kvh) * 64u + wave * 16u + row;
+            const uint64_t r = (((uint64_t)qb * nc + kk) * p.KVH + kvh) * (16u * p.nw) + wave * 16u + row;
             mv[kc] = pml[r * 2u];
             lv[kc] = pml[r * 2u + 1u];
             ov[kc] = po[r * HD + d];
@@ -1874,14 +1915,14 @@ __global__ __launch_bounds__(256) void pf_attn_merge_split_kernel(PrefillAttnPar
     constexpr uint32_t DPT = 8;                     // dims per thread
     __shared__ float red[4];
     const uint32_t t = blockIdx.x;
-    const uint32_t G = p.H / p.KVH, QT = 16u * (4u / G), nc = p.nc;
+    const uint32_t G = p.H / p.KVH, QT = 16u * (p.nw / G), nc = p.nc;
     const uint32_t qb = t / QT, qloc = t % QT, sub = qloc / 16u, row = qloc % 16u;
     const uint32_t q0 = qb * QT, nq = min(QT, p.T - q0);
     const uint32_t last = p.pos0 + q0 + nq - 1u;
     const uint32_t nlive = min(min(nc, MC), last / p.ch + 1u);
     const uint64_t nblk = (uint64_t)((p.T + QT - 1u) / QT) * nc * p.KVH;
     const float* po = p.part;
-    const float* pml = p.part + nblk * 64u * HD;
+    const float* pml = p.part + nblk * (16u * p.nw) * HD;
     const uint32_t qd = p.H * HD;
     const uint32_t e0 = threadIdx.x * DPT;          // first element of the row (qd <= 256 DPT)
     const bool on = e0 < qd;
@@ -1891,7 +1932,7 @@ __global__ __launch_bounds__(256) void pf_attn_merge_split_kernel(PrefillAttnPar
 #pragma unroll
     for (uint32_t kc = 0; kc < MC; ++kc) {
         const uint32_t kk = min(kc, nlive - 1u);
-        const uint64_t r = (((uint64_t)qb * nc + kk) * p.KVH + kvh) * 64u + wave * 16u + row;
+        const uint64_t r = (((uint64_t)qb * nc + kk) * p.KVH + kvh) * (16u * p.nw) + wave * 16u + row;
         mv[kc] = pml[r * 2u];
         lv[kc] = pml[r * 2u + 1u];
         const float4 a = *reinterpret_cast<const float4*>(po + r * HD + d0);

@@ -1,0 +1,40 @@
+"""Prompt attention (qora_hip_attn_prefill) at the edges of its query tiles (four or
+eight waves: 16 or 32 queries with four heads a KV head, up to 128 with one) and
+64-key steps, f32 and f16 caches, against float64. 64 heads over 16 take the eight
+waves from 113 tokens on. The bound is the prompt attention
+tests' own kind: fp32 sums of products held to 22 bits, relative to max |v|."""
+import numpy as np
+import pytest
+
+from helpers import device, rng
+
+pytestmark = pytest.mark.gpu
+
+
+def _truth(q, k, v, pos0, T, H, KVH, hd):
+    out = np.empty((T, H, hd))
+    q, k, v = q.reshape(T, H, hd), k.reshape(-1, KVH, hd), v.reshape(-1, KVH, hd)
+    for h in range(H):
+        g = h // (H // KVH)
+        s = q[:, h] @ k[:, g].T / np.sqrt(hd)
+        s[np.arange(pos0 + T)[None, :] > pos0 + np.arange(T)[:, None]] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        out[:, h] = p / p.sum(1, keepdims=True) @ v[:, g]
+    return out.reshape(T, H * hd)
+
+
+@pytest.mark.parametrize("kv_f16", [0, 1])
+@pytest.mark.parametrize("H,KVH,hd", [(8, 2, 128), (4, 2, 64), (2, 2, 64), (2, 2, 128), (64, 16, 64)])
+@pytest.mark.parametrize("T,pos0", [(1, 0), (16, 47), (17, 0), (31, 1), (32, 32), (33, 63), (65, 64), (128, 0), (129, 200)])
+def test_query_and_key_tile_edges(ctx, kv_f16, H, KVH, hd, T, pos0):
+    r = rng(T * 7 + hd)
+    q = r.standard_normal((T, H * hd)).astype(np.float32) * 2
+    k, v = (r.standard_normal((pos0 + T, KVH * hd)).astype(np.float16 if kv_f16 else np.float32) for _ in range(2))
+    if kv_f16:
+        k.flat[::97] = np.float16(6e-8)         # subnormals
+    truth = _truth(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), pos0, T, H, KVH, hd)
+    with device(ctx) as d:
+        out = d.empty(T * H * hd * 4)
+        ctx.check(ctx.lib.qora_hip_attn_prefill(ctx.h, d.put(q), d.put(k), d.put(v), kv_f16, pos0, T, H, KVH, hd, out, None))
+        got = d.get(out, (T, H * hd), np.float32)
+    assert np.max(np.abs(got - truth)) <= 1e-5 * np.max(np.abs(v.astype(np.float64)))
