@@ -182,6 +182,11 @@ struct PreparedGemv {
     void* part_idx = nullptr;
 };
 
+// a counter per query block (16 rows or more) and KV head that the key split's
+// rows hold in two chunks or more; the rows' 128 values, m and l
+constexpr size_t kPfAttnOneCounts = kPfAttnOneRows / 64 / 2;
+constexpr size_t kPfAttnOneBytes = kPfAttnOneCounts * sizeof(uint32_t) + (size_t)kPfAttnOneRows * (128 + 2) * sizeof(float);
+
 struct qora_hip_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -217,6 +222,9 @@ struct qora_hip_ctx {
     uint64_t ws_pf_bytes = 0;
     float* ws_attn_part = nullptr;
     uint64_t ws_attn_part_n = 0;
+    // qora_hip_attn_prefill's key split, made with the context (17 MB; null if that
+    // allocation failed: calls then go unsplit): counters, then the chunks' rows
+    void* ws_pa = nullptr;
     int32_t* h_pin = nullptr;            // pinned staging: [0] token in, [1] token out, [2] pos
     // The step's argmax, stored by argmax_finish_kernel straight into mapped,
     // coherent pinned memory: reading it back takes the stream sync only, not
@@ -542,6 +550,15 @@ extern "C" int qora_hip_create(int device, qora_hip_ctx** out) {
     } else {
         c->h_tok = nullptr;
     }
+    if (hipMalloc(&c->ws_pa, kPfAttnOneBytes) == hipSuccess) {
+        if (hipMemsetAsync(c->ws_pa, 0, kPfAttnOneCounts * sizeof(uint32_t), c->stream) != hipSuccess) {
+            (void)hipFree(c->ws_pa);
+            c->ws_pa = nullptr;
+        }
+    } else {
+        (void)hipGetLastError();
+        c->ws_pa = nullptr;
+    }
     *out = c;
     return QORA_HIP_OK;
 }
@@ -558,7 +575,7 @@ extern "C" int qora_hip_destroy(qora_hip_ctx* c) {
         if (w.w) (void)hipFree(w.w);
         if (w.scales) (void)hipFree(w.scales);
     }
-    for (void* p : {(void*)c->ws_count, (void*)c->ws_attn_part, c->ws_pf, (void*)c->smp_rng, (void*)c->smp_pen, c->smp_sort})
+    for (void* p : {(void*)c->ws_count, (void*)c->ws_attn_part, c->ws_pa, c->ws_pf, (void*)c->smp_rng, (void*)c->smp_pen, c->smp_sort})
         if (p) (void)hipFree(p);
     for (void* p : c->ws_old) (void)hipFree(p);
     if (c->h_pin) (void)hipHostFree(c->h_pin);
@@ -2195,7 +2212,12 @@ extern "C" int qora_hip_attn_prefill(qora_hip_ctx* c, const float* q, const void
     a.hd = hd;
     a.scale = 1.0f / sqrtf((float)hd);
     a.out = out;
-    HIP_TRY(c, launch_pf_attn(a, pick_stream(c, stream)));
+    const hipStream_t s = pick_stream(c, stream);
+    if (c->ws_pa && in_order(c, s)) {
+        a.count = (uint32_t*)c->ws_pa;
+        a.part = (float*)(a.count + kPfAttnOneCounts);
+    }
+    HIP_TRY(c, launch_pf_attn(a, s));
     return QORA_HIP_OK;
 }
 

@@ -908,7 +908,7 @@ hipError_t launch_pf_attn(const PrefillAttnParams& p, hipStream_t stream) {
         PrefillAttnParams q = p;
         q.nc = 1;
         q.ch = 0;
-        if (p.part && p.part_nc >= 2 && p.part_nc <= 8) {   // 8: pf_attn_merge_kernel's bound
+        if (p.part && !p.count && p.part_nc >= 2 && p.part_nc <= 8) {   // 8: pf_attn_merge_kernel's bound
             const uint32_t keys = p.pos0 + p.T;
             uint32_t ch = 128;
             const char* ec = tuning_env("QORA_HIP_PF_ATTN_CH");
@@ -920,15 +920,40 @@ hipError_t launch_pf_attn(const PrefillAttnParams& p, hipStream_t stream) {
                 q.ch = ch;
             }
         }
-        // Eight waves share a staged tile where four-wave blocks come near the CUs'
-        // number (16 heads over 4, f32, calls on three streams: 512 tokens 17.0 ->
-        // 12.4 us, behind 700 positions 36.7 -> 25.9), or where one four-wave tile
-        // holds every query and the other waves only help to stage (16 tokens
-        // behind 700 positions, one stream: 48.2 -> 38.8 us). Between the two, four
-        // waves on CUs of their own are as fast or faster (128 tokens, three
-        // streams 4.58 against 4.78; two heads of 64, 160 tokens: 12.1 against 12.7).
         const uint32_t qt4 = 16u * (4u / G), nt4 = (p.T + qt4 - 1) / qt4;
-        q.nw = nt4 == 1 || (uint64_t)nt4 * p.KVH * q.nc >= 128u ? 8u : 4u;
+        const uint64_t blocks4 = (uint64_t)nt4 * p.KVH;
+        const uint64_t kt = ((uint64_t)p.pos0 + p.T + 63u) / 64u;   // 64-key tiles
+        // The one-launch split of the kernel-level entry. A tile takes a block
+        // 3.7 us (f32; f16 1.9) of a chain that only more blocks shorten, a chunk's
+        // store, arrival and merge some 4 us and 0.7 for each chunk to merge: two
+        // tiles a chunk, more with the root of their number, and no more chunks
+        // than give a block to every CU. From four tiles on (f16: six): 200 tokens
+        // 18.7 -> 16.1 us a call on one stream, 512 34.4 -> 24.3, 16 behind 1500
+        // positions 72 -> 22.5 (f16 47 -> 19.5); at three tiles 15.9 against 15.8.
+        if (p.count) {
+            q.count = nullptr;
+            uint64_t ct = 2;
+            while (3u * ct * ct < kt) ++ct;
+            const uint64_t rows = (blocks4 + p.KVH) * 64u;   // of a chunk, at most
+            const uint64_t most = std::min(kPfAttnOneRows / rows, 256u / blocks4);
+            if (kt >= (p.kv_f16 ? 6u : 4u) && most >= 2) {
+                ct = std::max(ct, (kt + most - 1) / most);
+                q.count = p.count;
+                q.ch = (uint32_t)(64u * ct);
+                q.nc = (uint32_t)((kt + ct - 1) / ct);
+            }
+        }
+        // Eight waves on a staged tile where one four-wave tile holds every query
+        // (the other waves help to stage: 16 tokens behind 700 positions, unsplit,
+        // 48.2 -> 38.8 us), and for f32, whose staging costs most, where the blocks
+        // outnumber what the CUs hold: unsplit from 128 four-wave blocks (512 tokens
+        // on three streams 17.0 -> 12.4 us), split from 2048 block tiles (512 behind
+        // 1500 positions 44.3 -> 35). Below, four waves on CUs of their own are as
+        // fast or faster (128 tokens on three streams 4.58 against 4.78; split, 512
+        // tokens 24.3 against 27.4), as for f16 (512 tokens, one stream, 21.3
+        // against 24.6).
+        const bool many = q.count ? blocks4 * kt >= 2048u : blocks4 * q.nc >= 128u;
+        q.nw = nt4 == 1 || (many && !p.kv_f16) ? 8u : 4u;
         const uint32_t qt = 16u * (q.nw / G);
         const dim3 grid((p.T + qt - 1) / qt * q.nc, p.KVH);
         // with split outputs and chunks, the merge writes the o GEMM's operand itself
@@ -944,7 +969,7 @@ hipError_t launch_pf_attn(const PrefillAttnParams& p, hipStream_t stream) {
         }                                                                                                   \
         if (merge_split)                                                                                    \
             hipLaunchKernelGGL((pf_attn_merge_split_kernel<HD>), dim3(p.T), dim3(256), 0, stream, q);        \
-        else if (q.nc > 1)                                                                                  \
+        else if (q.nc > 1 && !q.count)                                                                      \
             hipLaunchKernelGGL((pf_attn_merge_kernel<HD>), dim3(p.T, (p.H * HD + 255) / 256), dim3(256), 0,  \
                                stream, q);                                                                  \
     } while (0)

@@ -221,6 +221,10 @@ struct PfSmallParams {
     float* part;
 };
 
+// rows (hd values, m and l) of the one-launch key split's workspace: 256 blocks of
+// eight waves, 17 MB
+constexpr uint32_t kPfAttnOneRows = 256 * 128;
+
 struct PrefillAttnParams {
     const float* qkv;          // GEMM output rows [T][qd + 2 kvd]
     float* q;                  // rotated q [T][qd]
@@ -244,6 +248,10 @@ struct PrefillAttnParams {
     uint32_t part_nc;
     uint32_t nc, ch;
     uint32_t nw;
+    // a split in one launch (qora_hip_attn_prefill): part holds kPfAttnOneRows
+    // rows, and count a counter per (query block, KV head), zero between
+    // launches, by which a query block's last key chunk finds that it merges them
+    uint32_t* count;
     // pf_rope_cache_kernel: optional split-K partials of the q|k|v GEMM,
     // qkv_part[z][T][qd + 2 kvd] (z-stride qkv_part_stride), summed in split
     // order in place of the qkv rows (rows of at most kPfRopeRowMax floats)

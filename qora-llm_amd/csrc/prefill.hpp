@@ -1512,6 +1512,9 @@ __global__ __launch_bounds__(256) void pf_attn_vec_kernel(PrefillAttnParams p) {
 // eight waves and 800 with four, against 320 and 96 MFMAs of attention.
 // 512 tokens, 16 heads over 4, f32 cache, calls on three streams: 13.2 -> 11.7 us
 // a call (12.5 without the reordered MFMAs and the mask's unconditional reads below).
+// An f16 cache is staged as it is, without split or exponent: 512 tokens behind 1500
+// positions 102 -> 68 us. Few query tiles leave the chip idle while each block walks
+// its keys alone; with p.count the keys are split over blocks in the same launch.
 // Two key groups per block with 32-key tiles each measured 14.0. Per wave and key
 // tile:
 //   * S^T = K Q^T on the f16 matrix cores (v_mfma_f32_16x16x32_f16), K from
@@ -1536,14 +1539,15 @@ __global__ __launch_bounds__(256) void pf_attn_vec_kernel(PrefillAttnParams p) {
 // [j = l % 16] in register r.
 // ---------------------------------------------------------------------------
 template <int HD, bool F16KV, uint32_t NW>
-__global__ __launch_bounds__(64 * NW) void pf_attn_mfma_kernel(PrefillAttnParams p) {
+__global__ __launch_bounds__(64 * NW, 2) void pf_attn_mfma_kernel(PrefillAttnParams p) {
     constexpr int KT = 64;                          // keys per step
     constexpr uint32_t NT = 64u * NW;
     constexpr int NP = F16KV ? 1 : 2;               // binary16 parts of k and v (an f16 cache's are exact in one)
     constexpr int QC = HD / 32;                     // 32-deep contraction steps of K Q^T
     constexpr int OC = HD / 16;                     // 16-dim output tiles
     // K of the tile: kt[part][step st][key][32 dims] binary16 (dims 32 st ..),
-    // 16-byte chunk c of key r at chunk c ^ ((r >> 1) & 3); ksc[key] = 2^e_k
+    // 16-byte chunk c of key r at chunk c ^ ((r >> 1) & 3); ksc[key] = 2^e_k (an f16
+    // cache's values are staged as they are)
     __shared__ __align__(16) _Float16 kt[NP][QC][KT * 32];
     __shared__ __align__(16) float ksc[KT];
     // V of the tile: vt[part][half s][lane group g][dim d][8 keys], binary16
@@ -1685,11 +1689,12 @@ __global__ __launch_bounds__(64 * NW) void pf_attn_mfma_kernel(PrefillAttnParams
         for (int u = 0; u < KE; ++u) {
             const uint32_t e = t + NT * (uint32_t)u;
             const uint32_t r = e / (HD / 4), c4 = e % (HD / 4);
-            float4 kv = kreg[u];
-            if constexpr (F16KV) {
-                const uint32_t ax = __float_as_uint(kv.x), ay = __float_as_uint(kv.y);
-                kv = make_float4(h2f((uint16_t)(ax & 0xFFFFu)), h2f((uint16_t)(ax >> 16)),
-                                 h2f((uint16_t)(ay & 0xFFFFu)), h2f((uint16_t)(ay >> 16)));
+            const uint32_t st = c4 / 8u, ch = ((c4 % 8u) / 2u) ^ ((r >> 1) & 3u);
+            const uint32_t o4 = r * 32u + ch * 8u + (c4 % 2u) * 4u;
+            const float4 kv = kreg[u];
+            if constexpr (F16KV) {                  // the cache's own values: no exponent, nothing left over
+                *reinterpret_cast<uint2*>(&kt[0][st][o4]) = make_uint2(__float_as_uint(kv.x), __float_as_uint(kv.y));
+                continue;
             }
             const float amax = group_max<HD / 4>(fmaxf(fmaxf(fabsf(kv.x), fabsf(kv.y)), fmaxf(fabsf(kv.z), fabsf(kv.w))));
             const int ek = pf_row_exponent(amax);
@@ -1700,8 +1705,6 @@ __global__ __launch_bounds__(64 * NW) void pf_attn_mfma_kernel(PrefillAttnParams
                 kh[q4] = (_Float16)kin[q4];
                 kl[q4] = (_Float16)(kin[q4] - (float)kh[q4]);
             }
-            const uint32_t st = c4 / 8u, ch = ((c4 % 8u) / 2u) ^ ((r >> 1) & 3u);
-            const uint32_t o4 = r * 32u + ch * 8u + (c4 % 2u) * 4u;
             *reinterpret_cast<half4v*>(&kt[0][st][o4]) = half4v{kh[0], kh[1], kh[2], kh[3]};
             if constexpr (NP == 2) *reinterpret_cast<half4v*>(&kt[1][st][o4]) = half4v{kl[0], kl[1], kl[2], kl[3]};
             if (c4 == 0) ksc[r] = ldexpf(1.0f, ek);
@@ -1711,14 +1714,19 @@ __global__ __launch_bounds__(64 * NW) void pf_attn_mfma_kernel(PrefillAttnParams
             const uint32_t e = t + NT * (uint32_t)u;
             const uint32_t d = e % HD, quad = e / HD;   // keys 4 quad .. 4 quad + 3
             const uint32_t hs = quad / 8u, cq = (quad % 8u) / 4u, gq = quad % 4u;
+            const uint32_t o8 = ((hs * 4u + gq) * (uint32_t)HD + d) * 8u + cq * 4u;
+            if constexpr (F16KV) {
+                const uint32_t v01 = __float_as_uint(vreg[u][0]) | __float_as_uint(vreg[u][1]) << 16;
+                const uint32_t v23 = __float_as_uint(vreg[u][2]) | __float_as_uint(vreg[u][3]) << 16;
+                *reinterpret_cast<uint2*>(&vt[0][o8]) = make_uint2(v01, v23);
+                continue;
+            }
             _Float16 vh[4], vl[4];
 #pragma unroll
             for (int rr = 0; rr < 4; ++rr) {
-                const float v = F16KV ? h2f((uint16_t)__float_as_uint(vreg[u][rr])) : vreg[u][rr];
-                vh[rr] = (_Float16)v;
-                vl[rr] = (_Float16)(v - (float)vh[rr]);
+                vh[rr] = (_Float16)vreg[u][rr];
+                vl[rr] = (_Float16)(vreg[u][rr] - (float)vh[rr]);
             }
-            const uint32_t o8 = ((hs * 4u + gq) * (uint32_t)HD + d) * 8u + cq * 4u;
             *reinterpret_cast<half4v*>(&vt[0][o8]) = half4v{vh[0], vh[1], vh[2], vh[3]};
             if constexpr (NP == 2) *reinterpret_cast<half4v*>(&vt[1][o8]) = half4v{vl[0], vl[1], vl[2], vl[3]};
         }
@@ -1764,6 +1772,7 @@ __global__ __launch_bounds__(64 * NW) void pf_attn_mfma_kernel(PrefillAttnParams
         float kf[4][4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
+            if constexpr (F16KV) break;
             const float4 v = *reinterpret_cast<const float4*>(&ksc[16u * c + 4u * g4]);
             kf[c][0] = v.x; kf[c][1] = v.y; kf[c][2] = v.z; kf[c][3] = v.w;
 #pragma unroll
@@ -1776,7 +1785,7 @@ __global__ __launch_bounds__(64 * NW) void pf_attn_mfma_kernel(PrefillAttnParams
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const uint32_t kp = k0 + 16u * c + 4u * g4 + (uint32_t)r;
-                const float v = sacc[c][r] * (kf[c][r] * qf);
+                const float v = sacc[c][r] * (F16KV ? qf : kf[c][r] * qf);
                 sv[c][r] = kp <= qpos ? v : -INFINITY;
                 mx = fmaxf(mx, sv[c][r]);
             }
@@ -1832,11 +1841,80 @@ __global__ __launch_bounds__(64 * NW) void pf_attn_mfma_kernel(PrefillAttnParams
             }
         }
     }
-    if (!wave_on) return;
     // lane (g4, li): O^T[dims 16 c + 4 g4 + r][query li]
     const uint32_t row = li;                        // query within the wave's 16
-    if (wq0 + row >= q0 + nq) return;
-    if (nc > 1u) {
+    if (p.count && last >= p.ch) {
+        // One launch: every chunk stores its state past this XCD's L2 (each
+        // lane's 16-byte pieces 64 lanes apart, so a wave's stores are whole
+        // lines), and the last of the query block's chunks to arrive merges
+        // them in chunk order: out = sum_c 2^(m_c - M) o_c / sum_c 2^(m_c - M) l_c.
+        const uint32_t nlive = last / p.ch + 1u, kc = blockIdx.x % nc;
+        const uint64_t wrow = (((uint64_t)(blockIdx.x / nc) * p.KVH + kvh) * nc) * NW + wave;   // + NW per chunk
+        using u64 = unsigned long long;
+        union F4 { float f[4]; u64 u[2]; };
+        u64* const pw = reinterpret_cast<u64*>(p.part);
+        u64* const pm = pw + (uint64_t)kPfAttnOneRows * (HD / 2);
+        if (wave_on) {
+            const uint64_t w = wrow + (uint64_t)kc * NW;
+#pragma unroll
+            for (int c = 0; c < OC; ++c) {
+                F4 v;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v.f[r] = o[c][r];
+                u64* const d = pw + ((w * OC + c) * kWave + lane) * 2u;
+                __hip_atomic_store(d, v.u[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(d + 1, v.u[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if (g4 == 0) {
+                F4 v;
+                v.f[0] = m;
+                v.f[1] = l;
+                __hip_atomic_store(pm + w * 16u + li, v.u[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        __shared__ uint32_t s_arrived;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's state is in place
+        __syncthreads();
+        if (t == 0) {
+            uint32_t* cnt = p.count + (blockIdx.x / nc) * p.KVH + kvh;
+            const uint32_t n = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (n == nlive - 1u) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_arrived = n;
+        }
+        __syncthreads();
+        if (s_arrived != nlive - 1u || !wave_on) return;
+        float M = -INFINITY;
+        for (uint32_t k = 0; k < nlive; ++k) {
+            F4 v;
+            v.u[0] = __hip_atomic_load(pm + (wrow + (uint64_t)k * NW) * 16u + li, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+            M = fmaxf(M, v.f[0]);
+        }
+        const float mref = M == -INFINITY ? 0.f : M;
+        l = 0.f;
+#pragma unroll
+        for (int c = 0; c < OC; ++c) o[c] = f32x4v{0.f, 0.f, 0.f, 0.f};
+        for (uint32_t k = 0; k < nlive; ++k) {
+            const uint64_t w = wrow + (uint64_t)k * NW;
+            F4 ml, v[OC];
+            ml.u[0] = __hip_atomic_load(pm + w * 16u + li, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int c = 0; c < OC; ++c) {
+                u64* const d = pw + ((w * OC + c) * kWave + lane) * 2u;
+                v[c].u[0] = __hip_atomic_load(d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                v[c].u[1] = __hip_atomic_load(d + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            const float f = __builtin_amdgcn_exp2f(ml.f[0] - mref);
+            l = fmaf(f, ml.f[1], l);
+#pragma unroll
+            for (int c = 0; c < OC; ++c)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[c][r] = fmaf(f, v[c].f[r], o[c][r]);
+        }
+        if (wq0 + row >= q0 + nq) return;
+    } else if (!wave_on || wq0 + row >= q0 + nq) {
+        return;
+    } else if (nc > 1u && !p.count) {
         // partial state of the chunk: unnormalised o, running max m and sum l
         // per row, merged by pf_attn_merge_kernel / pf_attn_merge_split_kernel
         const uint64_t blk = (uint64_t)blockIdx.x * p.KVH + kvh;

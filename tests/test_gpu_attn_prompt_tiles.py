@@ -25,7 +25,8 @@ def _truth(q, k, v, pos0, T, H, KVH, hd):
 
 @pytest.mark.parametrize("kv_f16", [0, 1])
 @pytest.mark.parametrize("H,KVH,hd", [(8, 2, 128), (4, 2, 64), (2, 2, 64), (2, 2, 128), (64, 16, 64)])
-@pytest.mark.parametrize("T,pos0", [(1, 0), (16, 47), (17, 0), (31, 1), (32, 32), (33, 63), (65, 64), (128, 0), (129, 200)])
+@pytest.mark.parametrize("T,pos0", [(1, 0), (16, 47), (17, 0), (31, 1), (32, 32), (33, 63), (65, 64), (128, 0), (129, 200),
+                                    (1, 255), (20, 192), (60, 1111), (193, 0), (300, 5)])
 def test_query_and_key_tile_edges(ctx, kv_f16, H, KVH, hd, T, pos0):
     r = rng(T * 7 + hd)
     q = r.standard_normal((T, H * hd)).astype(np.float32) * 2
@@ -38,3 +39,41 @@ def test_query_and_key_tile_edges(ctx, kv_f16, H, KVH, hd, T, pos0):
         ctx.check(ctx.lib.qora_hip_attn_prefill(ctx.h, d.put(q), d.put(k), d.put(v), kv_f16, pos0, T, H, KVH, hd, out, None))
         got = d.get(out, (T, H * hd), np.float32)
     assert np.max(np.abs(got - truth)) <= 1e-5 * np.max(np.abs(v.astype(np.float64)))
+
+
+def test_f16_cache_of_subnormals(ctx):
+    """An f16 cache goes to the matrix cores as it is stored: subnormal keys and
+    values count in full (scores here are of order one, from q near 2^20)."""
+    r = rng(5)
+    T, H, hd = 70, 4, 64
+    k, v = ((r.integers(-900, 900, (T, hd)) * 2.0 ** -24).astype(np.float16) for _ in range(2))
+    q = (r.standard_normal((T, H * hd)) * 2.0 ** 13).astype(np.float32)
+    truth = _truth(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), 0, T, H, 1, hd)
+    with device(ctx) as d:
+        out = d.empty(T * H * hd * 4)
+        ctx.check(ctx.lib.qora_hip_attn_prefill(ctx.h, d.put(q), d.put(k), d.put(v), 1, 0, T, H, 1, hd, out, None))
+        got = d.get(out, (T, H * hd), np.float32)
+    assert np.max(np.abs(got - truth)) <= 1e-5 * np.max(np.abs(v.astype(np.float64)))
+
+
+def test_split_keys_come_out_as_whole_ones(ctx):
+    """Calls on the context's stream split the keys over blocks (193 or more of
+    them). Chunks merge in key order whichever block is last, so the bits are the
+    same call after call; (512, 1600) takes the split's eight waves, and the split's
+    counters are back at zero for the next shape."""
+    r = rng(9)
+    H, KVH, hd = 16, 4, 128
+    for T, pos0 in ((40, 700), (257, 0), (16, 180), (512, 90), (512, 1600), (40, 700)):
+        q = r.standard_normal((T, H * hd)).astype(np.float32)
+        k, v = (r.standard_normal((pos0 + T, KVH * hd)).astype(np.float32) for _ in range(2))
+        truth = _truth(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), pos0, T, H, KVH, hd)
+        with device(ctx) as d:
+            out = d.empty(T * H * hd * 4)
+            args = (ctx.h, d.put(q), d.put(k), d.put(v), 0, pos0, T, H, KVH, hd, out)
+            first = None
+            for _ in range(4):
+                ctx.check(ctx.lib.qora_hip_attn_prefill(*args, None))
+                got = d.get(out, (T, H * hd), np.float32)
+                first = got if first is None else first
+                np.testing.assert_array_equal(got, first)
+        assert np.max(np.abs(first - truth)) <= 1e-5 * np.max(np.abs(v))
