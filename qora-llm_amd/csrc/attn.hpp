@@ -101,6 +101,81 @@ __device__ __forceinline__ void attn_store_tile(const KvTileRegs<TL>& r, uint32_
     }
 }
 
+// The end of attn_decode_kernel in a launch that merges its own splits (AttnOneParams):
+// every split stores its state past this XCD's L2, and the KV head's last one to
+// arrive merges them as attn_combine_kernel does, with the same sums in the same
+// order. A second launch is what the small calls wait for: the host's 2.8 us and
+// the gap on the GPU.
+template <int DPL>
+__device__ __forceinline__ void attn_merge_last(const AttnOneParams& p, uint32_t kvh, uint32_t split, uint32_t hd,
+                                                uint32_t G, uint32_t g, const float (&acc)[DPL], float m, float l,
+                                                bool vlane, uint32_t dv0c, float* w) {
+    static_assert(kAttnMaxSplits <= kWave, "a split per lane");
+    __shared__ float s_inv[kAttnMaxGroups];
+    __shared__ uint32_t s_arrived;
+    const uint32_t t = threadIdx.x, lane = t % kWave, n = (p.L + p.chunk - 1) / p.chunk;
+    float* out = p.out + (uint64_t)kvh * G * hd;
+    if (n == 1) {
+        if (g < G && vlane) {
+            const float inv = 1.0f / l;
+#pragma unroll
+            for (int i = 0; i < DPL; ++i) out[g * hd + dv0c + i] = acc[i] * inv;
+        }
+        return;
+    }
+    float* base = p.part + (uint64_t)kvh * p.s_max * G * (hd + 2);
+    if (g < G) {
+        float* part = base + ((uint64_t)split * G + g) * (hd + 2);
+        if (vlane) {
+#pragma unroll
+            for (int i = 0; i < DPL; ++i)
+                __hip_atomic_store(part + dv0c + i, acc[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (lane == 0) {
+            __hip_atomic_store(part + hd, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(part + hd + 1, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's state is in place
+    __syncthreads();
+    if (t == 0) {
+        const uint32_t a = __hip_atomic_fetch_add(p.count + kvh, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (a == n - 1u) __hip_atomic_store(p.count + kvh, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_arrived = a;
+    }
+    __syncthreads();
+    if (s_arrived != n - 1u) return;
+    // w[g][split] = e^(m_s - M): one wave per query head
+    if (g < G) {
+        const float* ps = base + ((uint64_t)min(lane, n - 1u) * G + g) * (hd + 2);
+        const float ms = __hip_atomic_load(ps + hd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const float ls = __hip_atomic_load(ps + hd + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const float M = wave_max(lane < n ? ms : -INFINITY);
+        const float e = lane < n ? expf(ms - M) : 0.f;
+        const float den = wave_sum(lane < n ? ls * e : 0.f);
+        w[g * kWave + lane] = e;
+        if (lane == 0) s_inv[g] = 1.0f / den;
+    }
+    __syncthreads();
+    for (uint32_t i = t; i < G * hd; i += 256) {
+        const uint32_t gg = i / hd;
+        const float* pd = base + (uint64_t)gg * (hd + 2) + i % hd;
+        const float inv = s_inv[gg];
+        float v = 0.f;
+        for (uint32_t s0 = 0; s0 < n; s0 += 16) {
+            float x[16];
+#pragma unroll
+            for (uint32_t u = 0; u < 16; ++u)
+                x[u] = __hip_atomic_load(pd + (uint64_t)min(s0 + u, n - 1u) * G * (hd + 2), __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (uint32_t u = 0; u < 16; ++u)
+                if (s0 + u < n) v = fmaf(x[u], w[gg * kWave + s0 + u] * inv, v);
+        }
+        out[i] = v;
+    }
+}
+
 // Block (split, kvh) walks its positions in passes of 32. Each pass's K and
 // V rows are loaded once per block with coalesced 16-byte loads (256 lanes,
 // 4 KB per instruction) and staged in LDS as fp32; rows past the pass are
@@ -119,11 +194,11 @@ __device__ __forceinline__ void attn_store_tile(const KvTileRegs<TL>& r, uint32_
 // chunk = p.chunk, or attn_chunk_for(L) when 0 (the split count then stays
 // within kAttnMaxSplits at every context length). Contexts whose splits hold
 // many passes take attn_decode_long_kernel instead.
-template <int DPL, bool F16KV>
+template <int DPL, bool F16KV, bool ONE>
 __global__ __launch_bounds__(256) void attn_decode_kernel(const int32_t* pos_p, const long long* qkv,
                                                           const float* ssin, const float* rcos, const float* rsin,
                                                           uint32_t shape, uint32_t hh, uint32_t snn, uint32_t chunk_a,
-                                                          AttnParams p) {
+                                                          std::conditional_t<ONE, AttnOneParams, AttnParams> p) {
     // (first-load arguments preloaded; see launch_attn)
     const uint32_t half = (hh >> 16) & 0x7FFFu, H = hh & 0xFFFFu, KVH = shape >> 20;
     const bool use_rope = (hh >> 31) != 0u;
@@ -329,6 +404,10 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const int32_t* pos_p, 
             }
         }
         __syncthreads();                              // the tile is rewritten next pass
+    }
+    if constexpr (ONE) {
+        attn_merge_last<DPL>(p, kvh, split, hd, G, g, acc, m, l, vlane, dv0c, qs);
+        return;
     }
     if (g >= G) return;
     float* part = p.part + (((uint64_t)kvh * p.s_max + split) * G + g) * (hd + 2);

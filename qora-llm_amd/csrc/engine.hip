@@ -182,8 +182,9 @@ struct PreparedGemv {
     void* part_idx = nullptr;
 };
 
-// a counter per query block (16 rows or more) and KV head that the key split's
-// rows hold in two chunks or more; the rows' 128 values, m and l
+// a counter per query block (64 rows or more) and KV head that the key split's
+// rows hold in two chunks or more (qora_hip_attn_decode: one per KV head, up to
+// 128); the rows' 128 values, m and l
 constexpr size_t kPfAttnOneCounts = kPfAttnOneRows / 64 / 2;
 constexpr size_t kPfAttnOneBytes = kPfAttnOneCounts * sizeof(uint32_t) + (size_t)kPfAttnOneRows * (128 + 2) * sizeof(float);
 
@@ -222,8 +223,9 @@ struct qora_hip_ctx {
     uint64_t ws_pf_bytes = 0;
     float* ws_attn_part = nullptr;
     uint64_t ws_attn_part_n = 0;
-    // qora_hip_attn_prefill's key split, made with the context (17 MB; null if that
-    // allocation failed: calls then go unsplit): counters, then the chunks' rows
+    // the attention calls' one-launch splits, made with the context (17 MB; null if
+    // that allocation failed: calls then go unsplit or in two launches): counters,
+    // zero between launches, then qora_hip_attn_prefill's rows
     void* ws_pa = nullptr;
     int32_t* h_pin = nullptr;            // pinned staging: [0] token in, [1] token out, [2] pos
     // The step's argmax, stored by argmax_finish_kernel straight into mapped,
@@ -2089,6 +2091,19 @@ extern "C" int qora_hip_attn_decode(qora_hip_ctx* c, const float* q, const void*
     if (int rc = ensure_attn_ws(c, (uint64_t)KVH * a.s_max * a.groups * (hd + 2))) return rc;
     a.part = c->ws_attn_part;
     const hipStream_t s = pick_stream(c, stream);
+    // One launch where few splits are to be merged, which their last one does:
+    // 16 heads over 4, on one stream and on three, 64 positions 8.5 and 8.5 -> 7.3
+    // and 5.3 us a call, 500 9.1 and 8.3 -> 8.2 and 5.2, 858 (108 splits) 10.6 and
+    // 8.3 -> 10.2 and 5.0; beyond, one block a KV head merges slower than the
+    // combine kernel's block a head (1300 positions on one stream 11.3 -> 12.7).
+    if (c->ws_pa && a.nsg == 1 && (uint64_t)a.s_max * KVH <= 128u && in_order(c, s)) {
+        AttnOneParams one{};
+        static_cast<AttnParams&>(one) = a;
+        one.count = (uint32_t*)c->ws_pa;
+        one.out = out;
+        HIP_TRY(c, launch_attn(a, s, &one));
+        return QORA_HIP_OK;
+    }
     HIP_TRY(c, launch_attn(a, s));
     AttnCombineParams cp{a.part, nullptr, L, H, KVH, hd, a.groups, a.chunk, a.s_max, out};
     HIP_TRY(c, launch_attn_combine(cp, s));

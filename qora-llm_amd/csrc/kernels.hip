@@ -483,7 +483,7 @@ void attn_geometry(uint32_t positions, uint32_t* chunk, uint32_t* s_max) {
     *s_max = std::max<uint32_t>(1, (positions + c - 1) / c);
 }
 
-hipError_t launch_attn(const AttnParams& p, hipStream_t stream) {
+hipError_t launch_attn(const AttnParams& p, hipStream_t stream, const AttnOneParams* one) {
     const dim3 grid(p.s_max, p.KVH);
     const bool lng = p.nsg > 1;
     if (lng && p.kv_f16 && (p.hd == 128 || p.hd == 64) && p.groups <= (uint32_t)kAttnMaxGroups &&
@@ -504,20 +504,26 @@ hipError_t launch_attn(const AttnParams& p, hipStream_t stream) {
     const uint32_t shape = p.hd | (p.groups << 10) | (p.KVH << 20);
     const uint32_t hh = p.H | (p.half << 16) | (p.use_rope ? 0x80000000u : 0u);
     const uint32_t snn = p.ss_n | (p.norm_n << 8);
+#define QORA_ATTN_L(DPL, F16, ONE, PARAMS)                                                               \
+    hipLaunchKernelGGL((attn_decode_kernel<DPL, F16, ONE>), grid, block, 0, stream, p.pos, p.qkv_acc, p.ss_in, \
+                       p.rope_cos, p.rope_sin, shape, hh, snn, p.chunk, PARAMS)
+#define QORA_ATTN_ONE(DPL, F16)                                                                          \
+    do {                                                                                                \
+        if (one) QORA_ATTN_L(DPL, F16, true, *one);                                                      \
+        else QORA_ATTN_L(DPL, F16, false, p);                                                            \
+    } while (0)
 #define QORA_ATTN(DPL)                                                                                   \
     do {                                                                                                \
         if (lng && p.kv_f16) hipLaunchKernelGGL((attn_decode_long_kernel<DPL, true>), grid, block, 0, stream, p); \
         else if (lng) hipLaunchKernelGGL((attn_decode_long_kernel<DPL, false>), grid, block, 0, stream, p); \
-        else if (p.kv_f16)                                                                              \
-            hipLaunchKernelGGL((attn_decode_kernel<DPL, true>), grid, block, 0, stream, p.pos, p.qkv_acc, p.ss_in, \
-                               p.rope_cos, p.rope_sin, shape, hh, snn, p.chunk, p);                    \
-        else                                                                                            \
-            hipLaunchKernelGGL((attn_decode_kernel<DPL, false>), grid, block, 0, stream, p.pos, p.qkv_acc, p.ss_in, \
-                               p.rope_cos, p.rope_sin, shape, hh, snn, p.chunk, p);                    \
+        else if (p.kv_f16) QORA_ATTN_ONE(DPL, true);                                                     \
+        else QORA_ATTN_ONE(DPL, false);                                                                  \
     } while (0)
     if (p.hd <= 64) QORA_ATTN(1);
     else QORA_ATTN(2);
 #undef QORA_ATTN
+#undef QORA_ATTN_ONE
+#undef QORA_ATTN_L
     return hipGetLastError();
 }
 

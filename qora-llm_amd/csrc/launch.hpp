@@ -89,7 +89,7 @@ hipError_t launch_lmhead(uint32_t blocks, const LmHeadParams& p, hipStream_t str
 // Attention split geometry for up to `positions` positions: chunk is a
 // multiple of kAttnSub and s_max = ceil(positions / chunk) <= kAttnMaxSplits.
 void attn_geometry(uint32_t positions, uint32_t* chunk, uint32_t* s_max);
-hipError_t launch_attn(const AttnParams& p, hipStream_t stream);
+hipError_t launch_attn(const AttnParams& p, hipStream_t stream, const AttnOneParams* one = nullptr);   // one: as p (nsg = 1)
 hipError_t launch_attn_combine(const AttnCombineParams& p, hipStream_t stream);
 // Short-context decode: attention of each query head in the o GEMV's
 // prologue (gemv_q4m_attn_kernel). The o plan must be an MFMA plan with one

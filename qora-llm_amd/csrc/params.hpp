@@ -365,6 +365,13 @@ struct AttnParams {
     uint64_t kv_ps, kv_hs;
 };
 
+// attn_decode_kernel in a launch that merges its own splits into out [H*hd]:
+// count holds a counter per KV head, zero between launches
+struct AttnOneParams : AttnParams {
+    uint32_t* count;
+    float* out;
+};
+
 // o projection with the attention of its query head computed in the
 // prologue (gemv_q4m_attn_kernel): the GEMV part (K slice = one head) and
 // the model-mode attention inputs (q|k|v sums, RoPE tables, cache).
