@@ -2142,8 +2142,12 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
     }
     // n % 128 == 0 runs the prefill's GEMM (a Q4 weight packed into the
     // workspace for this call, with its own scales), anything else
-    // pf_gemm_kernel
-    const bool q4 = w->fmt == FMT_Q4, wide = pf_gemm2_supported(K, N), packed = q4 && wide;
+    // pf_gemm_kernel; so does an F16 weight wider than deep or with few tokens,
+    // whose column blocks fill the CUs without it (calls on three streams, 2048 ->
+    // 11008, 100 tokens: 23.9 us against 33.1; 11008 -> 2048, 100 tokens 28.5
+    // against 29.2, 512 tokens 103.4 against 84.1)
+    const bool q4 = w->fmt == FMT_Q4, packed = q4 && pf_gemm2_supported(K, N);
+    const bool wide = packed || (!q4 && pf_gemm2_supported(K, N) && N <= K && T > 128);
     const bool exps = q4 && !wide;
     // scratch: xh, xl [T][k] binary16, xe [T], then the packed weight (wq, sc)
     // or wf [n/32] and the exponent partials, then the split-K partials (each
