@@ -194,13 +194,14 @@ struct qora_hip_ctx {
     int cus = 0;
     std::string err;
     std::vector<DevWeight> weights;
-    long long* ws_acc = nullptr;         // kernel-level fixed-point accumulator
-    uint64_t ws_acc_n = 0;
-    // one-launch GEMV entries: the column tiles' sums behind the accumulator and
-    // their arrival counters ahead of it, all 0 between calls, used only by calls
-    // on the context's own stream outside a capture (one behind the other)
-    long long* ws_sum = nullptr;
+    // one-launch GEMV entries: the column tiles' arrival counters and behind them
+    // their sums, all 0 between calls, used only by calls on the context's own
+    // stream outside a capture (one behind the other); then the kernel-level
+    // fixed-point accumulator, which every call that uses it clears on its stream
     uint32_t* ws_count = nullptr;
+    long long* ws_sum = nullptr;
+    long long* ws_acc = nullptr;
+    uint64_t ws_acc_n = 0;
     uint64_t ws_tiles = 0;
     std::vector<SamplePenalty> pen;      // sampling: the call's penalty list and its look-up table
     std::vector<uint32_t> pen_at;
@@ -273,9 +274,12 @@ int dalloc(qora_hip_ctx* c, size_t bytes, void** p) {
 
 hipStream_t pick_stream(qora_hip_ctx* c, void* s) { return s ? reinterpret_cast<hipStream_t>(s) : c->stream; }
 
-// Grow the kernel-level scratch: one allocation of tile counters, the
-// fixed-point accumulator (n words) and the one-launch GEMVs' sums (a tile has
-// at most 512 columns, the last one partly past n).
+// Grow the kernel-level scratch: one allocation of the one-launch GEMVs' tile
+// counters and sums (a tile has at most 512 columns, the last one partly past
+// n), zero between calls, then the fixed-point accumulator (n words). Only the
+// counters and sums are cleared here: calls on the context's stream alone use
+// them, so the clear on that stream comes first. A call on a caller's stream
+// clears the accumulator there, and nothing orders that stream behind this one.
 int ensure_acc_ws(qora_hip_ctx* c, uint64_t n, uint64_t tiles = 0) {
     if (n <= c->ws_acc_n && tiles <= c->ws_tiles) return QORA_HIP_OK;
     if (c->capturing) return fail(c, QORA_HIP_E_STATE, "scratch must be sized by an eager call before capture");
@@ -283,9 +287,10 @@ int ensure_acc_ws(qora_hip_ctx* c, uint64_t n, uint64_t tiles = 0) {
     const uint64_t nn = std::max<uint64_t>({n, 2 * c->ws_acc_n, 32768});
     const uint64_t nt = std::max<uint64_t>({tiles, 2 * c->ws_tiles, (nn + 255) / 256 + 8});
     const uint64_t cb = nt * kGemvCountStride * sizeof(uint32_t), sw = nn + 512;
+    const uint64_t zeroed = cb + sw * sizeof(long long);
     void* p;
-    if (int rc = dalloc(c, cb + (nn + sw) * sizeof(long long), &p)) return rc;
-    const hipError_t e = hipMemsetAsync(p, 0, cb + (nn + sw) * sizeof(long long), c->stream);
+    if (int rc = dalloc(c, zeroed + nn * sizeof(long long), &p)) return rc;
+    const hipError_t e = hipMemsetAsync(p, 0, zeroed, c->stream);
     if (e != hipSuccess) {
         (void)hipFree(p);
         return fail(c, QORA_HIP_E_DEVICE, std::string("GEMV scratch: ") + hipGetErrorString(e));
@@ -293,9 +298,9 @@ int ensure_acc_ws(qora_hip_ctx* c, uint64_t n, uint64_t tiles = 0) {
     if (c->ws_count) c->ws_old.push_back(c->ws_count);
     c->ws_count = (uint32_t*)p;
     c->ws_tiles = nt;
-    c->ws_acc = (long long*)((uint8_t*)p + cb);
+    c->ws_sum = (long long*)((uint8_t*)p + cb);
+    c->ws_acc = c->ws_sum + sw;
     c->ws_acc_n = nn;
-    c->ws_sum = c->ws_acc + nn;
     return QORA_HIP_OK;
 }
 

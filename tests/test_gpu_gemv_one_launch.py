@@ -96,3 +96,65 @@ def test_captured_calls_match_eager(ctx, pkg):
                 assert np.array_equal(d.get(z, n, np.uint32), want)
         finally:
             ctx.graph_destroy(g)
+
+
+@pytest.mark.parametrize("fmt", ["q4", "f16"])
+@pytest.mark.parametrize("paired", [False, True])
+def test_scratch_grows_on_a_caller_stream_behind_queued_work(pkg, side_stream, fmt, paired):
+    """Calls on a caller's stream while the context's stream has work queued, from
+    the first call of a context on and from one that outgrows its scratch on:
+    nothing that the growth leaves on the context's stream, to run in the middle of
+    them, may touch what they accumulate in."""
+    ctx, hip, calls = pkg.HipContext(0), ctypes.CDLL("libamdhip64.so.7"), 300
+    try:
+        with device(ctx) as d:
+            big = pkg.synth_q4(3, 1, 8192, 8192)
+            bp, bs, bo = d.put(big[0]), d.put(big[1]), d.empty(8192 * 8192 * 4)
+            for k, n in ((2048, 512), (512, 80000)):            # the second outgrows the first's scratch
+                print(f"case growth {fmt} paired={paired} k={k} n={n}", flush=True)
+                w = _weights(pkg, d, fmt, paired, k, n, 17)
+                x, y = d.put(pkg.synth_f32(17, 3, k)), d.empty(n * 4 * calls)
+                ctx.synchronize()
+                for _ in range(16):                             # 256 MB written each: about 1 ms in all
+                    ctx.check(ctx.lib.qora_hip_dequant_q4(ctx.h, bp, bs, 8192, 8192, bo, None))
+                for i in range(calls):                          # 3 ms or more
+                    ctx.check(_call(ctx, pkg, d, fmt, paired, w, x, y + i * n * 4, k, n, side_stream))
+                assert hip.hipDeviceSynchronize() == 0
+                got = d.get(y, (calls, n), np.uint32)
+                want = d.empty(n * 4)
+                ctx.check(_call(ctx, pkg, d, fmt, paired, w, x, want, k, n, None))
+                assert (got == d.get(want, n, np.uint32)).all(), (k, n)
+    finally:
+        ctx.close()
+
+
+def test_outgrown_scratch_serves_the_graphs_that_hold_it(pkg):
+    """A call captured into a graph, then eager calls that outgrow the scratch the
+    graph was recorded with, then its replays: the outgrown scratch is kept."""
+    ctx = pkg.HipContext(0)
+    try:
+        with device(ctx) as d:
+            k, n = 2048, 512
+            w = _weights(pkg, d, "q4", False, k, n, 9)
+            x, y, z = d.put(pkg.synth_f32(9, 3, k)), d.empty(n * 4), d.empty(n * 4)
+            ctx.check(_call(ctx, pkg, d, "q4", False, w, x, y, k, n, None))
+            want = d.get(y, n, np.uint32)
+            ctx.capture_begin()
+            ctx.check(_call(ctx, pkg, d, "q4", False, w, x, z, k, n, None))
+            g = ctx.capture_end()
+            try:
+                for n2 in (80000, 400000):                      # each more than twice the scratch before it
+                    w2 = _weights(pkg, d, "q4", False, 64, n2, 10)
+                    y2 = d.empty(n2 * 4)
+                    ctx.check(_call(ctx, pkg, d, "q4", False, w2, d.put(pkg.synth_f32(9, 4, 64)), y2, 64, n2, None))
+                    hold = d.put(np.full(1 << 20, 0x5A5A5A5A, np.uint32))   # what a freed block would be given to
+                    ctx.h2d(z, np.zeros(n, np.float32))
+                    ctx.graph_launch(g)
+                    ctx.check(_call(ctx, pkg, d, "q4", False, w, x, y, k, n, None))
+                    assert np.array_equal(d.get(z, n, np.uint32), want)
+                    assert np.array_equal(d.get(y, n, np.uint32), want)
+                    assert (d.get(hold, 1 << 20, np.uint32) == 0x5A5A5A5A).all()
+            finally:
+                ctx.graph_destroy(g)
+    finally:
+        ctx.close()
