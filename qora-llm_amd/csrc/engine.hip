@@ -2307,11 +2307,13 @@ int sample_device(qora_hip_ctx* c, const float* logits, uint64_t vocab, const ui
         if (c->smp_rng) (void)hipFree(c->smp_rng);
         c->smp_rng = nullptr;
         c->smp_vocab = 0;
-        // one allocation: state, token and count; candidates; the penalised copy
+        // one allocation: state, token and count; candidates; the penalised copy.
+        // Only the count starts from 0, for calls on the context's stream: a
+        // caller's stream, which writes the other words, is not ordered behind it
         const size_t cb = (size_t)blocks * 64 * 8;
         void* q = nullptr;
         if (int rc = dalloc(c, 256 + cb + (size_t)V * 4, &q)) return rc;
-        const hipError_t e = hipMemsetAsync(q, 0, 256, c->stream);
+        const hipError_t e = hipMemsetAsync((uint8_t*)q + 128, 0, sizeof(uint32_t), c->stream);
         if (e != hipSuccess) {
             (void)hipFree(q);
             return fail(c, QORA_HIP_E_DEVICE, std::string("sampling scratch: ") + hipGetErrorString(e));

@@ -61,3 +61,40 @@ def test_penalty_list_sizes(ctx, pkg, orc, distinct):
             want, b = orc.sample(lg, hist.tolist(), SP["temperature"], SP["top_p"], SP["top_k"],
                                  SP["repetition_penalty"], SP["presence_penalty"], b)
             assert (tok, a) == (want, b)
+
+
+def test_first_calls_on_a_caller_stream_behind_queued_work(pkg, orc):
+    """A context's first sampling calls, and those after its scratch grew, on a
+    caller's stream while the context's stream has about 1 ms of work queued, then
+    one on the context's stream: nothing that the growth leaves on the context's
+    stream may touch the words the draws write."""
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    stream = ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0     # hipStreamNonBlocking
+    ctx = pkg.HipContext(0)
+    params = pkg.SampleParams(**SP)
+    a = b = 0x1234567890ABCDEF
+    try:
+        with device(ctx) as d:
+            w = pkg.synth_q4(3, 1, 8192, 8192)
+            wp, ws, wo = d.put(w[0]), d.put(w[1]), d.empty(8192 * 8192 * 4)
+            for vocab in (5000, 128256):
+                print(f"case sampling growth vocab={vocab}", flush=True)
+                lg = (rng(vocab).standard_normal(vocab) * 3).astype(np.float32)
+                hist = np.arange(0, 300, 7, dtype=np.uint32)
+                dl = d.put(lg)
+                for _ in range(16):
+                    ctx.check(ctx.lib.qora_hip_dequant_q4(ctx.h, wp, ws, 8192, 8192, wo, None))
+                for call in range(60):
+                    s = stream if call < 59 else None
+                    st, tk = ctypes.c_uint64(a), ctypes.c_uint32()
+                    ctx.check(ctx.lib.qora_hip_sample(ctx.h, dl, vocab, hist.ctypes.data, hist.size,
+                                                      ctypes.byref(params), ctypes.byref(st), ctypes.byref(tk), s))
+                    a = st.value
+                    want, b = orc.sample(lg, hist.tolist(), SP["temperature"], SP["top_p"], SP["top_k"],
+                                         SP["repetition_penalty"], SP["presence_penalty"], b)
+                    assert (tk.value, a) == (want, b), call
+    finally:
+        hip.hipDeviceSynchronize()
+        ctx.close()
+        assert hip.hipStreamDestroy(stream) == 0
