@@ -272,6 +272,20 @@ int dalloc(qora_hip_ctx* c, size_t bytes, void** p) {
     return QORA_HIP_OK;
 }
 
+// A stream that is being captured (or cannot say).
+bool stream_capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
+// Kernel-level scratch grows outside captures only, the context's own and one
+// that the caller began on the context's stream: there an allocation's clear
+// would become a node of the graph, and a synchronisation end the capture.
+int scratch_may_grow(qora_hip_ctx* c) {
+    if (!c->capturing && !stream_capturing(c->stream)) return QORA_HIP_OK;
+    return fail(c, QORA_HIP_E_STATE, "scratch must be sized by an eager call before capture");
+}
+
 hipStream_t pick_stream(qora_hip_ctx* c, void* s) { return s ? reinterpret_cast<hipStream_t>(s) : c->stream; }
 
 // Grow the kernel-level scratch: one allocation of the one-launch GEMVs' tile
@@ -282,7 +296,7 @@ hipStream_t pick_stream(qora_hip_ctx* c, void* s) { return s ? reinterpret_cast<
 // clears the accumulator there, and nothing orders that stream behind this one.
 int ensure_acc_ws(qora_hip_ctx* c, uint64_t n, uint64_t tiles = 0) {
     if (n <= c->ws_acc_n && tiles <= c->ws_tiles) return QORA_HIP_OK;
-    if (c->capturing) return fail(c, QORA_HIP_E_STATE, "scratch must be sized by an eager call before capture");
+    if (int rc = scratch_may_grow(c)) return rc;
     // (each growth at least doubles: the outgrown ones together stay below the current)
     const uint64_t nn = std::max<uint64_t>({n, 2 * c->ws_acc_n, 32768});
     const uint64_t nt = std::max<uint64_t>({tiles, 2 * c->ws_tiles, (nn + 255) / 256 + 8});
@@ -306,7 +320,7 @@ int ensure_acc_ws(qora_hip_ctx* c, uint64_t n, uint64_t tiles = 0) {
 
 int ensure_attn_ws(qora_hip_ctx* c, uint64_t part_floats) {
     if (part_floats <= c->ws_attn_part_n) return QORA_HIP_OK;
-    if (c->capturing) return fail(c, QORA_HIP_E_STATE, "scratch must be sized by an eager call before capture");
+    if (int rc = scratch_may_grow(c)) return rc;
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     if (c->ws_attn_part) (void)hipFree(c->ws_attn_part);
     c->ws_attn_part = nullptr;
@@ -320,7 +334,7 @@ int ensure_attn_ws(qora_hip_ctx* c, uint64_t part_floats) {
 
 int ensure_pf_ws(qora_hip_ctx* c, uint64_t bytes) {
     if (bytes <= c->ws_pf_bytes) return QORA_HIP_OK;
-    if (c->capturing) return fail(c, QORA_HIP_E_STATE, "scratch must be sized by an eager call before capture");
+    if (int rc = scratch_may_grow(c)) return rc;
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     if (c->ws_pf) (void)hipFree(c->ws_pf);
     c->ws_pf = nullptr;
@@ -1765,9 +1779,7 @@ int gemv_acc_entry(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, con
 // launches: on the context's own stream, outside a capture, calls run one
 // behind the other; a caller's stream or a captured graph could overlap them.
 bool in_order(qora_hip_ctx* c, hipStream_t s) {
-    if (s != c->stream || c->capturing) return false;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+    return s == c->stream && !c->capturing && !stream_capturing(s);
 }
 
 // y = W x (paired: y = silu(Wg x) * (Wu x)). On the context's stream one

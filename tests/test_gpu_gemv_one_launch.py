@@ -158,3 +158,47 @@ def test_outgrown_scratch_serves_the_graphs_that_hold_it(pkg):
                 ctx.graph_destroy(g)
     finally:
         ctx.close()
+
+
+def test_scratch_does_not_grow_in_a_capture_of_the_caller(pkg):
+    """A caller that captures the context's stream itself, in the mode that allows
+    allocations: calls whose scratch would have to grow are refused and leave no
+    node in the graph; once an eager call has sized it, they are captured, and eager
+    and replayed calls agree."""
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    ctx = pkg.HipContext(0)
+    stream = ctypes.c_void_p(ctx.lib.qora_hip_stream(ctx.h))
+    graph, ex = ctypes.c_void_p(), ctypes.c_void_p()
+    k, n, L = 2048, 512, 100
+    try:
+        with device(ctx) as d:
+            w = _weights(pkg, d, "q4", False, k, n, 9)
+            x, y, z = d.put(pkg.synth_f32(9, 3, k)), d.empty(n * 4), d.empty(n * 4)
+            wid = ctx.upload(pkg.Weight(k=k, n=n, packed=pkg.synth_q4(9, 1, k, n)[0], scales=pkg.synth_q4(9, 1, k, n)[1]))
+            kv = d.put(pkg.synth_f32(9, 4, L * 128))
+            ctx.synchronize()
+            assert hip.hipStreamBeginCapture(stream, 2) == 0          # hipStreamCaptureModeRelaxed
+            assert _call(ctx, pkg, d, "q4", False, w, x, z, k, n, None) == pkg.QORA_HIP_E_STATE
+            assert ctx.lib.qora_hip_gemm(ctx.h, wid, x, z, 1, None) == pkg.QORA_HIP_E_STATE
+            assert ctx.lib.qora_hip_attn_decode(ctx.h, x, kv, kv, 0, L, 1, 1, 128, z, None) == pkg.QORA_HIP_E_STATE
+            assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+            nodes = ctypes.c_size_t(99)
+            assert hip.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0 and nodes.value == 0
+            assert hip.hipGraphDestroy(graph) == 0
+            ctx.check(_call(ctx, pkg, d, "q4", False, w, x, y, k, n, None))
+            want = d.get(y, n, np.uint32)
+            assert hip.hipStreamBeginCapture(stream, 2) == 0
+            ctx.check(_call(ctx, pkg, d, "q4", False, w, x, z, k, n, None))
+            assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+            assert hip.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, 0) == 0
+            for _ in range(3):
+                ctx.h2d(z, np.zeros(n, np.float32))
+                ctx.h2d(y, np.zeros(n, np.float32))
+                assert hip.hipGraphLaunch(ex, stream) == 0
+                ctx.check(_call(ctx, pkg, d, "q4", False, w, x, y, k, n, None))
+                assert np.array_equal(d.get(y, n, np.uint32), want)
+                assert np.array_equal(d.get(z, n, np.uint32), want)
+            ctx.synchronize()
+            assert hip.hipGraphExecDestroy(ex) == 0 and hip.hipGraphDestroy(graph) == 0
+    finally:
+        ctx.close()
