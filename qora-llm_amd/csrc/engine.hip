@@ -297,8 +297,9 @@ hipStream_t pick_stream(qora_hip_ctx* c, void* s) { return s ? reinterpret_cast<
 int ensure_acc_ws(qora_hip_ctx* c, uint64_t n, uint64_t tiles = 0) {
     if (n <= c->ws_acc_n && tiles <= c->ws_tiles) return QORA_HIP_OK;
     if (int rc = scratch_may_grow(c)) return rc;
-    // (each growth at least doubles: the outgrown ones together stay below the current)
-    const uint64_t nn = std::max<uint64_t>({n, 2 * c->ws_acc_n, 32768});
+    // (each growth at least doubles: the outgrown ones together stay below the current;
+    // any eager call sizes it for captured ones of up to 65536 words)
+    const uint64_t nn = std::max<uint64_t>({n, 2 * c->ws_acc_n, 65536});
     const uint64_t nt = std::max<uint64_t>({tiles, 2 * c->ws_tiles, (nn + 255) / 256 + 8});
     const uint64_t cb = nt * kGemvCountStride * sizeof(uint32_t), sw = nn + 512;
     const uint64_t zeroed = cb + sw * sizeof(long long);

@@ -202,3 +202,27 @@ def test_scratch_does_not_grow_in_a_capture_of_the_caller(pkg):
             assert hip.hipGraphExecDestroy(ex) == 0 and hip.hipGraphDestroy(graph) == 0
     finally:
         ctx.close()
+
+
+def test_a_small_eager_call_sizes_captured_ones_up_to_65536_words(pkg):
+    ctx = pkg.HipContext(0)
+    try:
+        with device(ctx) as d:
+            small = _weights(pkg, d, "q4", False, 64, 32, 9)
+            x = d.put(pkg.synth_f32(9, 3, 64))
+            ctx.check(_call(ctx, pkg, d, "q4", False, small, x, d.empty(32 * 4), 64, 32, None))
+            for paired, n in ((False, 65536), (True, 32768)):
+                w = _weights(pkg, d, "q4", paired, 64, n, 11)
+                y, z = d.empty(n * 4), d.empty(n * 4)
+                ctx.capture_begin()
+                rc = _call(ctx, pkg, d, "q4", paired, w, x, z, 64, n, None)
+                g = ctx.capture_end()
+                ctx.check(rc)
+                ctx.check(_call(ctx, pkg, d, "q4", paired, w, x, y, 64, n, None))
+                for _ in range(3):
+                    ctx.h2d(z, np.zeros(n, np.float32))
+                    ctx.graph_launch(g)
+                    assert np.array_equal(d.get(z, n, np.uint32), d.get(y, n, np.uint32)), (paired, n)
+                ctx.graph_destroy(g)
+    finally:
+        ctx.close()
