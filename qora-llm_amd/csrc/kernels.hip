@@ -397,9 +397,11 @@ hipError_t launch_rowdot(int fmt, uint32_t blocks, const RowdotParams& p, hipStr
 }
 
 // The plain Q4 row-dot on the matrix cores, for the widths whose units come in
-// pairs of whole lines: faster than the VALU kernel at every row count measured
-// (1000 x 2048: 5.8 against 7.1 us a call; 4000 x 256: 4.1 / 5.8; 128256 x 512:
-// 9.0 / 12.0).
+// pairs of whole lines. Calls on one stream are faster than on the VALU kernel at
+// every row count measured (1000 x 2048: 6.8 against 7.2 us; 4000 x 256: 4.1 / 5.8;
+// 128256 x 512: 9.8 / 12.1, x 1024 17.6 / 21.1, x 2048 32.0 / 37.0); calls on three
+// streams, from cached weights, within 5% either way (x 1024 15.4 / 14.8, x 2048
+// 31.6 / 34.9).
 bool rowdot_q4m_supported(const RowdotParams& p) {
     return (p.cols == 256 || p.cols == 512 || p.cols == 1024 || p.cols == 2048) && p.x && !p.xacc && !p.gamma &&
            !p.do_argmax && !tuning_env("QORA_HIP_LM_ROWDOT");

@@ -28,6 +28,8 @@
 // lane l < 32: groups 4u + l/16 and 4u + 2 + l/16 of row l % 16.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "gemv_mfma.hpp"
 #include "params.hpp"
@@ -269,30 +271,39 @@ __global__ __launch_bounds__(256) void lmhead_q4m_kernel(LmHeadParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// The same row-dot on the reference layout (qora_hip_gemv_q4_rowdot): y[r] =
-// sum_c x[c] W[r][c], cols = 256 NV. A lane's 16-byte load is one whole scale
-// group of one row, so the contraction of an MFMA pair (even columns, odd
-// columns) is split by group over the lanes' quarters and every A row is used:
+// The row-dot on the reference layout (qora_hip_gemv_q4_rowdot): y[r] =
+// sum_c x[c] W[r][c], cols = 256 NV. x keeps all its fp32 bits: x[c] = M[c] *
+// 2^(E-62), 2^E bounding max |x|, M in eight signed base-256 limbs, exact for
+// every element of at least 2^-39 of the maximum; an x with smaller ones (not
+// zero) is summed in fp32 instead. A lane's 16-byte load is one whole scale group
+// of one row, so the contraction of an MFMA (even columns, then odd ones) is split
+// by group over the lanes' quarters and every A row is used:
 //   A[4 g' + limb][k of quarter g] = limb of x's group where g' == g, else 0
 //   C[4 g + limb][j]: lane (j, g) receives the four limb sums of its own row
-//   and group, one scale each.
+//   and group, one scale each; a second pair takes the upper four limbs.
 // Unit u of a tile of 16 rows: quarter kq holds group 4 u + kq of row l % 16.
 // The next tile's loads go out as a register is used. A byte of low nibbles is
 // 16 (q - 8) after shift, and, xor.
-// What bounds it: the weight stream. 128256 x 2048 (148 MB): 29.6 us, 5.0 TB/s
-// (a large copy's rate), against 32.6 on the VALU (rowdot_kernel: 17 instructions
-// per 8 weights against 5 and a quarter of an MFMA, and a 64-lane sum per row).
-// Two units share each 128-byte line, so the loads are ordinary ones:
-// non-temporal they took 42.8 us (33.4 with a quarter's two groups adjacent).
+// What bounds it: the weight stream. 128256 x 2048 (148 MB): 29.7 us against
+// 33.5 on the VALU in the same run (rowdot_kernel: 17 instructions per 8 weights
+// against 6 and half an MFMA, and a 64-lane sum per row). Four limbs took 29.5, but
+// dropped what lies 31 bits below the maximum: beside an outlier of 1e5 whose weight is 0 the
+// result was off by 1e-4. Three waves a SIMD (launch bounds): with two, 30.8. The
+// fp32 path takes 1.4 to 2 times the VALU kernel's time. Two units share each 128-byte
+// line, so the loads are ordinary ones: non-temporal they took 42.8 us (33.4 with a
+// quarter's two groups adjacent).
 // ---------------------------------------------------------------------------
 template <int NV>
-__global__ __launch_bounds__(256) void rowdot_q4m_kernel(RowdotParams p) {
+__global__ __launch_bounds__(256, 3) void rowdot_q4m_kernel(RowdotParams p) {
     kernarg_warm(p);
     constexpr int NT = 256, NW = 4;
     constexpr int COLS = 256 * NV, G = 8 * NV;
     constexpr int XPT = COLS / NT;
-    __shared__ __align__(16) uint8_t xl[G * 128 + 16];   // [group][even, odd][limb][16], then a zero slot
+    // [unit][even, odd][lower, upper limbs][quarter][limb][16 columns], then a zero
+    // slot; the fp32 path's x [group][33]
+    __shared__ __align__(16) uint8_t xl[G * 256 + 16];
     __shared__ float red[NW];
+    static_assert(sizeof(xl) >= G * 33 * sizeof(float), "x in fp32 fits");
 
     const int t = threadIdx.x;
     const int lane = t & (kWave - 1);
@@ -301,9 +312,9 @@ __global__ __launch_bounds__(256) void rowdot_q4m_kernel(RowdotParams p) {
     const uint32_t tiles = (p.rows + 15u) / 16u, W = gridDim.x * NW;
     uint32_t tile = blockIdx.x * NW + (uint32_t)wave;
 
-    float xv[XPT];
+    float xv[XPT];                                  // columns XPT t ..
 #pragma unroll
-    for (int j = 0; j < XPT; ++j) xv[j] = p.x[t + NT * j];
+    for (int j = 0; j < XPT; ++j) xv[j] = p.x[XPT * t + j];
 
     // a tile's loads (rows and tiles past the end read the last row)
     v4u32 wb[2 * NV];
@@ -326,41 +337,79 @@ __global__ __launch_bounds__(256) void rowdot_q4m_kernel(RowdotParams p) {
 #pragma unroll
     for (int j = 0; j < XPT; ++j) mx = fmaxf(mx, fabsf(xv[j]) <= 3.4028235e38f ? fabsf(xv[j]) : INFINITY);   // (NaN too)
     mx = block_max<NT>(mx, red);
-    if (mx == INFINITY) {
-        // an infinity or NaN in x: no common exponent; every row in fp32, as it was stored
+    const int em = (int)(__float_as_uint(mx) >> 23), ex = em - 126;   // (em 255: an infinity or NaN in x)
+    int rest = em == 255;                           // an element that the limbs cannot hold
+    // the limbs of the thread's even and of its odd columns, a byte each, side by side
+    constexpr int PB = XPT > 1 ? XPT / 2 : 1;
+    using Bytes = std::conditional_t<PB == 4, uint32_t, std::conditional_t<PB == 2, uint16_t, uint8_t>>;
+    uint32_t lb[2][8] = {};
+#pragma unroll
+    for (int j = 0; j < XPT; ++j) {
+        const uint32_t b = __float_as_uint(xv[j]);
+        const int e = (int)((b >> 23) & 0xFFu);
+        const uint32_t mant = (b & 0x7FFFFFu) | (e ? 0x800000u : 0u);
+        const int sh = max(e, 1) - em + 38;         // 38 for the largest (39 where it is subnormal)
+        rest |= mant != 0u && sh < 0;
+        const uint64_t m = (uint64_t)mant << (uint32_t)min(max(sh, 0), 39);
+        const uint64_t k8 = 0x0080808080808080ull;
+        const uint64_t limbs = (((b >> 31) ? 0ull - m : m) + k8) ^ k8;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) lb[j % 2][i] |= (uint32_t)((limbs >> (8 * i)) & 0xFFu) << (8 * (j / 2));
+    }
+    {
+        const uint32_t c = (uint32_t)(XPT * t), g = c / 32u;
+        uint8_t* dst = xl + (g / 4u) * 1024u + (c & 1u) * 512u + (g % 4u) * 64u + (c % 32u) / 2u;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int q = 0; q < (XPT > 1 ? 2 : 1); ++q)
+                *reinterpret_cast<Bytes*>(dst + q * 512 + (i / 4) * 256 + (i % 4) * 16) = (Bytes)lb[q][i];
+    }
+    if (t < 4) *reinterpret_cast<uint32_t*>(xl + G * 256 + t * 4) = 0u;
+    if (__syncthreads_or(rest)) {
+        // no common exponent: fp32, a lane per group (its x in registers), G lanes a row
+        float* xf = reinterpret_cast<float*>(xl);
+#pragma unroll
+        for (int j = 0; j < XPT; ++j) {
+            const uint32_t c = (uint32_t)(XPT * t + j);
+            xf[(c / 32u) * 33u + c % 32u] = xv[j];
+        }
+        __syncthreads();
+        const uint32_t g = (uint32_t)lane % (uint32_t)G;
+        float xr[32];
+#pragma unroll
+        for (int c = 0; c < 32; ++c) xr[c] = xf[g * 33u + c];
+        constexpr uint32_t RI = 64u / G, NB = 16u / RI < 4u ? 16u / RI : 4u;   // rows an instruction, instructions in flight
         for (; tile < tiles; tile += W)
-            for (uint32_t r = tile * 16u; r < min(tile * 16u + 16u, p.rows); ++r) {
-                float a = 0.f;
-                for (uint32_t c = (uint32_t)lane; c < (uint32_t)COLS; c += kWave) {
-                    const uint32_t b = p.w[((uint64_t)r * COLS + c) / 2u];
-                    const float q = (float)((int)((b >> (4u * (c & 1u))) & 0xFu) - 8);
-                    a = fmaf(p.x[c], h2f(p.scales[(uint64_t)r * G + c / 32u]) * q, a);
+            for (uint32_t i = 0; i < 16u; i += NB * RI) {
+                v4u32 w[NB];
+                float s[NB];
+#pragma unroll
+                for (uint32_t n = 0; n < NB; ++n) {
+                    const uint64_t o = (uint64_t)min(tile * 16u + i + n * RI + (uint32_t)lane / (uint32_t)G, p.rows - 1u) * G + g;
+                    w[n] = *reinterpret_cast<const v4u32*>(p.w + o * 16u);
+                    s[n] = h2f(p.scales[o]);
                 }
-                a = wave_sum(a);
-                if (lane == 0) p.y[r] = a;
+#pragma unroll
+                for (uint32_t n = 0; n < NB; ++n) {
+                    const uint32_t r = tile * 16u + i + n * RI + (uint32_t)lane / (uint32_t)G;
+                    float a = 0.f;
+#pragma unroll
+                    for (int c = 0; c < 32; ++c)
+                        a = fmaf(xr[c], s[n] * (float)((int)((w[n][c / 8] >> (4 * (c % 8))) & 0xFu) - 8), a);
+#pragma unroll
+                    for (int o = 1; o < G; o <<= 1) a += __shfl_xor(a, o, kWave);
+                    if (g == 0 && r < p.rows) p.y[r] = a;
+                }
             }
         return;
     }
-    const int ex = mx > 0.f ? (int)((__float_as_uint(mx) >> 23) & 0xFFu) - 126 : 0;
-#pragma unroll
-    for (int j = 0; j < XPT; ++j) {
-        const uint32_t c = (uint32_t)(t + NT * j);
-        const int M = (int)rintf(ldexpf(xv[j], 30 - ex));
-        const uint32_t limbs = (uint32_t)(M + 0x808080) ^ 0x808080u;
-        uint8_t* dst = xl + (c / 32u) * 128u + (c & 1u) * 64u + (c % 32u) / 2u;
-        dst[0] = (uint8_t)(limbs & 0xFFu);
-        dst[16] = (uint8_t)((limbs >> 8) & 0xFFu);
-        dst[32] = (uint8_t)((limbs >> 16) & 0xFFu);
-        dst[48] = (uint8_t)(limbs >> 24);
-    }
-    if (t < 4) *reinterpret_cast<uint32_t*>(xl + G * 128 + t * 4) = 0u;
-    __syncthreads();
 
-    // lanes with li / 4 == kq read their group's limb li % 4, the others the
-    // zero slot (both parities and every unit at a fixed stride from there)
+    // lanes with li / 4 == kq read their group's limbs li % 4 and 4 + li % 4, the
+    // others the zero slot (every unit, parity and half at a fixed stride from there)
     const bool nz = li / 4u == kq;
-    const uint32_t abase = nz ? kq * 128u + (li % 4u) * 16u : (uint32_t)(G * 128);
-    const uint32_t au = nz ? 512u : 0u, ap = nz ? 64u : 0u;
+    const uint32_t abase = nz ? kq * 64u + (li % 4u) * 16u : (uint32_t)(G * 256);
+    const uint32_t au = nz ? 1024u : 0u, ap = nz ? 512u : 0u, ah = nz ? 256u : 0u;
     const v4i32 zero = (v4i32){0, 0, 0, 0};
     for (; tile < tiles; tile += W) {
         uint32_t ao = abase;
@@ -378,6 +427,8 @@ __global__ __launch_bounds__(256) void rowdot_q4m_kernel(RowdotParams p) {
             const uint32_t a = ao + (uint32_t)u * au;
             const v4i32 ae = *reinterpret_cast<const v4i32*>(xl + a);
             const v4i32 ad = *reinterpret_cast<const v4i32*>(xl + a + ap);
+            const v4i32 he = *reinterpret_cast<const v4i32*>(xl + a + ah);
+            const v4i32 hd = *reinterpret_cast<const v4i32*>(xl + a + ap + ah);
             v4i32 be, bo;
 #pragma unroll
             for (int d = 0; d < 4; ++d) {
@@ -385,12 +436,14 @@ __global__ __launch_bounds__(256) void rowdot_q4m_kernel(RowdotParams p) {
                 bo[d] = (int)((w[d] & 0xF0F0F0F0u) ^ 0x80808080u);
             }
             v4i32 c = __builtin_amdgcn_mfma_i32_16x16x64_i8(ae, be, zero, 0, 0, 0);
+            v4i32 h = __builtin_amdgcn_mfma_i32_16x16x64_i8(he, be, zero, 0, 0, 0);
             c = __builtin_amdgcn_mfma_i32_16x16x64_i8(ad, bo, c, 0, 0, 0);
-            acc = fmaf(lm_limb_value(c), h2f(s), acc);
+            h = __builtin_amdgcn_mfma_i32_16x16x64_i8(hd, bo, h, 0, 0, 0);
+            acc = fmaf(fmaf(lm_limb_value(h), 4294967296.0f, lm_limb_value(c)), h2f(s), acc);
         }
         acc = sum_row_slots(acc);
         const uint32_t r = tile * 16u + (uint32_t)lane;
-        if (lane < 16 && r < p.rows) p.y[r] = ldexpf(acc, ex - 34);
+        if (lane < 16 && r < p.rows) p.y[r] = ldexpf(acc, ex - 66);
     }
 }
 

@@ -1,7 +1,8 @@
 """The Q4 row-dot on the matrix cores (widths 256, 512, 1024, 2048) at its edges:
 rows around a tile of 16, inputs spanning 2^-18 .. 2^6, scales with both signs and
-zeros, scales off a 4-byte boundary, and non-finite inputs, against
-float64. The bound is the row-dot tests' own (fp32 sums; x to 30 bits of its maximum)."""
+zeros, scales off a 4-byte boundary, inputs with an outlier, and non-finite
+inputs, against float64. The bound is the row-dot tests' own: fp32 sums of
+products of all 24 bits of x, each output against its own sum of |x w|."""
 import numpy as np
 import pytest
 
@@ -30,9 +31,35 @@ def test_rowdot_edges(ctx, pkg, rows, cols):
             ctx.check(ctx.lib.qora_hip_gemv_q4_rowdot(ctx.h, wd, sd + off, xd, yd, rows, cols, None))
             y = d.get(yd, rows, np.float32)
             assert rel_err(y, truth) <= 1e-5 or np.max(np.abs(truth)) == 0
-            # (x is held to 2^-31 of its largest value: that much of every weight too)
-            bound = 1e-5 * (np.abs(W) @ np.abs(x.astype(np.float64))) + 2.0 ** -30 * np.max(np.abs(x)) * np.abs(W).sum(1)
-            assert np.all(np.abs(y - truth) <= bound + 1e-30)
+            assert elem_err(y, truth, np.abs(W) @ np.abs(x.astype(np.float64))) <= 1e-5
+
+
+@pytest.mark.parametrize("cols", [256, 512, 1024, 2048])
+@pytest.mark.parametrize("outlier", [1e3, 1e5, 1e7, 1e9, 2.0 ** 36, 2.0 ** 45, 1e30, 3e38])
+@pytest.mark.parametrize("unit", [1.0, 2.0 ** -130])
+def test_rowdot_keeps_every_bit_beside_an_outlier(ctx, pkg, cols, outlier, unit):
+    """One large input whose weight is zero in every row: the others count with all
+    their bits, up to the widest spread that the integer sum holds and past it
+    (where x goes through fp32), and with the others subnormal. The row-dot in fp32
+    stays within 1e-6 of the sum of |x w| at any outlier."""
+    print(f"case rowdot outlier cols={cols} {outlier} {unit}", flush=True)
+    rows = 77
+    r = rng(cols)
+    packed, scales = pkg.synth_q4(6, cols, rows, cols)
+    packed = packed.reshape(rows, cols // 2).copy()
+    packed[:, 50] = (packed[:, 50] & 0xF0) | 8                   # column 100
+    x = (r.standard_normal(cols) * unit).astype(np.float32)
+    x[100] = min(outlier * unit, 3e38)
+    W = dequant_np(packed.reshape(-1), scales, rows, cols)
+    assert not W[:, 100].any()
+    with device(ctx) as d:
+        yd = d.empty(rows * 4)
+        ctx.check(ctx.lib.qora_hip_gemv_q4_rowdot(ctx.h, d.put(packed), d.put(scales), d.put(x), yd, rows, cols, None))
+        y = d.get(yd, rows, np.float32)
+    xd = x.astype(np.float64)
+    # (results of subnormal size: fp32's last place there, 2^-149, for each of the sums)
+    err = np.abs(y - W @ xd) - cols * 2.0 ** -149
+    assert np.all(err <= 1e-6 * (np.abs(W) @ np.abs(xd)))
 
 
 def test_rowdot_non_finite_inputs(ctx, pkg):
