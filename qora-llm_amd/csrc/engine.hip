@@ -1783,11 +1783,19 @@ bool in_order(qora_hip_ctx* c, hipStream_t s) {
     return s == c->stream && !c->capturing && !stream_capturing(s);
 }
 
+// Whether two buffers meet. A launch that reads one while another of its
+// workgroups already writes the other needs them apart; the forms in several
+// launches write their output after every read, so calls in place take those.
+bool overlap(const void* a, uint64_t a_bytes, const void* b, uint64_t b_bytes) {
+    const uint64_t x = (uint64_t)a, y = (uint64_t)b;
+    return x < y + b_bytes && y < x + a_bytes;
+}
+
 // y = W x (paired: y = silu(Wg x) * (Wu x)). On the context's stream one
 // launch: the last workgroup of each column tile sums the K slices (2048 ->
 // 512 in Q4: 4.1 us a call against 9.4 for three launches, which the host's
-// ~2.8 us a launch bounds). In a capture or on a caller's stream through the
-// context accumulator (clear, accumulate, convert): the same terms summed in
+// ~2.8 us a launch bounds). In a capture, on a caller's stream, or with y over x
+// through the context accumulator (clear, accumulate, convert): the same terms summed in
 // the same fixed point, so the same bits.
 int gemv_entry(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, const void* w1, const void* s1,
                const float* x, float* y, uint64_t k, uint64_t n, bool paired, void* stream) {
@@ -1796,7 +1804,7 @@ int gemv_entry(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, const v
     if (n == 0 || n > 0x7FFFFFFFull) return fail(c, QORA_HIP_E_INVALID, "GEMV needs 0 < n < 2^31");
     const hipStream_t s = pick_stream(c, stream);
     const uint64_t accn = paired ? 2 * n : n;
-    if (in_order(c, s)) {
+    if (in_order(c, s) && !overlap(x, k * sizeof(float), y, n * sizeof(float))) {
         GemvPlan pl;
         GemvParams p{};
         if (int rc = gemv_prepare_launch(c, fmt, w0, s0, w1, s1, x, k, n, paired, &pl, &p)) return rc;
@@ -2114,7 +2122,9 @@ extern "C" int qora_hip_attn_decode(qora_hip_ctx* c, const float* q, const void*
     // and 5.3 us a call, 500 9.1 and 8.3 -> 8.2 and 5.2, 858 (108 splits) 10.6 and
     // 8.3 -> 10.2 and 5.0; beyond, one block a KV head merges slower than the
     // combine kernel's block a head (1300 positions on one stream 11.3 -> 12.7).
-    if (c->ws_pa && a.nsg == 1 && (uint64_t)a.s_max * KVH <= 128u && in_order(c, s)) {
+    const uint64_t qb = (uint64_t)H * hd * sizeof(float), cb = (uint64_t)L * KVH * hd * (kv_f16 ? 2 : 4);
+    const bool apart = !overlap(out, qb, q, qb) && !overlap(out, qb, kc, cb) && !overlap(out, qb, vc, cb);
+    if (c->ws_pa && a.nsg == 1 && (uint64_t)a.s_max * KVH <= 128u && apart && in_order(c, s)) {
         AttnOneParams one{};
         static_cast<AttnParams&>(one) = a;
         one.count = (uint32_t*)c->ws_pa;
@@ -2138,7 +2148,9 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
     const uint32_t K = (uint32_t)w->k, N = (uint32_t)w->n;
     const hipStream_t s = pick_stream(c, stream);
     auto al = [](uint64_t b) { return (b + 255) & ~uint64_t(255); };
-    if (T <= kPfSmallT) {
+    const PfSmallShape ss = T <= kPfSmallT ? pf_small_shape((uint32_t)T, K, N, c->cus) : PfSmallShape{};
+    // (unsplit it writes y while other blocks read x)
+    if (T <= kPfSmallT && (ss.splits > 1 || !overlap(x, T * K * sizeof(float), y, T * N * sizeof(float)))) {
         // a few tokens: straight from the weight as it was uploaded
         PfSmallParams q{};
         q.x = x;
@@ -2148,11 +2160,10 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
         q.w = (const uint8_t*)w->w;
         q.scales = (const uint16_t*)w->scales;
         q.y = y;
-        const PfSmallShape sh = pf_small_shape(q.T, K, N, c->cus);
-        q.splits = sh.splits;
-        q.kper = sh.kper;
-        if (sh.splits > 1) {
-            if (int rc = ensure_pf_ws(c, al((uint64_t)sh.splits * T * N * 4))) return rc;
+        q.splits = ss.splits;
+        q.kper = ss.kper;
+        if (ss.splits > 1) {
+            if (int rc = ensure_pf_ws(c, al((uint64_t)ss.splits * T * N * 4))) return rc;
             q.part = (float*)c->ws_pf;
         }
         HIP_TRY(c, launch_pf_gemm_small(w->fmt, q, s));
