@@ -66,6 +66,8 @@ struct DevWeight {
     void* w = nullptr;      // packed bytes or f16 words
     void* scales = nullptr; // Q4 only
     bool alive = false;
+    // qora_hip_gemm: the workspace holds what calls of up to this many tokens take
+    uint64_t pf_sized = 0;
 };
 
 struct ModelState {
@@ -341,7 +343,10 @@ int ensure_pf_ws(qora_hip_ctx* c, uint64_t bytes) {
     c->ws_pf = nullptr;
     c->ws_pf_bytes = 0;
     void* p;
-    if (int rc = dalloc(c, bytes, &p)) return rc;
+    if (int rc = dalloc(c, bytes, &p)) {
+        for (DevWeight& w : c->weights) w.pf_sized = 0;
+        return rc;
+    }
     c->ws_pf = p;
     c->ws_pf_bytes = bytes;
     return QORA_HIP_OK;
@@ -2138,23 +2143,105 @@ extern "C" int qora_hip_attn_decode(qora_hip_ctx* c, const float* q, const void*
     return QORA_HIP_OK;
 }
 
-extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, float* y, uint64_t T, void* stream) {
+namespace {
+
+uint64_t al256(uint64_t b) { return (b + 255) & ~uint64_t(255); }
+
+// Scratch of qora_hip_gemm's general kernels: xh, xl [T][k] binary16, xe [T], the
+// packed weight (wq, sc) or wf [n/32] and the exponent partials, the split-K partials.
+struct PfGemmWs {
+    bool wide;                     // the prefill's GEMM (pf_gemm2_kernel), else pf_gemm_kernel
+    PfGemmShape sh;
+    PfGemm2Shape s2;
+    uint32_t splits;
+    uint64_t bx, be, bf, bs, bq, bc, bytes;
+};
+
+PfGemmWs pf_gemm_ws(int fmt, uint32_t T, uint32_t K, uint32_t N, bool wide, int cus) {
+    PfGemmWs g{};
+    g.wide = wide;
+    const bool q4 = fmt == FMT_Q4;
+    if (wide) g.s2 = pf_gemm2_shape(T, K, N, cus);
+    else g.sh = pf_gemm_shape(T, K, N, cus);
+    g.splits = wide ? g.s2.splits : g.sh.splits;
+    g.bx = al256((uint64_t)T * K * 2);
+    g.be = al256((uint64_t)T * 4);
+    g.bf = q4 && !wide ? al256(N / 32 + 1) : 0;
+    g.bs = q4 && !wide ? al256(pf_weight_exp_scratch(K, N / 32)) : 0;
+    g.bq = q4 && wide ? al256((uint64_t)K * N / 2) : 0;
+    g.bc = q4 && wide ? al256((uint64_t)K * N / 16) : 0;
+    g.bytes = 2 * g.bx + g.be + g.bf + g.bs + g.bq + g.bc + (g.splits > 1 ? al256((uint64_t)g.splits * T * N * 4) : 0);
+    return g;
+}
+
+uint64_t pf_small_bytes(const PfSmallShape& sh, uint32_t T, uint32_t N) {
+    return sh.splits > 1 ? al256((uint64_t)sh.splits * T * N * 4) : 0;
+}
+
+// The most that any kernel of a GEMM of T tokens or fewer takes (more tiles of 64
+// tokens mean fewer K splits, so fewer tokens can take more; from 64 tiles on
+// nothing is split that far).
+uint64_t pf_gemm_reserve(int fmt, uint32_t T, uint32_t K, uint32_t N, int cus) {
+    uint64_t b = 0;
+    for (uint32_t t : {16u, 32u, kPfSmallT}) {     // (the slices' length and the limit change there)
+        const uint32_t u = std::min(t, T);
+        b = std::max(b, std::min(pf_small_bytes(pf_small_shape(u, K, N, cus), u, N), pf_small_most(fmt, u, N, cus)));
+    }
+    const uint32_t tiles = std::min(64u, (T + 63u) / 64u);
+    for (uint32_t m = 1; m <= tiles; ++m) {
+        const uint32_t u = m == tiles ? T : 64u * m;
+        if (pf_gemm2_supported(K, N)) b = std::max(b, pf_gemm_ws(fmt, u, K, N, true, cus).bytes);
+        if (fmt != FMT_Q4 || !pf_gemm2_supported(K, N)) b = std::max(b, pf_gemm_ws(fmt, u, K, N, false, cus).bytes);
+    }
+    return b;
+}
+
+}  // namespace
+
+extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, float* y, uint64_t rows, void* stream) {
     if (!c) return QORA_HIP_E_INVALID;
     if (!x || !y) return fail(c, QORA_HIP_E_INVALID, "null argument");
-    const DevWeight* w = get_weight(c, wid);
-    if (!w) return fail(c, QORA_HIP_E_INVALID, "unknown weight id");
-    if (T == 0 || T > 0x7FFFFFFFull) return fail(c, QORA_HIP_E_INVALID, "bad row count");
+    if (!get_weight(c, wid)) return fail(c, QORA_HIP_E_INVALID, "unknown weight id");
+    DevWeight* w = &c->weights[wid];
+    if (rows == 0 || rows > 0x7FFFFFFFull) return fail(c, QORA_HIP_E_INVALID, "bad row count");
     if (!pf_gemm_supported((uint32_t)w->k, (uint32_t)w->n)) return fail(c, QORA_HIP_E_INVALID, "k must be a multiple of 32");
-    const uint32_t K = (uint32_t)w->k, N = (uint32_t)w->n;
+    const uint32_t K = (uint32_t)w->k, N = (uint32_t)w->n, T = (uint32_t)rows;
     const hipStream_t s = pick_stream(c, stream);
-    auto al = [](uint64_t b) { return (b + 255) & ~uint64_t(255); };
-    const PfSmallShape ss = T <= kPfSmallT ? pf_small_shape((uint32_t)T, K, N, c->cus) : PfSmallShape{};
-    // (unsplit it writes y while other blocks read x)
-    if (T <= kPfSmallT && (ss.splits > 1 || !overlap(x, T * K * sizeof(float), y, T * N * sizeof(float)))) {
-        // a few tokens: straight from the weight as it was uploaded
+    const bool q4 = w->fmt == FMT_Q4;
+    // The general kernels: n % 128 == 0 runs the prefill's GEMM (a Q4 weight packed
+    // into the workspace for this call, with its own scales), anything else
+    // pf_gemm_kernel; so does an F16 weight wider than deep or with few tokens,
+    // whose column blocks fill the CUs without it (calls on three streams, 2048 ->
+    // 11008, 100 tokens: 23.9 us against 33.1; 11008 -> 2048, 100 tokens 28.5
+    // against 29.2, 512 tokens 103.4 against 84.1)
+    const bool wide = pf_gemm2_supported(K, N) && (q4 || (N <= K && T > 128));
+    // A few tokens go straight from the weight as it was uploaded, where the slices'
+    // partial sums are few enough; not in place when unsplit, since it then
+    // writes y while other blocks read x.
+    const PfSmallShape ss = T <= kPfSmallT ? pf_small_shape(T, K, N, c->cus) : PfSmallShape{};
+    const uint64_t sb = pf_small_bytes(ss, T, N);
+    bool small = T <= kPfSmallT && ss.splits <= 65535u && sb <= pf_small_most(w->fmt, T, N, c->cus) &&
+                 (ss.splits > 1 || !overlap(x, (uint64_t)T * K * 4, y, (uint64_t)T * N * 4));
+    PfGemmWs g{};
+    if (!small) g = pf_gemm_ws(w->fmt, T, K, N, wide, c->cus);
+    // An eager call sizes the workspace for captured ones of its weight with as many
+    // tokens or fewer. A capture in a workspace that other weights' calls sized takes
+    // the kernel whose scratch it holds.
+    if (T > w->pf_sized && scratch_may_grow(c) == QORA_HIP_OK &&
+        ensure_pf_ws(c, pf_gemm_reserve(w->fmt, T, K, N, c->cus)) == QORA_HIP_OK)
+        w->pf_sized = T;
+    uint64_t need = small ? sb : g.bytes;
+    if (need > c->ws_pf_bytes && scratch_may_grow(c) != QORA_HIP_OK) {
+        g = pf_gemm_ws(w->fmt, T, K, N, wide, c->cus);
+        if (g.bytes > c->ws_pf_bytes && wide && !q4) g = pf_gemm_ws(w->fmt, T, K, N, false, c->cus);
+        small = false;
+        need = g.bytes;
+    }
+    if (int rc = ensure_pf_ws(c, need)) return rc;
+    if (small) {
         PfSmallParams q{};
         q.x = x;
-        q.T = (uint32_t)T;
+        q.T = T;
         q.k = K;
         q.n = N;
         q.w = (const uint8_t*)w->w;
@@ -2162,82 +2249,59 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
         q.y = y;
         q.splits = ss.splits;
         q.kper = ss.kper;
-        if (ss.splits > 1) {
-            if (int rc = ensure_pf_ws(c, al((uint64_t)ss.splits * T * N * 4))) return rc;
-            q.part = (float*)c->ws_pf;
-        }
+        q.part = ss.splits > 1 ? (float*)c->ws_pf : nullptr;
         HIP_TRY(c, launch_pf_gemm_small(w->fmt, q, s));
         return QORA_HIP_OK;
     }
-    // n % 128 == 0 runs the prefill's GEMM (a Q4 weight packed into the
-    // workspace for this call, with its own scales), anything else
-    // pf_gemm_kernel; so does an F16 weight wider than deep or with few tokens,
-    // whose column blocks fill the CUs without it (calls on three streams, 2048 ->
-    // 11008, 100 tokens: 23.9 us against 33.1; 11008 -> 2048, 100 tokens 28.5
-    // against 29.2, 512 tokens 103.4 against 84.1)
-    const bool q4 = w->fmt == FMT_Q4, packed = q4 && pf_gemm2_supported(K, N);
-    const bool wide = packed || (!q4 && pf_gemm2_supported(K, N) && N <= K && T > 128);
-    const bool exps = q4 && !wide;
-    // scratch: xh, xl [T][k] binary16, xe [T], then the packed weight (wq, sc)
-    // or wf [n/32] and the exponent partials, then the split-K partials (each
-    // part 256-byte aligned)
-    const uint64_t bx = al(T * K * 2), be = al(T * 4), bf = exps ? al(N / 32 + 1) : 0;
-    const uint64_t bs = exps ? al(pf_weight_exp_scratch(K, N / 32)) : 0;
-    const uint64_t bq = packed ? al((uint64_t)K * N / 2) : 0, bc = packed ? al((uint64_t)K * N / 16) : 0;
-    const PfGemmShape sh = pf_gemm_shape((uint32_t)T, K, N, c->cus);
-    const PfGemm2Shape s2 = wide ? pf_gemm2_shape((uint32_t)T, K, N, c->cus) : PfGemm2Shape{};
-    const uint32_t splits = wide ? s2.splits : sh.splits;
-    const uint64_t bp = splits > 1 ? al((uint64_t)splits * T * N * 4) : 0;
-    if (int rc = ensure_pf_ws(c, 2 * bx + be + bf + bs + bq + bc + bp)) return rc;
     uint8_t* base = (uint8_t*)c->ws_pf;
-    uint8_t* wq = base + 2 * bx + be + bf + bs;
-    float* part = splits > 1 ? (float*)(wq + bq + bc) : nullptr;
+    uint8_t* wq = base + 2 * g.bx + g.be + g.bf + g.bs;
+    float* part = g.splits > 1 ? (float*)(wq + g.bq + g.bc) : nullptr;
     PrefillRowParams r{};
     r.x = const_cast<float*>(x);
     r.n = K;
     r.xh = (uint16_t*)base;
-    r.xl = (uint16_t*)(base + bx);
-    r.xe = (int32_t*)(base + 2 * bx);
-    if (wide) {
-        if (q4) HIP_TRY(c, launch_pf_gemm_prep(x, (uint32_t)T, r.xh, r.xl, r.xe, (const uint8_t*)w->w, (const uint16_t*)w->scales,
-                                       K, N, (uint2*)wq, (uint16_t*)(wq + bq), s));
-        else HIP_TRY(c, launch_pf_rows(PF_ROW_SPLIT, r, (uint32_t)T, s));
+    r.xl = (uint16_t*)(base + g.bx);
+    r.xe = (int32_t*)(base + 2 * g.bx);
+    if (g.wide) {
+        if (q4) HIP_TRY(c, launch_pf_gemm_prep(x, T, r.xh, r.xl, r.xe, (const uint8_t*)w->w, (const uint16_t*)w->scales,
+                                               K, N, (uint2*)wq, (uint16_t*)(wq + g.bq), s));
+        else HIP_TRY(c, launch_pf_rows(PF_ROW_SPLIT, r, T, s));
         PfGemm2Params h{};
         h.xh = r.xh;
         h.xl = r.xl;
         h.xe = r.xe;
-        h.T = (uint32_t)T;
+        h.T = T;
         h.k = K;
         h.nseg = 1;
         h.ntot = N;
-        h.seg[0] = PfGemm2Seg{(const uint2*)(q4 ? wq : w->w), (const uint16_t*)(wq + bq), nullptr, N, 0, y, N, 0};
-        h.splits = s2.splits;
-        h.kper = s2.kper;
+        h.seg[0] = PfGemm2Seg{(const uint2*)(q4 ? wq : w->w), (const uint16_t*)(wq + g.bq), nullptr, N, 0, y, N, 0};
+        h.splits = g.s2.splits;
+        h.kper = g.s2.kper;
         h.part = part;
-        HIP_TRY(c, launch_pf_gemm2(s2.bm, h, s, true, q4 ? PF_W_RAW : PF_W_F16));
+        HIP_TRY(c, launch_pf_gemm2(g.s2.bm, h, s, true, q4 ? PF_W_RAW : PF_W_F16));
         return QORA_HIP_OK;
     }
-    HIP_TRY(c, launch_pf_rows(PF_ROW_SPLIT, r, (uint32_t)T, s));
-    int8_t* wf = (int8_t*)(base + 2 * bx + be);
-    if (exps)
-        HIP_TRY(c, launch_pf_weight_exp((const uint16_t*)w->scales, K, N / 32, wf, (uint32_t*)(base + 2 * bx + be + bf), s));
-    PrefillGemmParams g{};
-    g.xh = r.xh;
-    g.xl = r.xl;
-    g.xe = r.xe;
-    g.T = (uint32_t)T;
-    g.k = K;
-    g.n = N;
-    g.w = (const uint8_t*)w->w;
-    g.scales = (const uint16_t*)w->scales;
-    g.wf = exps ? wf : nullptr;
-    g.y = y;
-    g.ldy = N;
-    g.nt = sh.nt;
-    g.splits = sh.splits;
-    g.kper = sh.kper;
-    g.part = part;
-    HIP_TRY(c, launch_pf_gemm(w->fmt, g, s));
+    HIP_TRY(c, launch_pf_rows(PF_ROW_SPLIT, r, T, s));
+    int8_t* wf = (int8_t*)(base + 2 * g.bx + g.be);
+    if (q4)
+        HIP_TRY(c, launch_pf_weight_exp((const uint16_t*)w->scales, K, N / 32, wf, (uint32_t*)(base + 2 * g.bx + g.be + g.bf), s));
+    PrefillGemmParams h{};
+    h.xh = r.xh;
+    h.xl = r.xl;
+    h.xe = r.xe;
+    h.T = T;
+    h.k = K;
+    h.n = N;
+    h.w = (const uint8_t*)w->w;
+    h.scales = (const uint16_t*)w->scales;
+    h.wf = q4 ? wf : nullptr;
+    h.y = y;
+    h.ldy = N;
+    h.nt = g.sh.nt;
+    h.splits = g.sh.splits;
+    h.kper = g.sh.kper;
+    h.part = part;
+    HIP_TRY(c, launch_pf_gemm(w->fmt, h, s));
     return QORA_HIP_OK;
 }
 

@@ -782,6 +782,27 @@ PfSmallShape pf_small_shape(uint32_t T, uint32_t k, uint32_t n, int cus) {
     return sh;
 }
 
+// The most bytes of partial sums for which pf_gemm_small_kernel is taken: it writes
+// and reads them for slices as short as its LDS needs, where the general kernels
+// read x again instead. Calls on one and on three streams, 64 tokens unless said,
+// against the general path:
+//   up to 16 tokens they are an eighth of the weight's elements: faster up to a
+//   column block per CU (F16 11008 -> 8192 60 -> 45 us and 46 -> 37; 4096 -> 32768
+//   55 -> 57).
+//   Q4, whose general path packs the weight first: 16 MiB (1024 -> 32768, 33 tokens,
+//   16.5 MiB: 49 -> 36 and 26 -> 30), 36 while there are fewer column blocks than half
+//   the CUs, where the general path splits K as well (11008 -> 2048, 21.5: 80 -> 38 and
+//   36 -> 22; 8192 -> 11008, 88: 111 -> 100 and 74 -> 88).
+//   F16: 4 MiB (2048 -> 11008, 33 tokens, 11: 24 -> 28 and 15 -> 18), more as the column
+//   blocks fall below half the CUs (11008 -> 2048, 21.5: 49 -> 35 and 26 -> 20; 8192 -> 4096,
+//   32: 45 -> 39 and 30 -> 34).
+uint64_t pf_small_most(int fmt, uint32_t T, uint32_t n, int cus) {
+    const uint64_t MB = 1ull << 20, blocks = (n + 127u) / 128u, cu = (uint64_t)std::max(1, cus);
+    if (fmt == FMT_Q4) return T <= 16u ? ~0ull : (2 * blocks < cu ? 36 : 16) * MB;
+    if (T <= 16u && blocks < cu) return ~0ull;
+    return std::max(4 * MB, 2 * cu * MB / blocks);
+}
+
 hipError_t launch_pf_gemm_small(int fmt, const PfSmallParams& p, hipStream_t stream) {
     if (p.T == 0 || p.T > kPfSmallT || !pf_gemm_supported(p.k, p.n) || p.n % 32 != 0 || p.kper % 32 != 0 || p.kper == 0 ||
         p.kper > (p.T > 32u ? 256u : 512u) || (uint64_t)p.splits * p.kper < p.k ||

@@ -151,6 +151,8 @@ struct PfSmallShape {
     uint32_t splits, kper;
 };
 PfSmallShape pf_small_shape(uint32_t T, uint32_t k, uint32_t n, int cus);
+// the most bytes of partial sums (splits * T * n floats) for which it is the kernel to take
+uint64_t pf_small_most(int fmt, uint32_t T, uint32_t n, int cus);
 hipError_t launch_pf_gemm_small(int fmt, const PfSmallParams& p, hipStream_t stream);
 hipError_t launch_pf_rope_cache(const PrefillAttnParams& p, hipStream_t stream);
 hipError_t launch_pf_attn(const PrefillAttnParams& p, hipStream_t stream);

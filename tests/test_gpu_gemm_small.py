@@ -100,3 +100,85 @@ def test_gemm_f16_wide_vs_truth(ctx, pkg, T, k, n):
     assert rel_err(got, truth) <= TRUTH_TOL
     assert elem_err(got, truth, np.abs(x.astype(np.float64)) @ np.abs(W)) <= TRUTH_TOL
     ctx.lib.qora_hip_release_weight(ctx.h, wid)
+
+
+def _captured(ctx, wid, x, y, T):
+    ctx.capture_begin()
+    rc = ctx.lib.qora_hip_gemm(ctx.h, wid, x, y, T, None)
+    g = ctx.capture_end()
+    ctx.check(rc)
+    return g
+
+
+@pytest.mark.parametrize("fmt,k,n", [("q4", 11008, 2048), ("f16", 11008, 2048), ("q4", 2048, 11008), ("f16", 2048, 11008),
+                                     ("q4", 1024, 160), ("f16", 1024, 160)])
+@pytest.mark.parametrize("eager", [64, 100, 200])
+def test_an_eager_gemm_sizes_captured_ones_of_fewer_tokens(pkg, fmt, k, n, eager):
+    """Once an eager call of a weight has run, calls with as many tokens or fewer
+    are captured; their replays give the eager calls' bits."""
+    ctx = pkg.HipContext(0)
+    wt, _ = _weight(pkg, fmt, k, n, 3, None)
+    try:
+        wid = ctx.upload(wt)
+        x = rng(4).standard_normal((eager, k)).astype(np.float32)
+        with device(ctx) as d:
+            xd, y, z = d.put(x), d.empty(eager * n * 4), d.empty(eager * n * 4)
+            ctx.check(ctx.lib.qora_hip_gemm(ctx.h, wid, xd, y, eager, None))
+            for T in (eager, 130, 65, 64, 63, 33, 32, 17, 16, 1):
+                if T > eager:
+                    continue
+                print(f"case captured gemm {fmt} {k} {n} eager={eager} T={T}", flush=True)
+                g = _captured(ctx, wid, xd, z, T)
+                for _ in range(3):
+                    ctx.h2d(z, np.zeros((T, n), np.float32))
+                    ctx.graph_launch(g)
+                    ctx.check(ctx.lib.qora_hip_gemm(ctx.h, wid, xd, y, T, None))
+                    assert np.array_equal(d.get(z, (T, n), np.uint32), d.get(y, (T, n), np.uint32)), T
+                ctx.graph_destroy(g)
+    finally:
+        ctx.close()
+
+
+def test_a_captured_gemm_takes_what_another_weights_call_sized(pkg):
+    """Scratch sized by another weight's call, between what the general path and the
+    few-token kernel need: captured on the former."""
+    ctx = pkg.HipContext(0)
+    k, n, T = 11008, 2048, 64                    # 22.5 MB of partial sums; 19.9 MB on the general path
+    wt, W = _weight(pkg, "f16", k, n, 3, None)
+    x = rng(4).standard_normal((T, k)).astype(np.float32)
+    try:
+        other = ctx.upload(_weight(pkg, "f16", 45056, 32, 5, None)[0])
+        wid = ctx.upload(wt)
+        with device(ctx) as d:
+            xo = d.put(np.zeros((100, 45056), np.float32))
+            ctx.check(ctx.lib.qora_hip_gemm(ctx.h, other, xo, d.empty(100 * 32 * 4), 100, None))   # 20.3 MB
+            xd, z = d.put(x), d.empty(T * n * 4)
+            g = _captured(ctx, wid, xd, z, T)
+            for _ in range(2):
+                ctx.h2d(z, np.zeros((T, n), np.float32))
+                ctx.graph_launch(g)
+                got = d.get(z, (T, n), np.float32)
+                assert elem_err(got, x.astype(np.float64) @ W, np.abs(x.astype(np.float64)) @ np.abs(W)) <= TRUTH_TOL
+            ctx.graph_destroy(g)
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("fmt", ["q4", "f16"])
+@pytest.mark.parametrize("T,k,n", [(33, 2048, 11008), (64, 4096, 8192), (17, 4096, 32768), (16, 4096, 32768), (64, 11008, 2048),
+                                   (64, 8192, 11008)])
+def test_gemm_few_tokens_on_both_sides_of_the_partial_sum_limit(ctx, pkg, fmt, T, k, n):
+    """Wide and deep weights: the few-token kernel below the limit on its partial
+    sums, the general path above (each format has cases on either side)."""
+    wt, W = _weight(pkg, fmt, k, n, 6, None)
+    wid = ctx.upload(wt)
+    x = rng(T).standard_normal((T, k)).astype(np.float32)
+    cols = np.r_[0:64, n // 2:n // 2 + 64, n - 64:n]
+    with device(ctx) as d:
+        y = d.empty(T * n * 4)
+        ctx.check(ctx.lib.qora_hip_gemm(ctx.h, wid, d.put(x), y, T, None))
+        got = d.get(y, (T, n), np.float32)
+    Wc = W[:, cols]
+    assert np.isfinite(got).all()
+    assert elem_err(got[:, cols], x.astype(np.float64) @ Wc, np.abs(x.astype(np.float64)) @ np.abs(Wc)) <= TRUTH_TOL
+    ctx.lib.qora_hip_release_weight(ctx.h, wid)
