@@ -1732,7 +1732,8 @@ namespace {
 // reference layout; nothing is launched, so a refused call leaves the device
 // untouched.
 int gemv_prepare_launch(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, const void* w1, const void* s1,
-                        const float* x, uint64_t k, uint64_t n, bool paired, GemvPlan* plan, GemvParams* params) {
+                        const float* x, uint64_t k, uint64_t n, bool paired, GemvPlan* plan, GemvParams* params,
+                        bool sums = false) {
     if (!w0 || !x || (fmt == FMT_Q4 && !s0) || (paired && (!w1 || (fmt == FMT_Q4 && !s1))))
         return fail(c, QORA_HIP_E_INVALID, "null argument");
     if (k == 0 || n == 0 || n % 32 != 0 || k > 0xFFFFFFFFull || n / 32 > 0xFFFFFFFFull)
@@ -1740,7 +1741,7 @@ int gemv_prepare_launch(qora_hip_ctx* c, int fmt, const void* w0, const void* s0
     const uint32_t G = (uint32_t)(n / 32);
     const uint32_t groups[2] = {G, G};
     GemvPlan pl;
-    if (!plan_gemv(fmt, (uint32_t)k, groups, paired ? 2 : 1, paired, c->cus, &pl))
+    if (!plan_gemv(fmt, (uint32_t)k, groups, paired ? 2 : 1, paired, c->cus, &pl, 1, sums))
         return fail(c, QORA_HIP_E_INVALID, "unsupported GEMV shape");
     GemvParams p{};
     p.seg[0] = GemvSeg{(const uint8_t*)w0, (const uint16_t*)s0, G, 0, 0, 0};
@@ -1762,10 +1763,10 @@ int gemv_prepare_launch(qora_hip_ctx* c, int fmt, const void* w0, const void* s0
 // The same for acc[0:n] (+ acc[n:2n] when paired) += W x.
 int gemv_acc_prepare(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, const void* w1, const void* s1,
                      const float* x, long long* acc, uint64_t k, uint64_t n, bool paired, GemvPlan* plan,
-                     GemvParams* params) {
+                     GemvParams* params, bool sums = false) {
     if (!c) return QORA_HIP_E_INVALID;
     if (!acc) return fail(c, QORA_HIP_E_INVALID, "null argument");
-    if (int rc = gemv_prepare_launch(c, fmt, w0, s0, w1, s1, x, k, n, paired, plan, params)) return rc;
+    if (int rc = gemv_prepare_launch(c, fmt, w0, s0, w1, s1, x, k, n, paired, plan, params, sums)) return rc;
     params->acc = acc;
     return QORA_HIP_OK;
 }
@@ -1773,10 +1774,10 @@ int gemv_acc_prepare(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, c
 // acc[0:n] (+ acc[n:2n] when paired) += W x, one launch of the model's GEMV
 // kernel with the plain-vector prologue.
 int gemv_acc_entry(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, const void* w1, const void* s1,
-                   const float* x, long long* acc, uint64_t k, uint64_t n, bool paired, void* stream) {
+                   const float* x, long long* acc, uint64_t k, uint64_t n, bool paired, void* stream, bool sums = false) {
     GemvPlan pl;
     GemvParams p{};
-    if (int rc = gemv_acc_prepare(c, fmt, w0, s0, w1, s1, x, acc, k, n, paired, &pl, &p)) return rc;
+    if (int rc = gemv_acc_prepare(c, fmt, w0, s0, w1, s1, x, acc, k, n, paired, &pl, &p, sums)) return rc;
     HIP_TRY(c, launch_gemv(fmt, pl, p, pick_stream(c, stream)));
     return QORA_HIP_OK;
 }
@@ -1894,13 +1895,13 @@ extern "C" int qora_hip_gate_up_f16(qora_hip_ctx* c, const void* gw, const void*
 
 extern "C" int qora_hip_gemv_q4_accumulate(qora_hip_ctx* c, const void* packed, const void* scales,
                                            const float* x, long long* acc, uint64_t k, uint64_t n, void* stream) {
-    return gemv_acc_entry(c, FMT_Q4, packed, scales, nullptr, nullptr, x, acc, k, n, false, stream);
+    return gemv_acc_entry(c, FMT_Q4, packed, scales, nullptr, nullptr, x, acc, k, n, false, stream, true);
 }
 
 extern "C" int qora_hip_gate_up_q4_accumulate(qora_hip_ctx* c, const void* gp, const void* gs, const void* up,
                                               const void* us, const float* x, long long* acc, uint64_t k,
                                               uint64_t n, void* stream) {
-    return gemv_acc_entry(c, FMT_Q4, gp, gs, up, us, x, acc, k, n, true, stream);
+    return gemv_acc_entry(c, FMT_Q4, gp, gs, up, us, x, acc, k, n, true, stream, true);
 }
 
 extern "C" int qora_hip_gemv_prepare(qora_hip_ctx* c, uint32_t wid, uint32_t wid_up, int paired, uint32_t* gemv_id) {

@@ -28,17 +28,35 @@ static int env_int(const char* name, int dflt) {
 }
 
 // Rows a lane loads at a time in gemv_kernel: four (2048 -> 2048 in F16 4.1
-// against 4.4 us with two at a time).
-static int plan_batch(int rpl) { return std::min(rpl, 4); }
+// against 4.4 us with two at a time), and all eight of a Q4 slice that has eight
+// (11008 -> 2048 7.7 -> 7.1 us, 2048 -> 2 x 11008 11.9 -> 11.5; sixteen in eights
+// instead of fours 1024 -> 2 x 32768 14.6 -> 16.5).
+static int plan_batch(int fmt, int rpl) { return fmt == FMT_Q4 && rpl == 8 ? 8 : std::min(rpl, 4); }
 
+// Column tile and K slice of gemv_kernel. Times are calls on one stream / on three.
+// Tile: 8 groups, and 16 for a Q4 matrix (both of a pair) of 2^20 groups, 16 MB of
+// nibbles, or more: a row of a tile is then 256 bytes (128 of each of a pair, where 8
+// groups read half a line), which pays once the stream and not the latency bounds the
+// call. 4096 -> 2 x 4096 11.7 / 8.1 -> 7.8 / 6.7 us, 11008 -> 11008 22.4 / 17.0 -> 20.2 / 14.3,
+// 2048 -> 128256 41.3 / 39 -> 34.8 / 30.6; below, 4096 -> 4096 (2^19) 6.0 against 7.2, 2048
+// -> 2 x 2048 (2^18) 5.4 against 6.3.
+// Rows: 128 (64 where K is short, 256 for a long Q4 one): enough workgroups without
+// more than the hand-over or the atomics bear. Calls of the one-launch entry, rows
+// 64 / 128 / 256: 512 -> 512 Q4 5.0 / 5.1 / 5.5 us, 2048 -> 512 5.3 / 4.9 / 5.5, 11008 -> 2048
+// 8.2 / 8.1 / 7.5; sums left in the accumulator have no hand-over, and keep 128 there (5.6
+// against 6.5). The decode step's F16 11008 -> 2048 9.9 / 9.7 / 10.7 (gt 8), its gate|up
+// pair 18.3 / 18.4 / 19.0. With 16 groups 256 where 128 would give every CU four
+// workgroups or more (2048 -> 128256 35.9 / 32.8 -> 34.9 / 30.6; 2048 -> 2 x 11008, 688 of
+// them, 11.8 against 12.2).
 bool plan_gemv(int fmt, uint32_t k, const uint32_t* seg_groups, int nseg, bool paired, int cus,
-               GemvPlan* plan, uint32_t row_align) {
+               GemvPlan* plan, uint32_t row_align, bool sums) {
     if (k == 0 || nseg < 1 || nseg > 3 || row_align == 0) return false;
     if (paired && (nseg != 2 || seg_groups[0] != seg_groups[1])) return false;
     GemvPlan pl;
     uint64_t groups = 0;
     for (int i = 0; i < nseg; ++i) groups += seg_groups[i];
-    pl.gt = (paired && fmt == FMT_Q4 && groups >= 512) ? 16 : 8;
+    const bool q4 = fmt == FMT_Q4;
+    pl.gt = q4 && k * groups >= (1ull << 20) ? 16 : 8;
     const int forced_gt = env_int("QORA_GEMV_GT", 0);
     if (forced_gt == 8 || forced_gt == 16) pl.gt = forced_gt;
     if (paired) {
@@ -48,14 +66,9 @@ bool plan_gemv(int fmt, uint32_t k, const uint32_t* seg_groups, int nseg, bool p
         for (int i = 0; i < nseg; ++i) pl.tiles += (seg_groups[i] + pl.gt - 1) / pl.gt;
     }
     const uint32_t rl = 256u / (uint32_t)pl.gt;
-    // K slices of 128 rows (64 where K is short, 256 for a long Q4 one): enough
-    // workgroups without more than the hand-over or the atomics bear. Calls
-    // of the one-launch entry, rows 64 / 128 / 256: 512 -> 512 Q4 4.6 / 4.8 /
-    // 5.7 us, 2048 -> 512 5.4 / 5.0 / 5.8, 11008 -> 2048 - / 11.9 / 10.1; the
-    // decode step's F16 11008 -> 2048 9.9 / 9.7 / 10.7 (gt 8), its gate|up
-    // pair 18.3 / 18.4 / 19.0. Tiles of 16 groups pay for wide Q4 pairs only
-    // (2048 -> 2 x 11008: 12.4 against 14.3 us; F16 18.8 against 18.6).
-    int rpl = (k <= 1024u ? 64 : (fmt == FMT_Q4 && pl.gt == 8 && k > 4096u) ? 256 : 128) / (int)rl;
+    uint32_t rows = k <= 1024u ? 64u : (q4 && k > 4096u && !sums) ? 256u : 128u;
+    if (pl.gt == 16) rows = (uint64_t)pl.tiles * ((k + 127u) / 128u) >= 4ull * (uint64_t)std::max(1, cus) ? 256u : 128u;
+    int rpl = (int)(rows / rl);
     const int forced_rpl = env_int("QORA_GEMV_RPL", 0);
     if (forced_rpl == 1 || forced_rpl == 2 || (forced_rpl > 0 && forced_rpl % 4 == 0)) rpl = forced_rpl;
     if (row_align > 1) {
@@ -65,9 +78,11 @@ bool plan_gemv(int fmt, uint32_t k, const uint32_t* seg_groups, int nseg, bool p
         if ((rl * (uint32_t)rpl) % row_align != 0 || rl * (uint32_t)rpl > kGemvAttnRows) return false;
     }
     // at most kFixMaxTerms split-K terms per accumulator between two reads
-    // (the fixed-point range guard, params.hpp)
-    while ((k + rl * (uint32_t)rpl - 1) / (rl * (uint32_t)rpl) > kFixMaxTerms) {
-        if (row_align > 1 && (rpl >= 8 || 2 * rl * (uint32_t)rpl > kGemvAttnRows)) break;
+    // (the fixed-point range guard, params.hpp), as far as that goes with 16 rows a
+    // lane (F16: 8): a lane adds its rows up one by one in fp32
+    const int max_rpl = q4 ? 16 : 8;
+    while (rpl < max_rpl && (k + rl * (uint32_t)rpl - 1) / (rl * (uint32_t)rpl) > kFixMaxTerms) {
+        if (row_align > 1 && 2 * rl * (uint32_t)rpl > kGemvAttnRows) break;
         rpl *= 2;
     }
     pl.rpl = rpl;
@@ -180,13 +195,16 @@ static hipError_t launch_gemv_pro(const GemvPlan& plan, const GemvParams& p, hip
 #define QORA_GEMV_B(B_, LOOP_)                                                                                     \
     hipLaunchKernelGGL((gemv_kernel<FMT, GT, B_, LOOP_, PRO, TILED, OUT>), grid, block, 0, stream, p.tw, xin, xaux, p.k, \
                        p.tiles, p.rows_per_split, ss_nn, p)
-    const int b = plan_batch(plan.rpl);
+    const int b = plan_batch(FMT, plan.rpl);
     if (plan.rpl < 1 || plan.rpl % b != 0 || p.rows_per_split != (256u / GT) * (uint32_t)plan.rpl ||
         (PRO == PRO_ATTN && p.rows_per_split > kGemvAttnRows))
         return hipErrorInvalidValue;
     if (b == 1) QORA_GEMV_B(1, false);
     else if (b == 2) QORA_GEMV_B(2, false);
     else if (plan.rpl == 4) QORA_GEMV_B(4, false);
+    else if (b == 8) {
+        if constexpr (FMT == FMT_Q4) QORA_GEMV_B(8, false);
+    }
     else QORA_GEMV_B(4, true);
 #undef QORA_GEMV_B
     return hipGetLastError();

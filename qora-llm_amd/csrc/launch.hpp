@@ -33,9 +33,10 @@ struct GemvPlan {
 // segment; paired: gate/up lane pairing (two segments of equal groups).
 // cus: compute units on the device. Returns false if the shape is unsupported.
 // row_align (optional): K slices must start on multiples of it (head_dim
-// for the attention-merge prologue).
+// for the attention-merge prologue). sums: for a launch that leaves its sums in
+// the accumulator of the caller.
 bool plan_gemv(int fmt, uint32_t k, const uint32_t* seg_groups, int nseg, bool paired, int cus, GemvPlan* plan,
-               uint32_t row_align = 1);
+               uint32_t row_align = 1, bool sums = false);
 
 // Q4 GEMV on the matrix cores: one group per wave (QORA_GEMV_GW may force 2
 // or 4) and the deepest K slice of 256, 128 or 64 rows (QORA_GEMV_KW may

@@ -2,7 +2,7 @@
 the last workgroup of a column tile summing the K slices) against the same call
 on a caller's stream, which clears, accumulates and converts in three launches:
 the same fixed-point terms, so the same bits. Shapes at the edges of the column
-tile (8 groups; 16 for wide Q4 pairs), of the K slice (64, 128, 256 rows), of the
+tile (8 groups; 16 for large Q4 weights), of the K slice (64, 128, 256 rows), of the
 slices per workgroup and with one workgroup per tile (no hand-over); then calls
 of different shapes in a row on the one set of counters."""
 import ctypes
@@ -53,7 +53,7 @@ def side_stream():
 @pytest.mark.parametrize("fmt", ["q4", "f16"])
 @pytest.mark.parametrize("paired", [False, True])
 def test_one_launch_matches_accumulated(ctx, pkg, side_stream, fmt, paired):
-    shapes = SHAPES + ([(300, 8192), (2048, 11008)] if paired else [])
+    shapes = SHAPES + ([(300, 8192), (2048, 11008), (4096, 4096)] if paired else [(4100, 8224), (256, 131104)])
     with device(ctx) as d:
         held = []
         for k, n in shapes:
@@ -226,3 +226,24 @@ def test_a_small_eager_call_sizes_captured_ones_up_to_65536_words(pkg):
                 ctx.graph_destroy(g)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("fmt,rows", [("q4", 16), ("f16", 8)])
+def test_long_k_keeps_its_lanes_chains_short(ctx, pkg, fmt, rows):
+    """However long K is, a lane adds up at most 16 rows (F16: 8) one by one in
+    fp32. Every 2048th group of 32 rows weighs 1, the others half a unit in the last
+    place of that: a chain that starts with a 1 loses the rest of its rows, so the
+    error tells its length."""
+    k, n = 100000, 64
+    x = np.full(k, 2.0 ** -25, np.float32)
+    x[np.arange(k) % 2048 < 32] = 1.0
+    truth = x.astype(np.float64).sum()
+    with device(ctx) as d:
+        if fmt == "q4":
+            w = [d.put(np.full(k * n // 2, 0x99, np.uint8)), d.put(np.full(k * n // 32, 1.0, np.float16))]   # q = 9, scale 1
+        else:
+            w = [d.put(np.full(k * n, 1.0, np.float16))]
+        y = d.empty(n * 4)
+        ctx.check(_call(ctx, pkg, d, fmt, False, w, d.put(x), y, k, n, None))
+        got = d.get(y, n, np.float32).astype(np.float64)
+    assert np.max(np.abs(got - truth)) <= rows * 2.0 ** -24 * truth
