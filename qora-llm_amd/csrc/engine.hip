@@ -188,7 +188,7 @@ struct PreparedGemv {
 // rows hold in two chunks or more (qora_hip_attn_decode: one per KV head, up to
 // 128); the rows' 128 values, m and l
 constexpr size_t kPfAttnOneCounts = kPfAttnOneRows / 64 / 2;
-constexpr size_t kPfAttnOneBytes = kPfAttnOneCounts * sizeof(uint32_t) + (size_t)kPfAttnOneRows * (128 + 2) * sizeof(float);
+constexpr size_t kPfAttnOneBytes = (size_t)kPfAttnOneRows * (128 + 2) * sizeof(float);
 
 struct qora_hip_ctx {
     int device = 0;
@@ -226,10 +226,12 @@ struct qora_hip_ctx {
     uint64_t ws_pf_bytes = 0;
     float* ws_attn_part = nullptr;
     uint64_t ws_attn_part_n = 0;
-    // the attention calls' one-launch splits, made with the context (17 MB; null if
-    // that allocation failed: calls then go unsplit or in two launches): counters,
-    // zero between launches, then qora_hip_attn_prefill's rows
-    void* ws_pa = nullptr;
+    // the attention calls' one-launch splits: counters, zero between launches, made
+    // with the context (1 KB), and qora_hip_attn_prefill's rows, made by the first
+    // call that splits (17 MB). Null where an allocation failed: calls then go
+    // unsplit or in two launches
+    uint32_t* ws_pa_count = nullptr;
+    float* ws_pa = nullptr;
     int32_t* h_pin = nullptr;            // pinned staging: [0] token in, [1] token out, [2] pos
     // The step's argmax, stored by argmax_finish_kernel straight into mapped,
     // coherent pinned memory: reading it back takes the stream sync only, not
@@ -350,6 +352,16 @@ int ensure_pf_ws(qora_hip_ctx* c, uint64_t bytes) {
     c->ws_pf = p;
     c->ws_pf_bytes = bytes;
     return QORA_HIP_OK;
+}
+
+// The rows of qora_hip_attn_prefill's one-launch split; false: no memory, the call
+// goes unsplit.
+bool ensure_pa_ws(qora_hip_ctx* c) {
+    if (!c->ws_pa && hipMalloc((void**)&c->ws_pa, kPfAttnOneBytes) != hipSuccess) {
+        (void)hipGetLastError();
+        c->ws_pa = nullptr;
+    }
+    return c->ws_pa != nullptr;
 }
 
 void free_model(qora_hip_ctx* c) {
@@ -577,14 +589,14 @@ extern "C" int qora_hip_create(int device, qora_hip_ctx** out) {
     } else {
         c->h_tok = nullptr;
     }
-    if (hipMalloc(&c->ws_pa, kPfAttnOneBytes) == hipSuccess) {
-        if (hipMemsetAsync(c->ws_pa, 0, kPfAttnOneCounts * sizeof(uint32_t), c->stream) != hipSuccess) {
-            (void)hipFree(c->ws_pa);
-            c->ws_pa = nullptr;
+    if (hipMalloc((void**)&c->ws_pa_count, kPfAttnOneCounts * sizeof(uint32_t)) == hipSuccess) {
+        if (hipMemsetAsync(c->ws_pa_count, 0, kPfAttnOneCounts * sizeof(uint32_t), c->stream) != hipSuccess) {
+            (void)hipFree(c->ws_pa_count);
+            c->ws_pa_count = nullptr;
         }
     } else {
         (void)hipGetLastError();
-        c->ws_pa = nullptr;
+        c->ws_pa_count = nullptr;
     }
     *out = c;
     return QORA_HIP_OK;
@@ -602,7 +614,7 @@ extern "C" int qora_hip_destroy(qora_hip_ctx* c) {
         if (w.w) (void)hipFree(w.w);
         if (w.scales) (void)hipFree(w.scales);
     }
-    for (void* p : {(void*)c->ws_count, (void*)c->ws_attn_part, c->ws_pa, c->ws_pf, (void*)c->smp_rng, (void*)c->smp_pen, c->smp_sort})
+    for (void* p : {(void*)c->ws_count, (void*)c->ws_attn_part, (void*)c->ws_pa_count, (void*)c->ws_pa, c->ws_pf, (void*)c->smp_rng, (void*)c->smp_pen, c->smp_sort})
         if (p) (void)hipFree(p);
     for (void* p : c->ws_old) (void)hipFree(p);
     if (c->h_pin) (void)hipHostFree(c->h_pin);
@@ -2130,10 +2142,10 @@ extern "C" int qora_hip_attn_decode(qora_hip_ctx* c, const float* q, const void*
     // combine kernel's block a head (1300 positions on one stream 11.3 -> 12.7).
     const uint64_t qb = (uint64_t)H * hd * sizeof(float), cb = (uint64_t)L * KVH * hd * (kv_f16 ? 2 : 4);
     const bool apart = !overlap(out, qb, q, qb) && !overlap(out, qb, kc, cb) && !overlap(out, qb, vc, cb);
-    if (c->ws_pa && a.nsg == 1 && (uint64_t)a.s_max * KVH <= 128u && apart && in_order(c, s)) {
+    if (c->ws_pa_count && a.nsg == 1 && (uint64_t)a.s_max * KVH <= 128u && apart && in_order(c, s)) {
         AttnOneParams one{};
         static_cast<AttnParams&>(one) = a;
-        one.count = (uint32_t*)c->ws_pa;
+        one.count = c->ws_pa_count;
         one.out = out;
         HIP_TRY(c, launch_attn(a, s, &one));
         return QORA_HIP_OK;
@@ -2326,9 +2338,10 @@ extern "C" int qora_hip_attn_prefill(qora_hip_ctx* c, const float* q, const void
     a.scale = 1.0f / sqrtf((float)hd);
     a.out = out;
     const hipStream_t s = pick_stream(c, stream);
-    if (c->ws_pa && in_order(c, s)) {
-        a.count = (uint32_t*)c->ws_pa;
-        a.part = (float*)(a.count + kPfAttnOneCounts);
+    uint32_t ch, nc;
+    if (c->ws_pa_count && in_order(c, s) && pf_attn_one_split(a, &ch, &nc) && ensure_pa_ws(c)) {
+        a.count = c->ws_pa_count;
+        a.part = c->ws_pa;
     }
     HIP_TRY(c, launch_pf_attn(a, s));
     return QORA_HIP_OK;

@@ -942,6 +942,30 @@ static hipError_t launch_pf_attn_split(const PrefillAttnParams& p, hipStream_t s
     return launch_pf_rows(PF_ROW_SPLIT, r, p.T, stream);
 }
 
+// The one-launch split of the kernel-level entry. A tile takes a block
+// 3.7 us (f32; f16 1.9) of a chain that only more blocks shorten, a chunk's
+// store, arrival and merge some 4 us and 0.7 for each chunk to merge: two
+// tiles a chunk, more with the root of their number, and no more chunks
+// than give a block to every CU. From four tiles on (f16: six): 200 tokens
+// 18.7 -> 16.1 us a call on one stream, 512 34.4 -> 24.3, 16 behind 1500
+// positions 72 -> 22.5 (f16 47 -> 19.5); at three tiles 15.9 against 15.8.
+bool pf_attn_one_split(const PrefillAttnParams& p, uint32_t* ch, uint32_t* nc) {
+    const uint32_t G = p.KVH ? p.H / p.KVH : 0u;
+    if ((p.hd != 64 && p.hd != 128) || (G != 1 && G != 2 && G != 4)) return false;
+    const uint32_t qt4 = 16u * (4u / G);
+    const uint64_t blocks4 = (uint64_t)((p.T + qt4 - 1) / qt4) * p.KVH;
+    const uint64_t kt = ((uint64_t)p.pos0 + p.T + 63u) / 64u;   // 64-key tiles
+    const uint64_t rows = (blocks4 + p.KVH) * 64u;              // of a chunk, at most
+    const uint64_t most = std::min(kPfAttnOneRows / rows, 256u / blocks4);
+    if (kt < (p.kv_f16 ? 6u : 4u) || most < 2) return false;
+    uint64_t ct = 2;
+    while (3u * ct * ct < kt) ++ct;
+    ct = std::max(ct, (kt + most - 1) / most);
+    *ch = (uint32_t)(64u * ct);
+    *nc = (uint32_t)((kt + ct - 1) / ct);
+    return true;
+}
+
 hipError_t launch_pf_attn(const PrefillAttnParams& p, hipStream_t stream) {
     if (p.T == 0) return hipSuccess;
     if (p.hd > (uint32_t)kAttnMaxHd || p.hd % 8 != 0 || p.H % p.KVH != 0) return hipErrorInvalidValue;
@@ -970,26 +994,8 @@ hipError_t launch_pf_attn(const PrefillAttnParams& p, hipStream_t stream) {
         const uint32_t qt4 = 16u * (4u / G), nt4 = (p.T + qt4 - 1) / qt4;
         const uint64_t blocks4 = (uint64_t)nt4 * p.KVH;
         const uint64_t kt = ((uint64_t)p.pos0 + p.T + 63u) / 64u;   // 64-key tiles
-        // The one-launch split of the kernel-level entry. A tile takes a block
-        // 3.7 us (f32; f16 1.9) of a chain that only more blocks shorten, a chunk's
-        // store, arrival and merge some 4 us and 0.7 for each chunk to merge: two
-        // tiles a chunk, more with the root of their number, and no more chunks
-        // than give a block to every CU. From four tiles on (f16: six): 200 tokens
-        // 18.7 -> 16.1 us a call on one stream, 512 34.4 -> 24.3, 16 behind 1500
-        // positions 72 -> 22.5 (f16 47 -> 19.5); at three tiles 15.9 against 15.8.
-        if (p.count) {
-            q.count = nullptr;
-            uint64_t ct = 2;
-            while (3u * ct * ct < kt) ++ct;
-            const uint64_t rows = (blocks4 + p.KVH) * 64u;   // of a chunk, at most
-            const uint64_t most = std::min(kPfAttnOneRows / rows, 256u / blocks4);
-            if (kt >= (p.kv_f16 ? 6u : 4u) && most >= 2) {
-                ct = std::max(ct, (kt + most - 1) / most);
-                q.count = p.count;
-                q.ch = (uint32_t)(64u * ct);
-                q.nc = (uint32_t)((kt + ct - 1) / ct);
-            }
-        }
+        if (p.count && pf_attn_one_split(p, &q.ch, &q.nc)) q.count = p.count;
+        else q.count = nullptr;
         // Eight waves on a staged tile where one four-wave tile holds every query
         // (the other waves help to stage: 16 tokens behind 700 positions, unsplit,
         // 48.2 -> 38.8 us), and for f32, whose staging costs most, where the blocks

@@ -157,6 +157,9 @@ uint64_t pf_small_most(int fmt, uint32_t T, uint32_t n, int cus);
 hipError_t launch_pf_gemm_small(int fmt, const PfSmallParams& p, hipStream_t stream);
 hipError_t launch_pf_rope_cache(const PrefillAttnParams& p, hipStream_t stream);
 hipError_t launch_pf_attn(const PrefillAttnParams& p, hipStream_t stream);
+// Whether a launch with p.part and p.count splits the keys over blocks (keys a
+// chunk, chunks a query block).
+bool pf_attn_one_split(const PrefillAttnParams& p, uint32_t* ch, uint32_t* nc);
 
 // on-device sampling (sample.hpp): vocab <= 131072, 1 <= top_k <= 64
 uint32_t smp_blocks(uint32_t vocab);

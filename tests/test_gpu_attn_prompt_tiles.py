@@ -3,6 +3,8 @@ eight waves: 16 or 32 queries with four heads a KV head, up to 128 with one) and
 64-key steps, f32 and f16 caches, against float64. 64 heads over 16 take the eight
 waves from 113 tokens on. The bound is the prompt attention
 tests' own kind: fp32 sums of products held to 22 bits, relative to max |v|."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -77,3 +79,30 @@ def test_split_keys_come_out_as_whole_ones(ctx):
                 first = got if first is None else first
                 np.testing.assert_array_equal(got, first)
         assert np.max(np.abs(first - truth)) <= 1e-5 * np.max(np.abs(v))
+
+
+def test_the_splits_workspace_comes_with_the_first_split_call(pkg):
+    """Contexts that never split a prompt's keys hold no workspace for it."""
+    hip = ctypes.CDLL("libamdhip64.so.7")
+
+    def used(n, split):
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        ctxs = [pkg.HipContext(0) for _ in range(n)]
+        H, KVH, hd = 16, 4, 128
+        T = 300 if split else 60
+        try:
+            for c in ctxs:
+                with device(c) as d:
+                    x = d.empty(T * H * hd * 4)
+                    c.check(c.lib.qora_hip_attn_prefill(c.h, x, x, x, 0, 0, T, H, KVH, hd, d.empty(T * H * hd * 4), None))
+            assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+            return total.value - free.value
+        finally:
+            for c in ctxs:
+                c.close()
+
+    used(2, True)                                  # (what the process allocates once)
+    base, unsplit, split = used(1, False), used(17, False), used(17, True)
+    print("MB a context:", (unsplit - base) / 16 / 2 ** 20, (split - base) / 16 / 2 ** 20, flush=True)
+    assert unsplit - base < 16 * 8 * 2 ** 20
+    assert split - base >= 16 * 4 * 2 ** 20
