@@ -2385,8 +2385,8 @@ int sample_device(qora_hip_ctx* c, const float* logits, uint64_t vocab, const ui
     pen.clear();
     if (rep || pres) {
         const uint64_t first = pres ? 0 : n_history - std::min<uint64_t>(64, n_history);
-        size_t cap = 64;
-        while (cap < 2 * (n_history - first)) cap *= 2;
+        size_t cap = 64;                            // (twice the distinct tokens, or more)
+        while (cap < 2 * std::min(n_history - first, vocab)) cap *= 2;
         std::vector<uint32_t>& at = c->pen_at;
         at.assign(cap, 0);
         for (uint64_t i = first; i < n_history; ++i) {

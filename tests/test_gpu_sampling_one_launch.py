@@ -63,6 +63,32 @@ def test_penalty_list_sizes(ctx, pkg, orc, distinct):
             assert (tok, a) == (want, b)
 
 
+def test_a_long_history_costs_no_table_of_its_length(pkg, orc):
+    """The look-up table goes by the distinct tokens, at most the vocabulary, not by
+    the history's length, and stays small in the context."""
+    def resident():
+        with open("/proc/self/statm") as f:
+            return int(f.read().split()[1]) * 4096
+
+    vocab, n = 5000, 1 << 25
+    ctx = pkg.HipContext(0)
+    params = pkg.SampleParams(**SP)
+    try:
+        lg = (rng(1).standard_normal(vocab) * 3).astype(np.float32)
+        hist = np.tile(np.arange(0, 4096, dtype=np.uint32), n // 4096)
+        with device(ctx) as d:
+            dl = d.put(lg)
+            ctx.sample(dl, vocab, hist[:100], params, 5)
+            before = resident()
+            got = ctx.sample(dl, vocab, hist, params, 7)
+            grown = resident() - before
+            assert got == orc.sample(lg, hist[-4096:].tolist(), SP["temperature"], SP["top_p"], SP["top_k"],
+                                     SP["repetition_penalty"], SP["presence_penalty"], 7)
+            assert grown < 32 * 2 ** 20, grown        # (a table of the history's length: 256 MB)
+    finally:
+        ctx.close()
+
+
 def test_first_calls_on_a_caller_stream_behind_queued_work(pkg, orc):
     """A context's first sampling calls, and those after its scratch grew, on a
     caller's stream while the context's stream has about 1 ms of work queued, then
