@@ -1007,11 +1007,17 @@ __global__ __launch_bounds__(256) void pf_sum_splits_kernel(const float* part, u
 // (the weight has no second part), no exponent. An F16 model's layer then takes
 // four GEMM launches whose partial sums the next kernel adds, as a Q4 one does,
 // instead of seven with a sum each (a 100-token prompt and 16 steps through eight
-// layers: 9.80 -> 9.34 ms).
+// layers: 9.80 -> 9.34 ms). Its K slices are longer than pf_gemm_kernel's (k and v
+// 1024 rows against 256), so the sums of 256 rows leave the accumulators for a second
+// set: the distance of a 300-token prompt's logits from 64 bits, two layers, 0.84e-6 (f32
+// cache) and 1.97e-5 (f16), against 1.12e-6 and 1.81e-5 through pf_gemm_kernel and 1.35e-6
+// and 2.72e-5 with whole chains; 300 tokens 11008 -> 2048 1.7e-7 against 4.0e-7.
+// The adds cost 0 to 3% (prompts of 40 to 512 tokens through eight layers).
 template <int BM, int WM>
 __global__ __launch_bounds__(256, 2) void pf_gemm2_kernel(PfGemm2Params p) {
     constexpr bool RAW = WM == PF_W_RAW, F16 = WM == PF_W_F16;
     constexpr int BN = 128, KC = 32;
+    constexpr uint32_t kFold = 256;
     // LDS rows of 64 B (32 halves, no padding); the 16-byte chunk c of row r
     // sits at chunk c ^ ((r >> 1) & 3), which leaves the fragment reads and the
     // 64-token tiles' x' stores (four threads a row) free of bank conflicts
@@ -1156,6 +1162,21 @@ __global__ __launch_bounds__(256, 2) void pf_gemm2_kernel(PfGemm2Params p) {
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    // F16: the sums of whole runs of kFold rows, which leave acc there, so that no fp32
+    // chain is longer
+    f32x4v tot[F16 ? TM : 1][TN];
+    auto fold = [&](bool first) {
+        if constexpr (F16) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    tot[i][j] = first ? acc[i][j] : tot[i][j] + acc[i][j];
+                    acc[i][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+    };
+    fold(true);
     // A wave raises its issue priority while it reads its fragments and issues
     // its MFMAs (64-token tiles: 3-4% faster on the large shapes, same output;
     // no effect on 32-token tiles), so the matrix cores are fed ahead of the
@@ -1210,6 +1231,7 @@ __global__ __launch_bounds__(256, 2) void pf_gemm2_kernel(PfGemm2Params p) {
             compute(1, bhO, blO);
             store_x(se, 0);
             dequant(se, bhE, blE);
+            if (F16 && s % (kFold / KC) == kFold / KC - 2u) fold(false);
             __syncthreads();
         }
         compute(0, bhE, blE);
@@ -1219,6 +1241,12 @@ __global__ __launch_bounds__(256, 2) void pf_gemm2_kernel(PfGemm2Params p) {
             __syncthreads();
             compute(1, bhO, blO);
         }
+    }
+    if constexpr (F16) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] += tot[i][j];
     }
 
     if (pair) {

@@ -182,3 +182,20 @@ def test_gemm_few_tokens_on_both_sides_of_the_partial_sum_limit(ctx, pkg, fmt, T
     assert np.isfinite(got).all()
     assert elem_err(got[:, cols], x.astype(np.float64) @ Wc, np.abs(x.astype(np.float64)) @ np.abs(Wc)) <= TRUTH_TOL
     ctx.lib.qora_hip_release_weight(ctx.h, wid)
+
+
+def test_f16_gemm_keeps_its_fp32_chains_short(ctx, pkg):
+    """Above 128 tokens an F16 weight's sums run over 256 rows at a time, whatever the
+    K slices: rounding then leaves 1.7e-7 of the result's norm here, and 4.0e-7 where a
+    chain runs over a whole slice (1856 rows)."""
+    k, n, T = 11008, 2048, 300
+    wt, W = _weight(pkg, "f16", k, n, 8, None)
+    wid = ctx.upload(wt)
+    x = rng(8).standard_normal((T, k)).astype(np.float32)
+    with device(ctx) as d:
+        y = d.empty(T * n * 4)
+        ctx.check(ctx.lib.qora_hip_gemm(ctx.h, wid, d.put(x), y, T, None))
+        got = d.get(y, (T, n), np.float32)
+    truth = x.astype(np.float64) @ W
+    assert np.linalg.norm(got - truth) <= 2.5e-7 * np.linalg.norm(truth)
+    ctx.lib.qora_hip_release_weight(ctx.h, wid)
