@@ -2160,6 +2160,18 @@ namespace {
 
 uint64_t al256(uint64_t b) { return (b + 255) & ~uint64_t(255); }
 
+// Which of qora_hip_gemm's general kernels: n % 128 == 0 runs the prefill's GEMM (a Q4
+// weight packed into the workspace for this call, with its own scales), anything
+// else pf_gemm_kernel; so does an F16 weight wider than deep, with few tokens or of
+// more column blocks than a quarter of the CUs, which fill them without it. Calls on
+// one and on three streams through pf_gemm_kernel / through the prefill's: 11008 ->
+// 2048, 512 tokens 125 and 107 / 100 and 84 us, 100 tokens - and 29.2 / - and 28.5; 2048 ->
+// 11008, 100 tokens - and 23.9 / - and 33.1; 8192 -> 8192, 200 tokens 112 and 99 / 102 and 100;
+// 11008 -> 11008, 200 tokens 219 and 191 / 260 and 199.
+bool pf_gemm_wide(int fmt, uint32_t T, uint32_t K, uint32_t N, int cus) {
+    return pf_gemm2_supported(K, N) && (fmt == FMT_Q4 || (N <= K && T > 128u && (uint64_t)N / 128u * 4u <= (uint64_t)cus));
+}
+
 // Scratch of qora_hip_gemm's general kernels: xh, xl [T][k] binary16, xe [T], the
 // packed weight (wq, sc) or wf [n/32] and the exponent partials, the split-K partials.
 struct PfGemmWs {
@@ -2203,8 +2215,9 @@ uint64_t pf_gemm_reserve(int fmt, uint32_t T, uint32_t K, uint32_t N, int cus) {
     const uint32_t tiles = std::min(64u, (T + 63u) / 64u);
     for (uint32_t m = 1; m <= tiles; ++m) {
         const uint32_t u = m == tiles ? T : 64u * m;
-        if (pf_gemm2_supported(K, N)) b = std::max(b, pf_gemm_ws(fmt, u, K, N, true, cus).bytes);
-        if (fmt != FMT_Q4 || !pf_gemm2_supported(K, N)) b = std::max(b, pf_gemm_ws(fmt, u, K, N, false, cus).bytes);
+        const bool wide = pf_gemm_wide(fmt, u, K, N, cus);
+        if (wide) b = std::max(b, pf_gemm_ws(fmt, u, K, N, true, cus).bytes);
+        if (!wide || fmt != FMT_Q4) b = std::max(b, pf_gemm_ws(fmt, u, K, N, false, cus).bytes);
     }
     return b;
 }
@@ -2221,13 +2234,7 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
     const uint32_t K = (uint32_t)w->k, N = (uint32_t)w->n, T = (uint32_t)rows;
     const hipStream_t s = pick_stream(c, stream);
     const bool q4 = w->fmt == FMT_Q4;
-    // The general kernels: n % 128 == 0 runs the prefill's GEMM (a Q4 weight packed
-    // into the workspace for this call, with its own scales), anything else
-    // pf_gemm_kernel; so does an F16 weight wider than deep or with few tokens,
-    // whose column blocks fill the CUs without it (calls on three streams, 2048 ->
-    // 11008, 100 tokens: 23.9 us against 33.1; 11008 -> 2048, 100 tokens 28.5
-    // against 29.2, 512 tokens 103.4 against 84.1)
-    const bool wide = pf_gemm2_supported(K, N) && (q4 || (N <= K && T > 128));
+    const bool wide = pf_gemm_wide(w->fmt, T, K, N, c->cus);
     // A few tokens go straight from the weight as it was uploaded, where the slices'
     // partial sums are few enough; not in place when unsplit, since it then
     // writes y while other blocks read x.

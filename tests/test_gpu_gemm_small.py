@@ -85,7 +85,8 @@ def test_gemm_non_finite_row_stays_in_its_row(ctx, pkg):
     ctx.lib.qora_hip_release_weight(ctx.h, wid)
 
 
-@pytest.mark.parametrize("T,k,n", [(65, 96, 128), (130, 2048, 512), (200, 4128, 256), (512, 512, 1152)])
+@pytest.mark.parametrize("T,k,n", [(65, 96, 128), (130, 2048, 512), (200, 4128, 256), (512, 512, 1152), (129, 8192, 8192),
+                                   (129, 8448, 8320)])
 def test_gemm_f16_wide_vs_truth(ctx, pkg, T, k, n):
     """F16 weights whose width is a multiple of 128 above 64 tokens: 32- and
     64-token tiles, K split and unsplit."""
