@@ -226,6 +226,8 @@ struct qora_hip_ctx {
     uint64_t ws_pf_bytes = 0;
     float* ws_attn_part = nullptr;
     uint64_t ws_attn_part_n = 0;
+    // a captured call used the buffer of the name: outgrown, it goes to ws_old
+    bool ws_pf_captured = false, ws_attn_captured = false;
     // the attention calls' one-launch splits: counters, zero between launches, made
     // with the context (1 KB), and qora_hip_attn_prefill's rows, made by the first
     // call that splits (17 MB). Null where an allocation failed: calls then go
@@ -282,11 +284,14 @@ bool stream_capturing(hipStream_t s) {
     return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
 
+// Whether a call on stream s is being recorded.
+bool captured(qora_hip_ctx* c, hipStream_t s) { return c->capturing || stream_capturing(s); }
+
 // Kernel-level scratch grows outside captures only, the context's own and one
 // that the caller began on the context's stream: there an allocation's clear
 // would become a node of the graph, and a synchronisation end the capture.
 int scratch_may_grow(qora_hip_ctx* c) {
-    if (!c->capturing && !stream_capturing(c->stream)) return QORA_HIP_OK;
+    if (!captured(c, c->stream)) return QORA_HIP_OK;
     return fail(c, QORA_HIP_E_STATE, "scratch must be sized by an eager call before capture");
 }
 
@@ -323,11 +328,19 @@ int ensure_acc_ws(qora_hip_ctx* c, uint64_t n, uint64_t tiles = 0) {
     return QORA_HIP_OK;
 }
 
+// Lets go of an outgrown buffer: freed, or kept until the context ends when a
+// captured call used it (its graph may still run).
+void retire_ws(qora_hip_ctx* c, void* p, bool* captured) {
+    if (p && *captured) c->ws_old.push_back(p);
+    else if (p) (void)hipFree(p);
+    *captured = false;
+}
+
 int ensure_attn_ws(qora_hip_ctx* c, uint64_t part_floats) {
     if (part_floats <= c->ws_attn_part_n) return QORA_HIP_OK;
     if (int rc = scratch_may_grow(c)) return rc;
     HIP_TRY(c, hipStreamSynchronize(c->stream));
-    if (c->ws_attn_part) (void)hipFree(c->ws_attn_part);
+    retire_ws(c, c->ws_attn_part, &c->ws_attn_captured);
     c->ws_attn_part = nullptr;
     c->ws_attn_part_n = 0;
     void* p;
@@ -341,7 +354,7 @@ int ensure_pf_ws(qora_hip_ctx* c, uint64_t bytes) {
     if (bytes <= c->ws_pf_bytes) return QORA_HIP_OK;
     if (int rc = scratch_may_grow(c)) return rc;
     HIP_TRY(c, hipStreamSynchronize(c->stream));
-    if (c->ws_pf) (void)hipFree(c->ws_pf);
+    retire_ws(c, c->ws_pf, &c->ws_pf_captured);
     c->ws_pf = nullptr;
     c->ws_pf_bytes = 0;
     void* p;
@@ -1798,7 +1811,7 @@ int gemv_acc_entry(qora_hip_ctx* c, int fmt, const void* w0, const void* s0, con
 // launches: on the context's own stream, outside a capture, calls run one
 // behind the other; a caller's stream or a captured graph could overlap them.
 bool in_order(qora_hip_ctx* c, hipStream_t s) {
-    return s == c->stream && !c->capturing && !stream_capturing(s);
+    return s == c->stream && !captured(c, s);
 }
 
 // Whether two buffers meet. A launch that reads one while another of its
@@ -2135,6 +2148,7 @@ extern "C" int qora_hip_attn_decode(qora_hip_ctx* c, const float* q, const void*
     if (int rc = ensure_attn_ws(c, (uint64_t)KVH * a.s_max * a.groups * (hd + 2))) return rc;
     a.part = c->ws_attn_part;
     const hipStream_t s = pick_stream(c, stream);
+    c->ws_attn_captured = c->ws_attn_captured || captured(c, s);
     // One launch where few splits are to be merged, which their last one does:
     // 16 heads over 4, on one stream and on three, 64 positions 8.5 and 8.5 -> 7.3
     // and 5.3 us a call, 500 9.1 and 8.3 -> 8.2 and 5.2, 858 (108 splits) 10.6 and
@@ -2258,6 +2272,7 @@ extern "C" int qora_hip_gemm(qora_hip_ctx* c, uint32_t wid, const float* x, floa
         need = g.bytes;
     }
     if (int rc = ensure_pf_ws(c, need)) return rc;
+    c->ws_pf_captured = c->ws_pf_captured || captured(c, s);
     if (small) {
         PfSmallParams q{};
         q.x = x;

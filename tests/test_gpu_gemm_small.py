@@ -200,3 +200,39 @@ def test_f16_gemm_keeps_its_fp32_chains_short(ctx, pkg):
     truth = x.astype(np.float64) @ W
     assert np.linalg.norm(got - truth) <= 2.5e-7 * np.linalg.norm(truth)
     ctx.lib.qora_hip_release_weight(ctx.h, wid)
+
+
+def test_outgrown_workspaces_serve_the_graphs_that_hold_them(pkg):
+    """A GEMM and a decode attention captured, then eager calls that outgrow their
+    workspaces, then the replays: what a graph holds is kept."""
+    ctx = pkg.HipContext(0)
+    k, n, T, L, H, hd = 2048, 512, 16, 700, 4, 128
+    try:
+        wid = ctx.upload(_weight(pkg, "q4", k, n, 3, None)[0])
+        big = ctx.upload(_weight(pkg, "q4", 4096, 4096, 4, None)[0])
+        r = rng(5)
+        with device(ctx) as d:
+            x, kv = d.put(r.standard_normal((T, k)).astype(np.float32)), d.put(r.standard_normal((8 * L, H * hd)).astype(np.float32))
+            y, z, a, b = (d.empty(T * n * 4) for _ in range(4))
+            attn = lambda L, out: ctx.lib.qora_hip_attn_decode(ctx.h, x, kv, kv, 0, L, H, H, hd, out, None)
+            ctx.check(ctx.lib.qora_hip_gemm(ctx.h, wid, x, y, T, None))
+            ctx.check(attn(L, a))
+            want, wa = d.get(y, (T, n), np.uint32), d.get(a, H * hd, np.uint32)
+            ctx.capture_begin()
+            rc = ctx.lib.qora_hip_gemm(ctx.h, wid, x, z, T, None) or attn(L, b)
+            g = ctx.capture_end()
+            ctx.check(rc)
+            ctx.check(ctx.lib.qora_hip_gemm(ctx.h, big, d.put(np.ones((300, 4096), np.float32)), d.empty(300 * 4096 * 4), 300, None))
+            ctx.check(attn(8 * L, a))
+            hold = [d.put(np.full(1 << 18, 0x5A5A5A5A, np.uint32)) for _ in range(16)]   # what freed blocks would be given to
+            for _ in range(3):
+                ctx.h2d(z, np.zeros((T, n), np.float32))
+                ctx.h2d(b, np.zeros(H * hd, np.float32))
+                ctx.graph_launch(g)
+                assert np.array_equal(d.get(z, (T, n), np.uint32), want)
+                assert np.array_equal(d.get(b, H * hd, np.uint32), wa)
+            for h in hold:
+                assert (d.get(h, 1 << 18, np.uint32) == 0x5A5A5A5A).all()
+            ctx.graph_destroy(g)
+    finally:
+        ctx.close()
