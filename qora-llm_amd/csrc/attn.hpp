@@ -781,13 +781,17 @@ __global__ __launch_bounds__(256 * kAttnLongNsg) void attn_decode_long_kernel(At
 }
 
 // Long contexts with an f16 cache: no LDS staging of the cache. Block (KV
-// head, split) of NWV waves; wave w takes the 8-position passes w, w + NWV,
-// ... of the split (short passes keep every wave busy on splits of a few
+// head, split) of NWV waves; wave w takes the PP-position passes w, w + NWV,
+// ... of the split. PP = 8 (short passes keep every wave busy on splits of a few
 // hundred positions and the register set small: 8.8% faster decode at 8192
-// positions than 32-position passes, 2.8% at 32700). Every lane works on
-// the same slice of the row throughout: lane (c, j) = (l % 16, l / 16) holds
-// dims [c HD/16, (c + 1) HD/16) of positions 4 i + j (i < 2) of the pass,
-// so each K and V load instruction
+// positions than 32-position passes, 2.8% at 32700), and 16 for heads of 64, whose
+// rows are half as long, on splits of 128 positions or more, which give every wave
+// a pass of 16 (32700 positions of 8 KV heads, calls on one stream 25.5 -> 23.8 us and
+// on three 15.1 -> 13.7; 6000 of 2 KV heads, 94 a split, 12.5 against 13.0. Passes of 16
+// with rows of 128 cost registers, 8000 positions of 4 KV heads 16.6 -> 17.8).
+// Every lane works on the same slice of the row throughout: lane (c, j) =
+// (l % 16, l / 16) holds dims [c HD/16, (c + 1) HD/16) of positions 4 i + j
+// (i < PP / 4) of the pass, so each K and V load instruction
 // reads 4 whole rows (1 KB at HD 128) and a lane's scores are those of the
 // very positions whose V it holds: the probabilities never leave the lane.
 // Partial dot products are summed over the 16 lanes of a row (4 shuffles),
@@ -795,7 +799,7 @@ __global__ __launch_bounds__(256 * kAttnLongNsg) void attn_decode_long_kernel(At
 // (max, sum, p.V) states are merged in wave order at the end. The appended
 // row (model mode) comes from LDS, and positions at or past the split's end
 // never reach a sum (selection, not a zero weight: stale slots may hold NaN).
-template <int HD>
+template <int HD, int PP>
 __global__ __launch_bounds__(512) void attn_decode_direct_kernel(const int32_t* pos_a, AttnParams p) {
     // the position's pointer is preloaded into scalar registers at wave
     // launch: its load goes out with the parameter block's lines, and one
@@ -803,11 +807,6 @@ __global__ __launch_bounds__(512) void attn_decode_direct_kernel(const int32_t* 
     const int32_t pos_ld = pos_a ? ld_scalar_i32(pos_a) : 0;
     kernarg_warm(p);
     constexpr int NWV = 8;                           // waves per block
-    // positions per pass (2 rows a lane; 4 of a head of 64, whose rows are half as
-    // long: 32700 positions of 8 KV heads, on one stream 25.3 -> 23.7 us a call and
-    // on three 14.9 -> 13.1. Four rows of 128 cost registers, 8000 positions of 4
-    // KV heads 16.6 -> 17.8)
-    constexpr int PP = HD == 64 ? 16 : 8;
     constexpr int VD = HD / 16;                      // dims per lane
     constexpr int NI = PP / 4;                       // rows per lane per pass
     constexpr int G4 = kAttnMaxGroups;

@@ -509,8 +509,12 @@ hipError_t launch_attn(const AttnParams& p, hipStream_t stream, const AttnOnePar
     if (lng && p.kv_f16 && (p.hd == 128 || p.hd == 64) && p.groups <= (uint32_t)kAttnMaxGroups &&
         !tuning_env("QORA_HIP_ATTN_STAGED")) {
         const dim3 grid_t(p.KVH, p.s_max);
-        if (p.hd == 128) hipLaunchKernelGGL((attn_decode_direct_kernel<128>), grid_t, dim3(512), 0, stream, p.pos, p);
-        else hipLaunchKernelGGL((attn_decode_direct_kernel<64>), grid_t, dim3(512), 0, stream, p.pos, p);
+        // (a model's split length follows the position: the one of its full cache)
+        const uint64_t split = p.chunk ? p.chunk : p.kv_hs / p.hd / kAttnMaxSplits;
+        if (p.hd == 128) hipLaunchKernelGGL((attn_decode_direct_kernel<128, 8>), grid_t, dim3(512), 0, stream, p.pos, p);
+        else if (split >= 128u)
+            hipLaunchKernelGGL((attn_decode_direct_kernel<64, 16>), grid_t, dim3(512), 0, stream, p.pos, p);
+        else hipLaunchKernelGGL((attn_decode_direct_kernel<64, 8>), grid_t, dim3(512), 0, stream, p.pos, p);
         return hipGetLastError();
     }
     const dim3 block(lng ? 256 * kAttnLongNsg : 256);

@@ -40,3 +40,24 @@ def test_one_launch_has_the_two_launches_bits(ctx, side_stream, kv_f16, H, KVH, 
     truth = np.einsum("hl,lhd->hd", p / p.sum(1, keepdims=True), vd).reshape(-1)
     # scores to a few fp32 ulp of |q||k| ~ 3 hd / sqrt(hd): 1e-5 relative to max |v|
     assert np.max(np.abs(ref - truth)) <= 1e-5 * np.max(np.abs(vd))
+
+
+@pytest.mark.parametrize("L", [2049, 4096, 6000, 8064, 8065, 8200, 12001])
+def test_long_f16_heads_of_64_at_both_pass_lengths(ctx, L):
+    """Splits of fewer than 128 positions take passes of 8, longer ones of 16; L - 1
+    leaves the last pass of a split partly empty."""
+    H, KVH, hd = 8, 2, 64
+    r = rng(L)
+    q = r.standard_normal(H * hd).astype(np.float32) * 3
+    k, v = (r.standard_normal((L, KVH * hd)).astype(np.float16) for _ in range(2))
+    with device(ctx) as d:
+        qd, kd, vd, out = d.put(q), d.put(k), d.put(v), d.empty(H * hd * 4)
+        for n in (L, L - 1):
+            ctx.check(ctx.lib.qora_hip_attn_decode(ctx.h, qd, kd, vd, 1, n, H, KVH, hd, out, None))
+            got = d.get(out, H * hd, np.float32)
+            k64, v64 = (a[:n].astype(np.float64).reshape(n, KVH, hd).repeat(H // KVH, 1) for a in (k, v))
+            s = np.einsum("hd,lhd->hl", q.reshape(H, hd).astype(np.float64), k64) / np.sqrt(hd)
+            p = np.exp(s - s.max(1, keepdims=True))
+            truth = np.einsum("hl,lhd->hd", p / p.sum(1, keepdims=True), v64).reshape(-1)
+            # as above: scores to a few fp32 ulp
+            assert np.max(np.abs(got - truth)) <= 1e-5 * np.max(np.abs(v64))
