@@ -162,10 +162,11 @@ def copies_time(ctx, hip, srcs, launch):
 
 
 def valu_q4_roofline(ctx, hip, be, pkg):
-    """The VALU Q4 GEMV (gemv_kernel, the reference weight layout, one
-    launch through qora_hip_gemv_q4_accumulate / _gate_up_q4_accumulate)
-    and the VALU row-dot lm_head (qora_hip_gemv_q4_rowdot) on the shapes the
-    matrix-core kernels are timed on, for the comparison of the two."""
+    """The Q4 kernels on the reference weight layout, on the shapes the kernels
+    of the packed layout are timed on, for the comparison of the two: the VALU
+    GEMV (gemv_kernel, one launch through qora_hip_gemv_q4_accumulate /
+    _gate_up_q4_accumulate) and the row-dot lm_head (qora_hip_gemv_q4_rowdot,
+    which runs on the int8 matrix cores at 2048 columns)."""
     c = be.config
     lib, h = ctx.lib, ctx.h
     x = ctx.malloc(4 * c.intermediate)

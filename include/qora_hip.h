@@ -201,7 +201,10 @@ int qora_hip_graph_destroy(qora_hip_ctx* ctx, void* graph_exec);
 
 /* ---- kernel-level entry points ------------------------------------------
  * Device pointers, launched on `stream` (a hipStream_t; NULL = the context
- * stream). Scratch for split-K partials comes from the context. */
+ * stream). Scratch for split-K partials comes from the context; it does not
+ * grow under capture (QORA_HIP_E_STATE: run the call once eagerly first). The
+ * gemv, gate_up, gemm and attn_decode calls may write their output over their
+ * input. */
 
 /* gemv -> gemv_q4 (gemv.rs:382-387, 646-675; simd.rs:44-83): y = x . W,
  * W Q4 [k][n] in the projection layout. */

@@ -10,20 +10,22 @@
 //   * A "group" is 32 output columns of one input row: 16 bytes of nibbles
 //     plus one scale (Q4), or 64 bytes (F16). Each lane owns one group and
 //     accumulates its 32 columns in registers over RPL rows, so one 128-bit
-//     load feeds 32 multiply-adds, and all RPL loads are in flight at once.
+//     load feeds 32 multiply-adds, and the loads of four rows (of all eight of a
+//     Q4 slice that has eight) are in flight at once.
 //   * A workgroup (256 lanes) covers a column tile of GT groups and a slice of
 //     KR = (256/GT)*RPL input rows. Lanes t = rl*GT + gi: the GT lanes of a
 //     row read GT*16 contiguous bytes (128 B or 256 B row segments).
 //   * The row lanes of a group are summed in registers and the waves through
 //     LDS; each column's sum is then added to a fixed-point int64 accumulator
 //     with one fire-and-forget 64-bit atomic (or, for the kernel-level entries
-//     that return y, left for the tile's last workgroup: OUT below). Integer addition is exact, so the result does not
-//     depend on the order the K slices land in (deterministic), and no
-//     fence or counter is needed: the kernel boundary publishes the sums.
-//   * The prologue builds the K slice of the input in LDS: plain x, RMSNorm
-//     of the fixed-point residual, silu(gate)*up of the fixed-point gate/up
-//     sums, or the merge of split attention partials. Consumers therefore
-//     finish the previous phase's reduction on the fly.
+//     that return y, left for the tile's last workgroup: OUT below). Integer
+//     addition is exact, so the result does not depend on the order the K slices
+//     land in (deterministic), and no fence or counter is needed: the kernel
+//     boundary publishes the sums.
+//   * The prologue forms a lane's inputs: plain x, RMSNorm of the fixed-point
+//     residual, silu(gate)*up of the fixed-point gate/up sums, or (through LDS)
+//     the merge of split attention partials. Consumers therefore finish the
+//     previous phase's reduction on the fly.
 // Segments: up to three weight matrices are addressed as one virtual matrix
 // (q|k|v concatenated by column tiles), or two matrices are paired lane by
 // lane (gate|up).
