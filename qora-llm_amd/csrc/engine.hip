@@ -368,12 +368,15 @@ int ensure_pf_ws(qora_hip_ctx* c, uint64_t bytes) {
 }
 
 // The rows of qora_hip_attn_prefill's one-launch split; false: no memory, the call
-// goes unsplit.
+// goes unsplit. (Allocated in relaxed mode: in the default one it would end a capture
+// that the caller has going on a stream of its own, which this call does not touch.)
 bool ensure_pa_ws(qora_hip_ctx* c) {
-    if (!c->ws_pa && hipMalloc((void**)&c->ws_pa, kPfAttnOneBytes) != hipSuccess) {
-        (void)hipGetLastError();
-        c->ws_pa = nullptr;
-    }
+    if (c->ws_pa) return true;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    if (!relaxed || hipMalloc((void**)&c->ws_pa, kPfAttnOneBytes) != hipSuccess) c->ws_pa = nullptr;
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!c->ws_pa) (void)hipGetLastError();
     return c->ws_pa != nullptr;
 }
 

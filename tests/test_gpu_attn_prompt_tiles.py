@@ -106,3 +106,34 @@ def test_the_splits_workspace_comes_with_the_first_split_call(pkg):
     print("MB a context:", (unsplit - base) / 16 / 2 ** 20, (split - base) / 16 / 2 ** 20, flush=True)
     assert unsplit - base < 16 * 8 * 2 ** 20
     assert split - base >= 16 * 4 * 2 ** 20
+
+
+def test_the_first_split_call_leaves_another_streams_capture_alone(pkg):
+    """A context's first split call, on its own stream, while the caller captures
+    another stream in the default mode: that capture still ends in a graph."""
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    H, KVH, hd, T = 4, 1, 128, 300
+    r = rng(12)
+    q = r.standard_normal((T, H * hd)).astype(np.float32)
+    k, v = (r.standard_normal((T, KVH * hd)).astype(np.float32) for _ in range(2))
+    truth = _truth(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), 0, T, H, KVH, hd)
+    ctx, other, graph = pkg.HipContext(0), ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(other), 1) == 0     # hipStreamNonBlocking
+    try:
+        with device(ctx) as d:
+            out = d.empty(T * H * hd * 4)
+            args = (ctx.h, d.put(q), d.put(k), d.put(v), 0, 0, T, H, KVH, hd, out)
+            ctx.synchronize()
+            assert hip.hipStreamBeginCapture(other, 0) == 0              # hipStreamCaptureModeGlobal
+            rc = ctx.lib.qora_hip_attn_prefill(*args, None)
+            end = hip.hipStreamEndCapture(other, ctypes.byref(graph))
+            ctx.check(rc)
+            assert end == 0
+            assert hip.hipGraphDestroy(graph) == 0
+            got = d.get(out, (T, H * hd), np.float32)
+            assert np.max(np.abs(got - truth)) <= 1e-5 * np.max(np.abs(v))
+            ctx.check(ctx.lib.qora_hip_attn_prefill(*args, None))
+            np.testing.assert_array_equal(d.get(out, (T, H * hd), np.float32), got)
+    finally:
+        ctx.close()
+        assert hip.hipStreamDestroy(other) == 0
